@@ -1,38 +1,33 @@
-// Tiled MFMA GEMM for the projections at prefill sizes (more than 32 token rows):
+// Tiled MFMA GEMM for the projections beyond the decode step's few rows (linear.hip):
 //   y[t, g*N + n] = sum_k x[t, g*K + k] * w[g*N + n, k]      (v4mlx/mla.py:16-18, and the grouped
 //   product of v4mlx/mla.py:49-53 for G > 1; ref_torch/compressor.py:28-29 with fp32 operands)
 //
 // Both operands are K-contiguous (x rows, w rows), which is the operand order of the gfx950 MFMA:
 // a lane's A fragment is 8 consecutive k of one token row, its B fragment 8 consecutive k of one
-// weight row.  A workgroup of 4 waves computes a 128 (tokens) x 128 (outputs) tile, each wave a
+// weight row.  Rows past T or N are loaded clamped (finite) and never stored.
+//
+// gemm_ring_kernel (bf16, K a multiple of 64): the K loop of gemm_tile.h in one of four tile forms.
+// A product of a few hundred tokens has far fewer large tiles than the chip has CUs, and each tile's
+// K range is a serial chain of steps, so the time is that chain's: the plan weighs smaller tiles (more
+// workgroups, more operand bytes each) against splitting the K range over up to 8 workgroups per
+// tile, whose fp32 partial sums gemm_reduce_kernel adds in split order.  Before and after, us:
+//   [64, 8192] x [4096, 8192]^T 156 -> 16 (67 MB of weights at 4.2 TB/s), [300, 8192] x the same 184 ->
+//   33, 8 groups of [300, 4096] x [1024, 4096]^T 100 -> 33, [1024, 4096] x [1024, 4096]^T 83 -> 17,
+//   [4096, 8192] x [4096, 8192]^T 244 -> 210, [4096, 1024] x [32768, 1024]^T 291 -> 265.
+//
+// gemm_kernel (fp32 operands, and K tails): 4 waves computing a 128 x 128 tile, each wave a
 // 64 x 64 quarter as 2 x 2 blocks of v_mfma_f32_32x32x16_bf16 (bf16 operands) or
 // v_mfma_f32_32x32x2f32 (fp32 operands), accumulating in fp32.  K advances in steps of 128 bytes
 // per row (64 bf16 / 32 fp32): the next step's tiles are loaded into registers while the current
 // ones are multiplied out of LDS, two LDS stages, one barrier per step.  LDS rows are padded to
-// 144 bytes so the 16-byte fragment reads of 32 consecutive rows spread over the banks.
-// Rows past T or N are loaded clamped (finite) and never stored; K is a multiple of 16 bytes, and
-// the 16-byte chunks of the last step that lie past K are zero.
+// 144 bytes so the 16-byte fragment reads of 32 consecutive rows spread over the banks.  K is a
+// multiple of 16 bytes, and the 16-byte chunks of the last step that lie past K are zero.
 //
 // ROPE (bf16, the attention output projection of oracle/decode_engine.py:118-119): the K step that
-// holds the last rd = 64 dims of a head has its (x0, x1) pairs rotated back to position 0 while it
-// is loaded (inverse RoPE at pos[t], every product and sum rounded in float32, then bf16), the
+// holds the last rd = 64 dims of a head has its (x0, x1) pairs rotated back to position 0 before it
+// is read (inverse RoPE at pos[t], every product and sum rounded in float32, then bf16), the
 // arithmetic of smla_rope.
-//
-// Large bf16 products (gemm_dma_kernel: K a multiple of 64 and enough 256 x 256 tiles for every
-// CU, else 128 x 128 tiles of 4 waves, two workgroups per CU, when those suffice):
-// 8 waves per 256 x 256 workgroup, each a 128 x 64 quarter-octant as 4 x 2 blocks of
-// v_mfma_f32_32x32x16_bf16.  Operands go HBM -> LDS by global_load_lds_dwordx4 (no register
-// staging) into a ring of two 64 KB stages; a K step (64 k) is 32 MFMAs per wave, two waves per
-// SIMD, long enough to cover the next step's copies, with one barrier per step.  A copy
-// instruction lands 64 x 16 bytes contiguously (8 rows of 128 bytes), so the rows cannot be
-// padded: chunk c of row r is stored in slot c ^ ((r / 2) mod 8) instead, so that the fragment
-// reads of 16 consecutive rows (two rows per 256-byte bank cycle) fall in distinct banks.  A
-// 128 x 128 tile per workgroup with register staging (gemm_kernel) moves twice the operand bytes
-// per product through LDS and had only 16 MFMAs per step to hide its next loads: 370-660 TFLOP/s
-// on the prompt-size projections against 1.0-1.2 PFLOP/s here.  Measured and not kept: the same
-// tile with register-staged operands (0.98-1.04), a 4-stage ring of 32-k steps (0.98-1.02),
-// fragments of the next sub-step read ahead of the MFMAs (equal).
-#include "attn_common.h"
+#include "gemm_tile.h"
 #include "smla_internal.h"
 
 namespace {
@@ -42,8 +37,6 @@ constexpr int kRowBytes = 128;        // bytes of one tile row per K step
 constexpr int kLdsRow = 144;          // padded LDS row
 constexpr int kTileLds = kBM * kLdsRow;
 constexpr int kChunks = kBM * kRowBytes / 16 / 256;  // 16-byte chunks per thread per operand (4)
-
-typedef float f32x16_t_g __attribute__((ext_vector_type(16)));
 
 __device__ inline float mul_rn_g(float a, float b) {
 #pragma clang fp contract(off)
@@ -136,7 +129,7 @@ __global__ __launch_bounds__(256) void gemm_kernel(const uint8_t* __restrict__ x
     }
   };
 
-  f32x16_t_g acc[2][2];
+  f32x16_t acc[2][2];
 #pragma unroll
   for (int mb = 0; mb < 2; mb++)
 #pragma unroll
@@ -215,187 +208,278 @@ __global__ __launch_bounds__(256) void gemm_kernel(const uint8_t* __restrict__ x
     }
 }
 
-// BT x BT tiles (tokens x outputs): BT = 256 with 8 waves of 128 x 64, or BT = 128 with 4 waves of
-// 64 x 64 (two workgroups per CU); either way 8 one-KB copy instructions per wave per stage
-template <int BT>
-struct DmaTile {
-  static constexpr int NW = BT == 256 ? 8 : 4;        // waves
-  static constexpr int WROWS = BT / 2;                 // rows per wave (2 row halves)
-  static constexpr int MB = WROWS / 32;                // 32-row MFMA blocks per wave
-  static constexpr int OPB = BT * kRowBytes;           // one operand's rows of one K step
-  static constexpr int STAGE = 2 * OPB;                // A then B
-  static constexpr int COPIES = STAGE / 1024 / NW;     // per wave per stage (8)
-  static constexpr int ACH = BT * 8 / (64 * NW);       // A chunks per thread (rotation of a RoPE step: 4)
+// ---- the ring kernel's tile forms (tokens x outputs, waves of .. x .., stages)
+template <int FORM>
+struct Form;
+template <>
+struct Form<0> {  // 4 waves, 64 KB: two workgroups per CU
+  static constexpr int BM = 64, BN = 64, WM = 32, WN = 32, D = 4;
+};
+template <>
+struct Form<1> {  // 4 waves, 128 KB
+  static constexpr int BM = 128, BN = 128, WM = 64, WN = 64, D = 4;
+};
+template <>
+struct Form<2> {  // 8 waves, 144 KB
+  static constexpr int BM = 128, BN = 256, WM = 64, WN = 64, D = 3;
+};
+template <>
+struct Form<3> {  // 8 waves, 128 KB
+  static constexpr int BM = 256, BN = 256, WM = 128, WN = 64, D = 2;
+};
+constexpr int kForms = 4;
+constexpr int kFormBM[kForms] = {64, 128, 128, 256}, kFormBN[kForms] = {64, 128, 256, 256};
+constexpr int kFormD[kForms] = {Form<0>::D, Form<1>::D, Form<2>::D, Form<3>::D};  // least K steps of a workgroup
+constexpr int kMaxSplits = 8;
+
+struct RingArgs {
+  const uint8_t* x;
+  const uint8_t* w;
+  int64_t ldx;  // bytes
+  int T, N, K, G, nt, nn, splits;
+  const int32_t* pos;
+  const float* cos_t;
+  const float* sin_t;
+  int head_dim;
+  uint8_t* y;
+  int64_t ldy, split_stride;  // elements
+  int vec;                    // rows and groups of y start at multiples of 16 bytes
+  int rot;                    // K steps between the starts of neighbouring token tiles
 };
 
-template <int YDT, bool ROPE, int BT>
-__global__ __launch_bounds__(DmaTile<BT>::NW * 64) void gemm_dma_kernel(const uint8_t* __restrict__ x, int64_t ldx,
-                                                       const uint8_t* __restrict__ w, int T, int N, int K, int ntn,
-                                                       const int32_t* __restrict__ pos, const float* __restrict__ cos_t,
-                                                       const float* __restrict__ sin_t, int head_dim,
-                                                       void* __restrict__ y, int64_t ldy) {
-  using namespace smla_attn;
-  using L = DmaTile<BT>;
-  constexpr int kStageBytes = L::STAGE, kOperandBytes = L::OPB, kCopiesPerWave = L::COPIES;
+// Workgroup order: the launch deals workgroups to the 8 XCDs round-robin; each XCD takes a
+// contiguous run of tiles, ordered in groups of 4 token tiles over all output tiles, so that the
+// tiles running together on an XCD share x and w rows in its L2.  Splits are outermost.
+template <int FORM, int YDT, bool ROPE>
+__global__ __launch_bounds__((Form<FORM>::BM / Form<FORM>::WM) * (Form<FORM>::BN / Form<FORM>::WN) * 64) void
+gemm_ring_kernel(const RingArgs p) {
+  using namespace smla_gemm;
+  using F = Form<FORM>;
+  constexpr int BM = F::BM, BN = F::BN, WM = F::WM, WN = F::WN, D = F::D;
+  using L = Tile<BM, BN, WM, WN, D>;
   extern __shared__ __align__(16) uint8_t lds_g[];
-  lds_u8_t* lds = (lds_u8_t*)lds_g;
-  const uint32_t lds_base = (uint32_t)(uintptr_t)lds;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int g = blockIdx.x / ntn;
-  const int n0 = (blockIdx.x % ntn) * BT;
-  const int t0 = blockIdx.y * BT;
-  const int wm = wave & 1, wn = wave >> 1;  // row half, 64-column slice
-  // copy instruction q = 8 wave + i covers stage bytes [1024 q, 1024 q + 1024): rows
-  // 8 (q mod BT/8) .. +7 of A (q < BT/8) or of B; lane L takes row + L / 8, slot L mod 8 <- chunk
-  // (L mod 8) ^ ((row / 2) mod 8)
-  const uint8_t* src[kCopiesPerWave];
-#pragma unroll
-  for (int i = 0; i < kCopiesPerWave; i++) {
-    const int q = wave * kCopiesPerWave + i;
-    const int r = 8 * (q % (BT / 8)) + (lane >> 3);
-    const int c = (lane & 7) ^ ((r >> 1) & 7);
-    if (q < BT / 8) {
-      const int t = min(t0 + r, T - 1);
-      src[i] = x + ((int64_t)t * ldx + (int64_t)g * K) * 2 + 16 * c;
-    } else {
-      const int n = min(n0 + r, N - 1);
-      src[i] = w + ((int64_t)g * N + n) * (int64_t)K * 2 + 16 * c;
-    }
-  }
-  auto issue = [&](int stage, int ks) __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < kCopiesPerWave; i++) {
-      const uint32_t ld =
-          __builtin_amdgcn_readfirstlane(lds_base + stage * kStageBytes + (wave * kCopiesPerWave + i) * 1024);
-      dma16(src[i] + (int64_t)ks * kRowBytes, ld);
-    }
-  };
+  const uint32_t tot = gridDim.x, per = tot / kXcds, rem = tot % kXcds, xcd = blockIdx.x % kXcds;
+  uint32_t id = xcd * per + (xcd < rem ? xcd : rem) + blockIdx.x / kXcds;
+  const uint32_t tiles = (uint32_t)p.nt * p.nn;
+  const uint32_t sg = id / tiles;  // split * G + group
+  id -= sg * tiles;
+  const int sp = sg / p.G, g = sg - sp * p.G;
+  const uint32_t grp = id / (4u * p.nn), gs = min(4u, (uint32_t)p.nt - 4 * grp), in = id - grp * 4u * p.nn;
+  const int t0 = (4 * grp + in % gs) * BM, n0 = (in / gs) * BN;
+  const int nk = p.K / 64, k0 = nk * sp / p.splits, k1 = nk * (sp + 1) / p.splits;
+  const uint8_t* xk = p.x + (int64_t)t0 * p.ldx + (int64_t)g * p.K * 2 + (int64_t)k0 * kRow;
+  const uint8_t* wk = p.w + ((int64_t)g * p.N + n0) * (int64_t)p.K * 2 + (int64_t)k0 * kRow;
 
-  f32x16_t_g acc[L::MB][2];
-#pragma unroll
-  for (int mb = 0; mb < L::MB; mb++)
-#pragma unroll
-    for (int nb = 0; nb < 2; nb++)
-#pragma unroll
-      for (int r = 0; r < 16; r++) acc[mb][nb][r] = 0.f;
-  // fragment rows of this lane: A row 128 wm + 32 mb + lane % 32, B row 64 wn + 32 nb + lane % 32;
-  // the lane half h holds k 16 kk + 8 h .. +7, chunk 2 kk + h of the row
-  const int r32 = lane & 31, khalf = lane >> 5;
-  // ROPE: the A chunks this thread rotates in a RoPE step, j = tid + 512 i (row j / 8, slot j mod 8),
-  // and their rows' offsets in the cos / sin tables (32 pairs per position)
-  int prow[L::ACH] = {};
+  const int rot = (int)(in % gs) * p.rot % (k1 - k0);
+  // ROPE: the chunks of x this thread rotates in a step that holds a head's last 64 dims: chunk
+  // tid + i threads (row j / 8, slot j mod 8, 4 (x0, x1) pairs from pair 4 c, c = slot ^ ((row / 2) mod
+  // 8)); offsets of their rows in the cos / sin tables (32 pairs per position)
+  constexpr int NT = L::NW * 64, ACH = BM * 8 / NT;
+  int prow[ACH] = {};
   if constexpr (ROPE) {
 #pragma unroll
-    for (int i = 0; i < L::ACH; i++) prow[i] = pos[min(t0 + ((tid + 64 * L::NW * i) >> 3), T - 1)] * 32;
+    for (int i = 0; i < ACH; i++) prow[i] = p.pos[min(t0 + (((int)threadIdx.x + NT * i) >> 3), p.T - 1)] * 32;
   }
-  const int nk = K / 64;
-  issue(0, 0);
-  for (int ks = 0; ks < nk; ks++) {
-    wait_vm(0);     // this wave's copies of step ks
-    lds_barrier();  // everyone's copies of step ks landed; step ks - 1 is read by every wave
-    if (ks + 1 < nk) issue((ks + 1) & 1, ks + 1);
-    const lds_u8_t* A = lds + (ks & 1) * kStageBytes;
-    const lds_u8_t* B = A + kOperandBytes;
+  f32x16_t acc[L::MB][L::NB];
+  tile_loop<BM, BN, WM, WN, D>((lds_u8_t*)lds_g, xk, p.ldx, p.T - 1 - t0, wk, (int64_t)p.K * 2, p.N - 1 - n0, k1 - k0,
+                               rot, acc, [&](int ks, lds_u8_t* stage) __attribute__((always_inline)) {
     if constexpr (ROPE) {
-      // the step holding a head's last 64 dims: every A chunk (4 (x0, x1) pairs, pairs 4c .. 4c + 3
-      // of its row's position, c = slot ^ ((row / 2) mod 8)) rotated back in place, then a barrier
-      if ((ks * 64) % head_dim == head_dim - 64) {
+      const int k = ks + rot < k1 - k0 ? ks + rot : ks + rot - (k1 - k0);
+      if (((k0 + k) * 64) % p.head_dim == p.head_dim - 64) {
 #pragma unroll
-        for (int i = 0; i < L::ACH; i++) {
-          const int j = tid + 64 * L::NW * i, r = j >> 3, sl = j & 7, c = sl ^ ((r >> 1) & 7);
-          lds_u32x4_t* pa = (lds_u32x4_t*)(lds + (ks & 1) * kStageBytes + r * kRowBytes + 16 * sl);
-          *pa = inv_rope4(*pa, cos_t + prow[i] + 4 * c, sin_t + prow[i] + 4 * c);
+        for (int i = 0; i < ACH; i++) {
+          const int j = threadIdx.x + NT * i, r = j >> 3, sl = j & 7, c = sl ^ ((r >> 1) & 7);
+          lds_u32x4_t* pa = (lds_u32x4_t*)(stage + r * kRow + 16 * sl);
+          *pa = inv_rope4(*pa, p.cos_t + prow[i] + 4 * c, p.sin_t + prow[i] + 4 * c);
         }
         lds_barrier();
       }
     }
-#pragma unroll
-    for (int kk = 0; kk < 4; kk++) {
-      const int c = 2 * kk + khalf;
-      bf16x8_t a[L::MB], b[2];
-#pragma unroll
-      for (int mb = 0; mb < L::MB; mb++) {
-        const int r = L::WROWS * wm + 32 * mb + r32;
-        a[mb] = as_bf16x8(*(const lds_u32x4_t*)(A + r * kRowBytes + 16 * (c ^ ((r >> 1) & 7))));
-      }
-#pragma unroll
-      for (int nb = 0; nb < 2; nb++) {
-        const int r = 64 * wn + 32 * nb + r32;
-        b[nb] = as_bf16x8(*(const lds_u32x4_t*)(B + r * kRowBytes + 16 * (c ^ ((r >> 1) & 7))));
-      }
-#pragma unroll
-      for (int mb = 0; mb < L::MB; mb++)
-#pragma unroll
-        for (int nb = 0; nb < 2; nb++)
-          acc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[mb], b[nb], acc[mb][nb], 0, 0, 0);
-    }
-  }
+  });
 
-  // accumulator r of block (mb, nb): token WROWS wm + 32 mb + 8 (r / 4) + 4 (lane / 32) + r % 4,
-  // output 64 wn + 32 nb + lane % 32.  Nontemporal stores (the output is not read back by this
-  // launch; 64-byte runs per half wave): the grouped 4096 x 8 x 1024 x 4096 product 287 -> 275 us,
-  // the other prompt-size shapes equal.
+  // Output rows leave through LDS (each wave its own region, MBP blocks of 32 rows at a time), so that
+  // a lane stores 16 bytes and a wave whole 128-byte lines: 16 stores per wave instead of 128 of two
+  // bytes per lane, few enough to stay in flight when the wave ends.  Chunk c of row r sits in slot
+  // c ^ swizzle(r), so that the two rows of a write (r and r + 4) and the rows of a read use distinct
+  // banks.  Nontemporal: the output is not read back by this launch.
+  constexpr int ES = YDT == SMLA_BF16 ? 2 : 4, CH = WN * ES / 16, RPI = 64 / CH;  // chunks per row, rows per store
+  constexpr int FIT = L::LDS / (L::NW * 32 * WN * ES), MBP = FIT < L::MB ? FIT : L::MB;
+  static_assert(MBP >= 1 && L::MB % MBP == 0, "the waves' regions fit the ring's LDS");
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = wave % (BM / WM), wn = wave / (BM / WM);
+  const int64_t base = sp * p.split_stride + (int64_t)g * p.N;
+  if (p.vec) {  // uniform
+    lds_u8_t* reg = (lds_u8_t*)lds_g + wave * (MBP * 32 * WN * ES);
+    auto slot = [](int r, int c) { return CH == 16 ? c ^ ((r << 1) & 8) : c ^ (r & (CH - 1)); };
+    lds_barrier();  // every wave has read its last fragments
+#pragma unroll
+    for (int m0 = 0; m0 < L::MB; m0 += MBP) {
+#pragma unroll
+      for (int mb = 0; mb < MBP; mb++)
+#pragma unroll
+        for (int nb = 0; nb < L::NB; nb++)
+#pragma unroll
+          for (int r = 0; r < 16; r++) {
+            const int row = 32 * mb + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3), col = (32 * nb + (lane & 31)) * ES;
+            lds_u8_t* q = reg + row * (WN * ES) + 16 * slot(row, col >> 4) + (col & 15);
+            if constexpr (YDT == SMLA_BF16) *(smla_attn::lds_u16_t*)q = bf16_rne(acc[m0 + mb][nb][r]);
+            else *(smla_attn::lds_f32_t*)q = acc[m0 + mb][nb][r];
+          }
+      const int n = n0 + WN * wn + (lane % CH) * (16 / ES);
+#pragma unroll
+      for (int i = 0; i < MBP * 32 / RPI; i++) {
+        const int row = RPI * i + lane / CH, t = t0 + WM * wm + 32 * m0 + row;
+        const u32x4_t v = *(lds_u32x4_t*)(reg + row * (WN * ES) + 16 * slot(row, lane % CH));
+        if (t < p.T && n < p.N)
+          __builtin_nontemporal_store(v, (u32x4_t*)(p.y + (base + (int64_t)t * p.ldy + n) * ES));
+      }
+    }
+    return;
+  }
 #pragma unroll
   for (int mb = 0; mb < L::MB; mb++)
 #pragma unroll
-    for (int nb = 0; nb < 2; nb++) {
-      const int n = n0 + 64 * wn + 32 * nb + r32;
-      if (n >= N) continue;
+    for (int nb = 0; nb < L::NB; nb++) {
+      const int n = n0 + WN * wn + 32 * nb + (lane & 31);
+      const int t1 = t0 + WM * wm + 32 * mb + 4 * (lane >> 5);
+      if (n >= p.N) continue;
 #pragma unroll
       for (int r = 0; r < 16; r++) {
-        const int t = t0 + L::WROWS * wm + 32 * mb + 8 * (r >> 2) + 4 * khalf + (r & 3);
-        if (t < T) {
-          const int64_t o = (int64_t)t * ldy + (int64_t)g * N + n;
-          if constexpr (YDT == SMLA_BF16)
-            __builtin_nontemporal_store((uint16_t)bf16_rne(acc[mb][nb][r]), (uint16_t*)y + o);
-          else
-            __builtin_nontemporal_store(acc[mb][nb][r], (float*)y + o);
+        const int t = t1 + 8 * (r >> 2) + (r & 3);
+        if (t < p.T) {
+          const int64_t o = base + (int64_t)t * p.ldy + n;
+          if constexpr (YDT == SMLA_BF16) ((uint16_t*)p.y)[o] = bf16_rne(acc[mb][nb][r]);
+          else ((float*)p.y)[o] = acc[mb][nb][r];
         }
       }
     }
 }
 
-}  // namespace
+// y[i] = part[0][i] + part[1][i] + ... in split order; V elements per thread
+template <int YDT, int V>
+__global__ __launch_bounds__(256) void gemm_reduce_kernel(const float* __restrict__ part, int splits, int64_t n,
+                                                          void* __restrict__ y) {
+  const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * V;
+  if (i >= n) return;
+  typedef float vec_t __attribute__((ext_vector_type(V)));
+  vec_t v[kMaxSplits];
+#pragma unroll
+  for (int s = 0; s < kMaxSplits; s++) v[s] = *(const vec_t*)(part + min(s, splits - 1) * n + i);
+  vec_t sum = v[0];
+#pragma unroll
+  for (int s = 1; s < kMaxSplits; s++)
+    if (s < splits) sum += v[s];
+  if constexpr (YDT == SMLA_F32) {
+    *(vec_t*)((float*)y + i) = sum;
+  } else if constexpr (V == 4) {
+    *(u32x2_t*)((uint16_t*)y + i) = (u32x2_t){pack_bf16x2(sum[0], sum[1]), pack_bf16x2(sum[2], sum[3])};
+  } else {
+    ((uint16_t*)y)[i] = bf16_rne(sum[0]);
+  }
+}
 
-template <int BT>
-static int launch_gemm_dma(const void* x, int64_t ldx, const void* w, int64_t T, int64_t G, int64_t N, int64_t K,
-                           const int32_t* pos, const float* cos_t, const float* sin_t, int64_t head_dim, void* y,
-                           int y_dtype, hipStream_t st) {
-  using L = DmaTile<BT>;
-  const int64_t ntb = (N + BT - 1) / BT;
-  const dim3 gb((unsigned)(ntb * G), (unsigned)((T + BT - 1) / BT));
-  auto kern = pos ? (y_dtype == SMLA_BF16 ? gemm_dma_kernel<SMLA_BF16, true, BT> : gemm_dma_kernel<SMLA_F32, true, BT>)
-                  : (y_dtype == SMLA_BF16 ? gemm_dma_kernel<SMLA_BF16, false, BT> : gemm_dma_kernel<SMLA_F32, false, BT>);
+// ---- the plan: tile form and splits for a bf16 product
+struct RingPlan {
+  int form, splits;
+};
+
+// whether the ring kernel takes the shape (else gemm_kernel): whole 64-k steps, enough of them for
+// the shortest ring, and a tile's row offsets within 31 bits
+bool ring_takes(int64_t ldx, int64_t K) {
+  return K % 64 == 0 && K / 64 >= kFormD[3] && ldx % 8 == 0 && ldx * 2 * 256 < (1ll << 31) && K * 2 * 256 < (1ll << 31);
+}
+
+RingPlan ring_plan(int64_t T, int64_t G, int64_t N, int64_t K, bool may_split) {
+  // A model of the launch in microseconds, its constants fitted to every (form, splits) of 154 products
+  // (T 12 .. 4096 by the layer's weights, K 1024 .. 8192); the plan it picks is 1 % off the fastest on
+  // average and 12 % at worst.  One 64-k step of a tile takes kIdle when few CUs run and kBusy when all
+  // do (kPair for two co-resident 64 x 64 workgroups); the weights and tokens come in at 4.8 TB/s at
+  // best; a split adds the reduce launch and its partial sums at 4.3 TB/s.
+  constexpr double kIdle[kForms] = {0.24, 0.31, 0.57, 1.03}, kBusy[kForms] = {0.24, 0.53, 0.875, 1.47}, kPair = 0.36;
+  constexpr double kEnds = 2.5, kReduce = 2.0, kHbm = 4.8e6, kPartial = 8 / 4.3e6;
+  const int64_t cus = smla_num_cus(), nk = K / 64;
+  const double in = 2.0 * K * G * (N + T) / kHbm;
+  RingPlan best{3, 1};
+  double bt = 1e30;
+  for (int f = 0; f < kForms; f++) {
+    const int64_t tiles = (T + kFormBM[f] - 1) / kFormBM[f] * G * ((N + kFormBN[f] - 1) / kFormBN[f]);
+    const int64_t cap = f == 0 ? 2 * cus : cus;  // workgroups resident together
+    for (int s = 1; s <= (may_split ? kMaxSplits : 1) && nk / s >= kFormD[f]; s++) {
+      const int64_t rest = tiles * s % cap;
+      double t = (double)(tiles * s / cap) * (f == 0 ? kPair : kBusy[f]);
+      if (rest > cus) t += kPair;
+      else if (rest > 0) t += kIdle[f] + (kBusy[f] - kIdle[f]) * (double)rest / (double)cus;
+      t *= (double)((nk + s - 1) / s);
+      t = kEnds + (t > in ? t : in);
+      if (s > 1) t += kReduce + s * (double)T * G * N * kPartial;
+      if (t < bt) bt = t, best = {f, s};
+    }
+  }
+  return best;
+}
+
+template <int FORM>
+int launch_ring(const RingArgs& a, int64_t wgs, bool rope, int y_dtype, hipStream_t st) {
+  using F = Form<FORM>;
+  using L = smla_gemm::Tile<F::BM, F::BN, F::WM, F::WN, F::D>;
+  auto kern = rope ? (y_dtype == SMLA_BF16 ? gemm_ring_kernel<FORM, SMLA_BF16, true> : gemm_ring_kernel<FORM, SMLA_F32, true>)
+                   : (y_dtype == SMLA_BF16 ? gemm_ring_kernel<FORM, SMLA_BF16, false> : gemm_ring_kernel<FORM, SMLA_F32, false>);
   // devices whose LDS limit is raised, one set per kernel (RoPE form x output type)
   static std::atomic<uint64_t> lds_attr[4] = {{0}, {0}, {0}, {0}};
-  if (hipError_t e = smla_set_dynamic_lds((const void*)kern, 2 * L::STAGE,
-                                          lds_attr[(pos ? 2 : 0) + (y_dtype == SMLA_BF16 ? 1 : 0)]);
+  if (hipError_t e = smla_set_dynamic_lds((const void*)kern, L::LDS, lds_attr[(rope ? 2 : 0) + (y_dtype == SMLA_BF16 ? 1 : 0)]);
       e != hipSuccess)
     return (int)e;
-  hipLaunchKernelGGL(kern, gb, dim3(L::NW * 64), 2 * L::STAGE, st, (const uint8_t*)x, ldx, (const uint8_t*)w, (int)T,
-                     (int)N, (int)K, (int)ntb, pos, cos_t, sin_t, (int)head_dim, y, G * N);
+  hipLaunchKernelGGL(kern, dim3((unsigned)wgs), dim3(L::NW * 64), L::LDS, st, a);
   SMLA_HIP_CHECK_LAUNCH();
   return SMLA_OK;
 }
 
+}  // namespace
+
+bool gemm_tiled_takes(int64_t G, int64_t K) { return ring_takes(G * K, K); }
+
+int64_t gemm_tiled_workspace(int64_t T, int64_t G, int64_t N, int64_t K, bool f32_operands) {
+  if (f32_operands || !ring_takes(G * K, K)) return 0;
+  const RingPlan p = ring_plan(T, G, N, K, true);
+  return p.splits > 1 ? p.splits * T * G * N * (int64_t)sizeof(float) : 0;
+}
+
 // y [T, G*N] (row stride G*N) = grouped x [T, G*K] (row stride ldx elements) times w [G*N, K]^T.
-// x and w both bf16 (x_f32 false) or both fp32; y bf16 or fp32.  With pos (bf16 only), inverse RoPE
+// x and w both bf16 (f32_operands false) or both fp32; y bf16 or fp32.  With pos (bf16 only), inverse RoPE
 // of the last 64 dims of every head_dim-wide head of x on load.  16-byte aligned rows (K % 8 for
-// bf16, K % 4 for fp32).  Returns SMLA_OK or a hipError_t.
+// bf16, K % 4 for fp32).  ws: gemm_tiled_workspace bytes for the partial sums of a split K range, or
+// less (null): the plan without splits.  Returns SMLA_OK or a hipError_t.
 int launch_gemm_tiled(const void* x, int64_t ldx, bool f32_operands, const void* w, int64_t T, int64_t G, int64_t N,
                       int64_t K, const int32_t* pos, const float* cos_t, const float* sin_t, int64_t head_dim,
-                      void* y, int y_dtype, hipStream_t st) {
+                      void* y, int y_dtype, void* ws, size_t ws_bytes, hipStream_t st) {
   const int64_t ldy = G * N;
-  // bf16 operands, 16-byte aligned, K a multiple of 64 (and the RoPE dims one K step per head): the
-  // DMA tiles, 256 x 256 when they give every CU one, else 128 x 128 when those do
-  if (!f32_operands && K % 64 == 0 && ldx % 8 == 0 && (!pos || head_dim % 64 == 0) &&
-      (((uintptr_t)x | (uintptr_t)w) & 15) == 0) {
-    const int64_t cus = smla_num_cus();
-    auto tiles = [&](int64_t bt) { return (T + bt - 1) / bt * G * ((N + bt - 1) / bt); };
-    if (tiles(256) >= cus)
-      return launch_gemm_dma<256>(x, ldx, w, T, G, N, K, pos, cos_t, sin_t, head_dim, y, y_dtype, st);
-    if (tiles(128) >= cus)
-      return launch_gemm_dma<128>(x, ldx, w, T, G, N, K, pos, cos_t, sin_t, head_dim, y, y_dtype, st);
+  if (!f32_operands && ring_takes(ldx, K) && (!pos || head_dim % 64 == 0)) {
+    const int64_t need = gemm_tiled_workspace(T, G, N, K, false);
+    const bool split = need > 0 && ws && ws_bytes >= (size_t)need;
+    const RingPlan p = ring_plan(T, G, N, K, split);
+    const int bm = kFormBM[p.form], bn = kFormBN[p.form];
+    const int64_t nt = (T + bm - 1) / bm, nn = (N + bn - 1) / bn, wgs = nt * nn * G * p.splits;
+    if (wgs > 0x7fffffff) return SMLA_E_UNSUPPORTED;
+    RingArgs a{(const uint8_t*)x, (const uint8_t*)w, ldx * 2, (int)T, (int)N, (int)K, (int)G, (int)nt, (int)nn, p.splits,
+               pos, cos_t, sin_t, (int)head_dim, (uint8_t*)(p.splits > 1 ? ws : y), ldy, T * ldy, 0, 0};
+    const int odt = p.splits > 1 ? SMLA_F32 : y_dtype;
+    // rows of x 64 KB apart fall in the same sets of an L2, which the 4 token tiles of a group would
+    // then all want at once: they start 4 steps apart (8 groups of [4096, 4096] x [1024, 4096]^T 281 ->
+    // 262 us; with closer rows, which it does not help, a rotation costs up to 3 %)
+    a.rot = p.form == 3 && a.ldx % 65536 == 0 ? 4 : 0;
+    a.vec = N % (odt == SMLA_BF16 ? 8 : 4) == 0 && ((uintptr_t)a.y & 15) == 0;
+    const int rc = p.form == 0   ? launch_ring<0>(a, wgs, pos != nullptr, odt, st)
+                   : p.form == 1 ? launch_ring<1>(a, wgs, pos != nullptr, odt, st)
+                   : p.form == 2 ? launch_ring<2>(a, wgs, pos != nullptr, odt, st)
+                                 : launch_ring<3>(a, wgs, pos != nullptr, odt, st);
+    if (rc != SMLA_OK || p.splits == 1) return rc;
+    const int64_t n = T * ldy;
+    const bool v4 = n % 4 == 0;
+    const dim3 grid((unsigned)((n / (v4 ? 4 : 1) + 255) / 256));
+    auto red = y_dtype == SMLA_BF16 ? (v4 ? gemm_reduce_kernel<SMLA_BF16, 4> : gemm_reduce_kernel<SMLA_BF16, 1>)
+                                    : (v4 ? gemm_reduce_kernel<SMLA_F32, 4> : gemm_reduce_kernel<SMLA_F32, 1>);
+    hipLaunchKernelGGL(red, grid, dim3(256), 0, st, (const float*)ws, p.splits, n, y);
+    SMLA_HIP_CHECK_LAUNCH();
+    return SMLA_OK;
   }
   const int64_t ntn = (N + kBN - 1) / kBN;
   const dim3 grid((unsigned)(ntn * G), (unsigned)((T + kBM - 1) / kBM)), blk(256);

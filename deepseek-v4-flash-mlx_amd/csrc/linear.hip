@@ -1,4 +1,4 @@
-// Projections of the decode step: few tokens (T <= 32) against a large bf16 weight, on MFMA.
+// Projections of the decode step: few tokens (at most 32) against a large bf16 weight, on MFMA.
 //
 //  * linear_kernel<TT, ROPE, YDT> : y[t, n] = sum_k x'[t, g*K + k] * W[n, k] for the rows n of
 //      group g = n / N (G groups of N rows; G = 1 is a plain linear).  With ROPE, x is the
@@ -359,11 +359,20 @@ int launch_linear(const void* x, const void* w, int64_t T, int64_t G, int64_t N,
   return launch_linear_t<false, SMLA_F32>(xb, wb, T, G, N, K, ldx, nullptr, nullptr, nullptr, 0, 0, y, st);
 }
 
-// The decode form (the weight-streaming kernels above) takes up to 32 bf16 token rows with N % 16 == 0
-// and K % 512 == 0; everything else goes to the tiled MFMA GEMM (gemm.hip): bf16 or fp32 operands,
-// rows of a multiple of 16 bytes (K % 8 bf16, K % 4 fp32).
+// The decode form (the weight-streaming kernels above) can take up to 32 bf16 token rows with N % 16
+// == 0 and K % 512 == 0; everything else goes to the tiled MFMA GEMM (gemm.hip): bf16 or fp32
+// operands, rows of a multiple of 16 bytes (K % 8 bf16, K % 4 fp32).
 bool decode_form(int x_dtype, int64_t T, int64_t N, int64_t K) {
   return x_dtype == SMLA_BF16 && T <= 32 && N % 16 == 0 && K % (64 * kLinWaves) == 0;
+}
+
+// Whether a shape that the decode form can take runs on it.  From 9 rows on the tiled GEMM is faster
+// when its plan needs no workspace or has it ([12, 4096] x [1024, 4096]^T 7.4 against 9.4 us, [32, 1024]
+// x [32768, 1024]^T 12.6 against 32.7: the decode kernel re-reads x from L2 per 16 outputs), slower
+// when it would have to split K and cannot (16 against 8.6 us for [12, 4096] x [512, 4096]^T).
+bool decode_runs(int x_dtype, int64_t T, int64_t G, int64_t N, int64_t K, bool tiled_can, bool has_ws) {
+  if (!decode_form(x_dtype, T, N, K)) return false;
+  return T <= 8 || !tiled_can || !gemm_tiled_takes(G, K) || (gemm_tiled_workspace(T, G, N, K, false) > 0 && !has_ws);
 }
 
 int check_linear(const void* x, int x_dtype, const void* w, int w_dtype, int64_t T, int64_t G, int64_t N, int64_t K,
@@ -388,14 +397,25 @@ int check_rope_args(const int32_t* pos, const float* cos_t, const float* sin_t, 
 
 }  // namespace
 
-extern "C" int smla_linear(const void* x, int x_dtype, const void* w, int w_dtype, int64_t T, int64_t G, int64_t N,
-                           int64_t K, void* y, int y_dtype, void* stream) {
+extern "C" int smla_linear_ws(const void* x, int x_dtype, const void* w, int w_dtype, int64_t T, int64_t G, int64_t N,
+                              int64_t K, void* y, int y_dtype, void* workspace, size_t workspace_bytes,
+                              void* stream) {
   int rc = check_linear(x, x_dtype, w, w_dtype, T, G, N, K, y, y_dtype);
   if (rc) return rc;
-  if (!decode_form(x_dtype, T, N, K))
+  if (!decode_runs(x_dtype, T, G, N, K, true, workspace && workspace_bytes >= smla_linear_workspace(T, G, N, K, x_dtype)))
     return launch_gemm_tiled(x, G * K, x_dtype == SMLA_F32, w, T, G, N, K, nullptr, nullptr, nullptr, 0, y, y_dtype,
-                             (hipStream_t)stream);
+                             workspace, workspace_bytes, (hipStream_t)stream);
   return launch_linear(x, w, T, G, N, K, nullptr, nullptr, nullptr, 0, 0, y, y_dtype, (hipStream_t)stream);
+}
+
+extern "C" int smla_linear(const void* x, int x_dtype, const void* w, int w_dtype, int64_t T, int64_t G, int64_t N,
+                           int64_t K, void* y, int y_dtype, void* stream) {
+  return smla_linear_ws(x, x_dtype, w, w_dtype, T, G, N, K, y, y_dtype, nullptr, 0, stream);
+}
+
+extern "C" size_t smla_linear_workspace(int64_t T, int64_t G, int64_t N, int64_t K, int x_dtype) {
+  if (T <= 0 || G <= 0 || N <= 0 || K <= 0 || decode_runs(x_dtype, T, G, N, K, true, true)) return 0;
+  return (size_t)gemm_tiled_workspace(T, G, N, K, x_dtype == SMLA_F32);
 }
 
 extern "C" int smla_rope(void* x, int x_dtype, int64_t T, int64_t heads, int64_t head_dim, int64_t rd,
@@ -421,10 +441,26 @@ extern "C" int smla_rope(void* x, int x_dtype, int64_t T, int64_t heads, int64_t
   return SMLA_OK;
 }
 
+extern "C" size_t smla_o_proj_workspace(int64_t T, int64_t heads, int64_t head_dim, int64_t G, int64_t R, int64_t dim) {
+  if (T <= 0 || heads <= 0 || head_dim <= 0 || G <= 0 || R <= 0 || dim <= 0) return 0;
+  // the two products run one after the other and share it
+  const size_t a = smla_linear_workspace(T, G, R, heads * head_dim / G, SMLA_BF16);
+  const size_t b = smla_linear_workspace(T, 1, dim, G * R, SMLA_BF16);
+  return a > b ? a : b;
+}
+
 extern "C" int smla_o_proj(const void* o, int o_dtype, const int32_t* pos, const float* cos_t, const float* sin_t,
                            int64_t n_pos, int64_t T, int64_t heads, int64_t head_dim, int64_t rd, int64_t G, int64_t R,
                            const void* wo_a, const void* wo_b, int w_dtype, int64_t dim, void* mid, void* y,
                            int y_dtype, void* stream) {
+  return smla_o_proj_ws(o, o_dtype, pos, cos_t, sin_t, n_pos, T, heads, head_dim, rd, G, R, wo_a, wo_b, w_dtype, dim, mid,
+                        y, y_dtype, nullptr, 0, stream);
+}
+
+extern "C" int smla_o_proj_ws(const void* o, int o_dtype, const int32_t* pos, const float* cos_t, const float* sin_t,
+                              int64_t n_pos, int64_t T, int64_t heads, int64_t head_dim, int64_t rd, int64_t G,
+                              int64_t R, const void* wo_a, const void* wo_b, int w_dtype, int64_t dim, void* mid,
+                              void* y, int y_dtype, void* workspace, size_t workspace_bytes, void* stream) {
   if (!o || !wo_a || !wo_b || !mid || !y) return SMLA_E_NULL;
   if (T <= 0 || heads <= 0 || head_dim <= 0 || G <= 0 || R <= 0 || dim <= 0) return SMLA_E_SHAPE;
   if ((heads * head_dim) % G != 0) return SMLA_E_SHAPE;
@@ -434,21 +470,25 @@ extern "C" int smla_o_proj(const void* o, int o_dtype, const int32_t* pos, const
   if (rc) return rc;
   rc = check_linear(mid, SMLA_BF16, wo_b, w_dtype, T, 1, dim, G * R, y, y_dtype);
   if (rc) return rc;
-  const bool dform = decode_form(o_dtype, T, R, Kg);
+  const bool rot64 = !pos || rd == 64;  // the tiled GEMM rotates exactly the last 64 dims of each head
+  const bool dform = decode_runs(o_dtype, T, G, R, Kg, rot64,
+                                 workspace && workspace_bytes >= smla_linear_workspace(T, G, R, Kg, SMLA_BF16));
   if (pos) {
     rc = check_rope_args(pos, cos_t, sin_t, n_pos, heads, head_dim, rd);
     if (rc) return rc;
-    // every 64-wide K step lies inside one head, all rope dims or none; the tiled GEMM rotates
-    // exactly the last 64 dims of each head
-    if (head_dim % 64 != 0 || rd % 64 != 0 || Kg % head_dim != 0 || (!dform && rd != 64)) return SMLA_E_UNSUPPORTED;
+    // every 64-wide K step lies inside one head, all rope dims or none
+    if (head_dim % 64 != 0 || rd % 64 != 0 || Kg % head_dim != 0 || (!dform && !rot64)) return SMLA_E_UNSUPPORTED;
   }
   hipStream_t st = (hipStream_t)stream;
   if (dform)
     rc = launch_linear(o, wo_a, T, G, R, Kg, pos, cos_t, sin_t, (int)head_dim, (int)rd, mid, SMLA_BF16, st);
   else
-    rc = launch_gemm_tiled(o, G * Kg, false, wo_a, T, G, R, Kg, pos, cos_t, sin_t, head_dim, mid, SMLA_BF16, st);
+    rc = launch_gemm_tiled(o, G * Kg, false, wo_a, T, G, R, Kg, pos, cos_t, sin_t, head_dim, mid, SMLA_BF16, workspace,
+                           workspace_bytes, st);
   if (rc) return rc;
-  if (!decode_form(SMLA_BF16, T, dim, G * R))
-    return launch_gemm_tiled(mid, G * R, false, wo_b, T, 1, dim, G * R, nullptr, nullptr, nullptr, 0, y, y_dtype, st);
+  if (!decode_runs(SMLA_BF16, T, 1, dim, G * R, true,
+                   workspace && workspace_bytes >= smla_linear_workspace(T, 1, dim, G * R, SMLA_BF16)))
+    return launch_gemm_tiled(mid, G * R, false, wo_b, T, 1, dim, G * R, nullptr, nullptr, nullptr, 0, y, y_dtype,
+                             workspace, workspace_bytes, st);
   return launch_linear(mid, wo_b, T, 1, dim, G * R, nullptr, nullptr, nullptr, 0, 0, y, y_dtype, st);
 }

@@ -63,6 +63,11 @@ _SIGNATURES = {
     "smla_rotate_fp4": (_int, [_vp, _int, _i64, _i64, _int, _vp, _vp, _vp, _vp]),
     "smla_rope": (_int, [_vp, _int, _i64, _i64, _i64, _i64, _vp, _vp, _vp, _i64, _int, _vp]),
     "smla_linear": (_int, [_vp, _int, _vp, _int, _i64, _i64, _i64, _i64, _vp, _int, _vp]),
+    "smla_linear_workspace": (_sz, [_i64, _i64, _i64, _i64, _int]),
+    "smla_linear_ws": (_int, [_vp, _int, _vp, _int, _i64, _i64, _i64, _i64, _vp, _int, _vp, _sz, _vp]),
+    "smla_o_proj_workspace": (_sz, [_i64] * 6),
+    "smla_o_proj_ws": (_int, [_vp, _int, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _vp, _vp, _int,
+                              _i64, _vp, _vp, _int, _vp, _sz, _vp]),
     "smla_o_proj": (_int, [_vp, _int, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _vp, _vp, _int,
                            _i64, _vp, _vp, _int, _vp]),
 }

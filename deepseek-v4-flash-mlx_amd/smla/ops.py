@@ -422,8 +422,12 @@ def linear_op(x: torch.Tensor, w: torch.Tensor, groups: int, out_dtype: torch.dt
     if x.shape[1] != groups * K or w.shape[0] != groups * N:
         raise ValueError("linear: x [T, G*K] and w [G*N, K] do not agree")
     y = torch.empty(T, groups * N, dtype=out_dtype, device=x.device)
-    _lib.call("smla_linear", _p(x), dtype_code(x), _p(w), dtype_code(w), T, groups, N, K, _p(y), _YDT[out_dtype],
-              _stream(x))
+    # no workspace up to 8 rows on the weight-streaming kernel (the library says 0 there)
+    wsb = 0 if T <= 8 and x.dtype == torch.bfloat16 and K % 512 == 0 and N % 16 == 0 else \
+        _lib.lib().smla_linear_workspace(T, groups, N, K, dtype_code(x))
+    ws = torch.empty(wsb, dtype=torch.uint8, device=x.device) if wsb else None
+    _lib.call("smla_linear_ws", _p(x), dtype_code(x), _p(w), dtype_code(w), T, groups, N, K, _p(y), _YDT[out_dtype],
+              _p(ws), wsb, _stream(x))
     return y
 
 
@@ -469,8 +473,10 @@ def o_proj_op(o: torch.Tensor, pos: Optional[torch.Tensor], cos_t: Optional[torc
         pos = pos.to(torch.int32).contiguous()
         cos_t, sin_t = cos_t.float().contiguous(), sin_t.float().contiguous()
         rd, n_pos = 2 * cos_t.shape[1], cos_t.shape[0]
-    _lib.call("smla_o_proj", _p(o), dtype_code(o), _p(pos), _p(cos_t), _p(sin_t), n_pos, T, H, D, rd, groups, R,
-              _p(wo_a), _p(wo_b), dtype_code(wo_a), dim, _p(mid), _p(y), _YDT[out_dtype], _stream(o))
+    wsb = _lib.lib().smla_o_proj_workspace(T, H, D, groups, R, dim)
+    ws = torch.empty(wsb, dtype=torch.uint8, device=o.device) if wsb else None
+    _lib.call("smla_o_proj_ws", _p(o), dtype_code(o), _p(pos), _p(cos_t), _p(sin_t), n_pos, T, H, D, rd, groups, R,
+              _p(wo_a), _p(wo_b), dtype_code(wo_a), dim, _p(mid), _p(y), _YDT[out_dtype], _p(ws), wsb, _stream(o))
     return y
 
 

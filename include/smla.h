@@ -35,7 +35,8 @@
  *   smla_rope                 ref_torch/norm_rope.py:53-62     apply_rotary_emb(x, freqs_cis, inverse) in place
  *                             v4mlx/norm_rope.py:46-62         (MLX twin, cos/sin tables)
  *   smla_linear               v4mlx/mla.py:16-18               linear(x, W) (and the grouped form of mla.py:49-53)
- *   smla_o_proj               oracle/decode_engine.py:118-119  inverse RoPE of o's rope dims + o_grouped
+ *   smla_linear_ws            v4mlx/mla.py:16-18               (the same, with a workspace)
+ *   smla_o_proj, _ws          oracle/decode_engine.py:118-119  inverse RoPE of o's rope dims + o_grouped
  *                             v4mlx/mla.py:42-56               o_grouped(o, wo_a, wo_b)
  */
 #ifndef SMLA_H
@@ -433,10 +434,20 @@ int smla_rope(void* x, int x_dtype, int64_t T, int64_t heads, int64_t head_dim, 
  * is v4mlx/mla.py:16-18, y = x @ W^T; G > 1 is the grouped product of v4mlx/mla.py:49-53).
  *   x [T, G*K], w [G*N, K]: both BF16 or both F32; y [T, G*N] BF16 or F32; float32 accumulation.
  *   16-byte aligned pointers; K % 8 == 0 (BF16) or K % 4 == 0 (F32); any T >= 1.
- *   Decode shapes (BF16, T <= 32, N % 16 == 0, K % 512 == 0) stream w from HBM once (the bound);
- *   other shapes run a tiled MFMA GEMM (128 x 128 tiles, bf16 or fp32 MFMA by operand type). */
+ *   Decode shapes (BF16, T <= 8, N % 16 == 0, K % 512 == 0) stream w from HBM once (the bound), and
+ *   so do up to 32 rows where the tiled GEMM would need a workspace it does not have; other shapes
+ *   run a tiled MFMA GEMM. */
 int smla_linear(const void* x, int x_dtype, const void* w, int w_dtype, int64_t T, int64_t G,
                 int64_t N, int64_t K, void* y, int y_dtype, void* stream);
+
+/* smla_linear with a workspace of smla_linear_workspace(...) bytes (may be 0): products whose output
+ * has too few tiles to occupy the device split their K range over workgroups, whose fp32 partial sums
+ * go through the workspace and are added in a fixed order.  With less workspace (or NULL) it is
+ * smla_linear: the same product without the split. */
+size_t smla_linear_workspace(int64_t T, int64_t G, int64_t N, int64_t K, int x_dtype);
+int smla_linear_ws(const void* x, int x_dtype, const void* w, int w_dtype, int64_t T, int64_t G,
+                   int64_t N, int64_t K, void* y, int y_dtype, void* workspace, size_t workspace_bytes,
+                   void* stream);
 
 /* smla_o_proj: the attention output path of oracle/decode_engine.py:118-119 for T tokens:
  *   o [T, heads, head_dim] BF16; when pos != NULL the last rd dims of every head are rotated back
@@ -444,12 +455,21 @@ int smla_linear(const void* x, int x_dtype, const void* w, int w_dtype, int64_t 
  *   mid [T, G*R] BF16 (caller workspace) = grouped projection with wo_a [G*R, heads*head_dim/G];
  *   y [T, dim] BF16 or F32 = mid @ wo_b^T with wo_b [dim, G*R].  w_dtype: BF16.
  *   Same limits as smla_linear (BF16 operands); with RoPE head_dim % 64 == 0, rd % 64 == 0 and
- *   each group's slice a whole number of heads, and rd == 64 outside the decode shapes.
+ *   each group's slice a whole number of heads, and rd == 64 beyond 32 tokens.
  *   Replaces v4mlx/mla.py:42-56 (o_grouped) after the inverse rotary call. */
 int smla_o_proj(const void* o, int o_dtype, const int32_t* pos, const float* cos_t,
                 const float* sin_t, int64_t n_pos, int64_t T, int64_t heads, int64_t head_dim,
                 int64_t rd, int64_t G, int64_t R, const void* wo_a, const void* wo_b, int w_dtype,
                 int64_t dim, void* mid, void* y, int y_dtype, void* stream);
+
+/* smla_o_proj with a workspace of smla_o_proj_workspace(...) bytes (may be 0; shared by its two
+ * products, as in smla_linear_ws). */
+size_t smla_o_proj_workspace(int64_t T, int64_t heads, int64_t head_dim, int64_t G, int64_t R, int64_t dim);
+int smla_o_proj_ws(const void* o, int o_dtype, const int32_t* pos, const float* cos_t,
+                   const float* sin_t, int64_t n_pos, int64_t T, int64_t heads, int64_t head_dim,
+                   int64_t rd, int64_t G, int64_t R, const void* wo_a, const void* wo_b, int w_dtype,
+                   int64_t dim, void* mid, void* y, int y_dtype, void* workspace, size_t workspace_bytes,
+                   void* stream);
 
 #ifdef __cplusplus
 }

@@ -6,8 +6,8 @@
   accumulation error (1e-5 of sum |x||w|, far below what a dropped K slice or a wrong row would
   change), plus half a bf16 ulp when the output is bf16; with fp32 operands (the tiled GEMM only)
   within (K + 8) 2^-23 of sum |x||w|, twice the textbook bound of a K-term fp32 dot product.
-  Up to 32 bf16 rows run the weight-streaming kernel, other shapes the tiled MFMA GEMM
-  (ragged token and output tiles, K tails, groups, fp32 operands).
+  Up to 8 bf16 rows run the weight-streaming kernel, other shapes the tiled MFMA GEMM
+  (ragged token and output tiles, K tails, groups, fp32 operands, split K ranges).
 * ``smla_o_proj`` with the fused inverse RoPE equals, bit for bit, the standalone inverse rotation
   followed by the unrotated projection, and the oracle's o_project within bf16 tolerance.
 """
@@ -70,6 +70,54 @@ def test_linear_vs_fp64(dev, T, G, N, K, out_dtype, operands):
     torch.cuda.synchronize()
     assert y.dtype == out_dtype and y.shape == (T, G * N)
     _check_linear(y.float(), x, w, G, out_dtype)
+
+
+@pytest.mark.parametrize("T,G,N,K", [
+    # one case or more per tile form of the bf16 GEMM, with ragged tokens and outputs; N not a multiple
+    # of 8 (4) takes the element-wise stores of bf16 (fp32) outputs
+    (9, 1, 48, 128),         # two K steps, one 256 x 256 tile mostly past the edges
+    (40, 1, 72, 192),        # three steps, 128 x 256
+    (70, 1, 333, 512),       # 64 x 64, odd N
+    (65, 3, 90, 1152),       # 64 x 64, four splits of 4 or 5 steps, three groups
+    (33, 1, 1000, 2048),     # 64 x 64, eight splits
+    (150, 1, 520, 4160),     # eight splits of a range they do not divide
+    (130, 2, 4100, 320),     # 64 x 64 over many tiles, five steps
+    (300, 1, 4104, 4096),    # 128 x 128, two splits
+    (420, 1, 4090, 8192),    # the same, N not a multiple of 4
+    (1300, 1, 2050, 2048),   # 128 x 128
+    (700, 8, 1000, 1024),    # 128 x 256, eight groups
+    (257, 1, 32776, 256),    # 128 x 256, one token past two tiles
+    (513, 1, 33000, 128),    # 256 x 256, two steps
+])
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
+def test_linear_tile_forms(dev, T, G, N, K, out_dtype):
+    from smla import ops
+    announce(f"linear tile forms T={T} G={G} N={N} K={K} out={out_dtype}")
+    g = torch.Generator(device=dev).manual_seed(T + N + K)
+    x = torch.randn(T, G * K, generator=g, device=dev).to(torch.bfloat16)
+    w = (torch.randn(G * N, K, generator=g, device=dev) * 0.05).to(torch.bfloat16)
+    y = ops.linear_op(x, w, G, out_dtype)
+    x64, w64 = x.double().view(T, G, K), w.double().view(G, N, K)
+    for i in range(G):       # the bounds of _check_linear, evaluated on the GPU
+        ref, mag = x64[:, i] @ w64[i].t(), x64[:, i].abs() @ w64[i].abs().t()
+        tol = 1e-5 * mag + (ref.abs() * 2.0 ** -8 if out_dtype == torch.bfloat16 else 0.0)
+        assert bool(((y[:, i * N:(i + 1) * N].double() - ref).abs() <= tol).all())
+
+
+@pytest.mark.parametrize("T,G,N,K", [(9, 1, 64, 1536), (17, 2, 48, 1024), (32, 1, 512, 4096), (100, 1, 1024, 4096)])
+def test_linear_without_workspace(dev, T, G, N, K):
+    """smla_linear (no workspace): 9 to 32 rows whose GEMM would split K run the weight-streaming
+    kernel, more rows the GEMM without the split; both as exact as with a workspace."""
+    from smla import _lib
+    announce(f"linear without workspace T={T} G={G} N={N} K={K}")
+    g = torch.Generator().manual_seed(T)
+    x = torch.randn(T, G * K, generator=g).to(torch.bfloat16)
+    w = (torch.randn(G * N, K, generator=g) * 0.05).to(torch.bfloat16)
+    xd, wd, y = x.to(dev), w.to(dev), torch.empty(T, G * N, device=dev)
+    assert _lib.lib().smla_linear_workspace(T, G, N, K, _lib.BF16) > 0
+    _lib.call("smla_linear", xd.data_ptr(), _lib.BF16, wd.data_ptr(), _lib.BF16, T, G, N, K, y.data_ptr(), _lib.F32,
+              torch.cuda.current_stream().cuda_stream)
+    _check_linear(y, x, w, G, torch.float32)
 
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
