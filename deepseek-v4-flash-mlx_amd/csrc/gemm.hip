@@ -27,6 +27,7 @@
 // holds the last rd = 64 dims of a head has its (x0, x1) pairs rotated back to position 0 before it
 // is read (inverse RoPE at pos[t], every product and sum rounded in float32, then bf16), the
 // arithmetic of smla_rope.
+#include "gemm_f32.h"
 #include "gemm_tile.h"
 #include "smla_internal.h"
 
@@ -247,68 +248,27 @@ struct RingArgs {
   int rot;                    // K steps between the starts of neighbouring token tiles
 };
 
-// Workgroup order: the launch deals workgroups to the 8 XCDs round-robin; each XCD takes a
-// contiguous run of tiles, ordered in groups of 4 token tiles over all output tiles, so that the
-// tiles running together on an XCD share x and w rows in its L2.  Splits are outermost.
-template <int FORM, int YDT, bool ROPE>
-__global__ __launch_bounds__((Form<FORM>::BM / Form<FORM>::WM) * (Form<FORM>::BN / Form<FORM>::WN) * 64) void
-gemm_ring_kernel(const RingArgs p) {
+// The tile's outputs from the accumulators (layout of tile_loop) to rows t0 .., columns n0 .. of group g
+// (of split sp's partial sums, with splits).
+// Output rows leave through LDS (each wave its own region, MBP blocks of 32 rows at a time), so that
+// a lane stores 16 bytes and a wave whole 128-byte lines: 16 stores per wave instead of 128 of two
+// bytes per lane, few enough to stay in flight when the wave ends.  Chunk c of row r sits in slot
+// c ^ swizzle(r), so that the two rows of a write (r and r + 4) and the rows of a read use distinct
+// banks.  Nontemporal: the output is not read back by this launch.
+template <class F, int YDT>
+__device__ __attribute__((always_inline)) inline void store_tile(smla_attn::lds_u8_t* lds, const RingArgs& p, int sp,
+                                                                 int g, int t0, int n0,
+                                                                 const f32x16_t (&acc)[F::WM / 32][F::WN / 32]) {
   using namespace smla_gemm;
-  using F = Form<FORM>;
-  constexpr int BM = F::BM, BN = F::BN, WM = F::WM, WN = F::WN, D = F::D;
-  using L = Tile<BM, BN, WM, WN, D>;
-  extern __shared__ __align__(16) uint8_t lds_g[];
-  const uint32_t tot = gridDim.x, per = tot / kXcds, rem = tot % kXcds, xcd = blockIdx.x % kXcds;
-  uint32_t id = xcd * per + (xcd < rem ? xcd : rem) + blockIdx.x / kXcds;
-  const uint32_t tiles = (uint32_t)p.nt * p.nn;
-  const uint32_t sg = id / tiles;  // split * G + group
-  id -= sg * tiles;
-  const int sp = sg / p.G, g = sg - sp * p.G;
-  const uint32_t grp = id / (4u * p.nn), gs = min(4u, (uint32_t)p.nt - 4 * grp), in = id - grp * 4u * p.nn;
-  const int t0 = (4 * grp + in % gs) * BM, n0 = (in / gs) * BN;
-  const int nk = p.K / 64, k0 = nk * sp / p.splits, k1 = nk * (sp + 1) / p.splits;
-  const uint8_t* xk = p.x + (int64_t)t0 * p.ldx + (int64_t)g * p.K * 2 + (int64_t)k0 * kRow;
-  const uint8_t* wk = p.w + ((int64_t)g * p.N + n0) * (int64_t)p.K * 2 + (int64_t)k0 * kRow;
-
-  const int rot = (int)(in % gs) * p.rot % (k1 - k0);
-  // ROPE: the chunks of x this thread rotates in a step that holds a head's last 64 dims: chunk
-  // tid + i threads (row j / 8, slot j mod 8, 4 (x0, x1) pairs from pair 4 c, c = slot ^ ((row / 2) mod
-  // 8)); offsets of their rows in the cos / sin tables (32 pairs per position)
-  constexpr int NT = L::NW * 64, ACH = BM * 8 / NT;
-  int prow[ACH] = {};
-  if constexpr (ROPE) {
-#pragma unroll
-    for (int i = 0; i < ACH; i++) prow[i] = p.pos[min(t0 + (((int)threadIdx.x + NT * i) >> 3), p.T - 1)] * 32;
-  }
-  f32x16_t acc[L::MB][L::NB];
-  tile_loop<BM, BN, WM, WN, D>((lds_u8_t*)lds_g, xk, p.ldx, p.T - 1 - t0, wk, (int64_t)p.K * 2, p.N - 1 - n0, k1 - k0,
-                               rot, acc, [&](int ks, lds_u8_t* stage) __attribute__((always_inline)) {
-    if constexpr (ROPE) {
-      const int k = ks + rot < k1 - k0 ? ks + rot : ks + rot - (k1 - k0);
-      if (((k0 + k) * 64) % p.head_dim == p.head_dim - 64) {
-#pragma unroll
-        for (int i = 0; i < ACH; i++) {
-          const int j = threadIdx.x + NT * i, r = j >> 3, sl = j & 7, c = sl ^ ((r >> 1) & 7);
-          lds_u32x4_t* pa = (lds_u32x4_t*)(stage + r * kRow + 16 * sl);
-          *pa = inv_rope4(*pa, p.cos_t + prow[i] + 4 * c, p.sin_t + prow[i] + 4 * c);
-        }
-        lds_barrier();
-      }
-    }
-  });
-
-  // Output rows leave through LDS (each wave its own region, MBP blocks of 32 rows at a time), so that
-  // a lane stores 16 bytes and a wave whole 128-byte lines: 16 stores per wave instead of 128 of two
-  // bytes per lane, few enough to stay in flight when the wave ends.  Chunk c of row r sits in slot
-  // c ^ swizzle(r), so that the two rows of a write (r and r + 4) and the rows of a read use distinct
-  // banks.  Nontemporal: the output is not read back by this launch.
+  constexpr int BM = F::BM, WM = F::WM, WN = F::WN;
+  using L = Tile<F::BM, F::BN, F::WM, F::WN, F::D>;
   constexpr int ES = YDT == SMLA_BF16 ? 2 : 4, CH = WN * ES / 16, RPI = 64 / CH;  // chunks per row, rows per store
   constexpr int FIT = L::LDS / (L::NW * 32 * WN * ES), MBP = FIT < L::MB ? FIT : L::MB;
   static_assert(MBP >= 1 && L::MB % MBP == 0, "the waves' regions fit the ring's LDS");
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = wave % (BM / WM), wn = wave / (BM / WM);
   const int64_t base = sp * p.split_stride + (int64_t)g * p.N;
   if (p.vec) {  // uniform
-    lds_u8_t* reg = (lds_u8_t*)lds_g + wave * (MBP * 32 * WN * ES);
+    lds_u8_t* reg = lds + wave * (MBP * 32 * WN * ES);
     auto slot = [](int r, int c) { return CH == 16 ? c ^ ((r << 1) & 8) : c ^ (r & (CH - 1)); };
     lds_barrier();  // every wave has read its last fragments
 #pragma unroll
@@ -352,6 +312,131 @@ gemm_ring_kernel(const RingArgs p) {
         }
       }
     }
+}
+
+// Workgroup order: the launch deals workgroups to the 8 XCDs round-robin; each XCD takes a
+// contiguous run of tiles, ordered in groups of 4 token tiles over all output tiles, so that the
+// tiles running together on an XCD share x and w rows in its L2.  Splits are outermost.
+struct TileId {
+  int sp, g, tm, tn, in_group;  // split, group, token tile, output tile; token tile within its 4
+};
+__device__ inline TileId tile_id(const RingArgs& p) {
+  const uint32_t tot = gridDim.x, per = tot / kXcds, rem = tot % kXcds, xcd = blockIdx.x % kXcds;
+  uint32_t id = xcd * per + (xcd < rem ? xcd : rem) + blockIdx.x / kXcds;
+  const uint32_t tiles = (uint32_t)p.nt * p.nn;
+  const uint32_t sg = id / tiles;  // split * G + group
+  id -= sg * tiles;
+  const uint32_t grp = id / (4u * p.nn), gs = min(4u, (uint32_t)p.nt - 4 * grp), in = id - grp * 4u * p.nn;
+  TileId t;
+  t.sp = sg / p.G;
+  t.g = sg - t.sp * p.G;
+  t.in_group = in % gs;
+  t.tm = 4 * grp + t.in_group;
+  t.tn = in / gs;
+  return t;
+}
+
+template <int FORM, int YDT, bool ROPE>
+__global__ __launch_bounds__((Form<FORM>::BM / Form<FORM>::WM) * (Form<FORM>::BN / Form<FORM>::WN) * 64) void
+gemm_ring_kernel(const RingArgs p) {
+  using namespace smla_gemm;
+  using F = Form<FORM>;
+  constexpr int BM = F::BM, BN = F::BN, WM = F::WM, WN = F::WN, D = F::D;
+  using L = Tile<BM, BN, WM, WN, D>;
+  extern __shared__ __align__(16) uint8_t lds_g[];
+  const TileId id = tile_id(p);
+  const int sp = id.sp, g = id.g, t0 = id.tm * BM, n0 = id.tn * BN;
+  const int nk = p.K / 64, k0 = nk * sp / p.splits, k1 = nk * (sp + 1) / p.splits;
+  const uint8_t* xk = p.x + (int64_t)t0 * p.ldx + (int64_t)g * p.K * 2 + (int64_t)k0 * kRow;
+  const uint8_t* wk = p.w + ((int64_t)g * p.N + n0) * (int64_t)p.K * 2 + (int64_t)k0 * kRow;
+
+  const int rot = id.in_group * p.rot % (k1 - k0);
+  // ROPE: the chunks of x this thread rotates in a step that holds a head's last 64 dims: chunk
+  // tid + i threads (row j / 8, slot j mod 8, 4 (x0, x1) pairs from pair 4 c, c = slot ^ ((row / 2) mod
+  // 8)); offsets of their rows in the cos / sin tables (32 pairs per position)
+  constexpr int NT = L::NW * 64, ACH = BM * 8 / NT;
+  int prow[ACH] = {};
+  if constexpr (ROPE) {
+#pragma unroll
+    for (int i = 0; i < ACH; i++) prow[i] = p.pos[min(t0 + (((int)threadIdx.x + NT * i) >> 3), p.T - 1)] * 32;
+  }
+  f32x16_t acc[L::MB][L::NB];
+  tile_loop<BM, BN, WM, WN, D>((lds_u8_t*)lds_g, xk, p.ldx, p.T - 1 - t0, wk, (int64_t)p.K * 2, p.N - 1 - n0, k1 - k0,
+                               rot, acc, [&](int ks, lds_u8_t* stage) __attribute__((always_inline)) {
+    if constexpr (ROPE) {
+      const int k = ks + rot < k1 - k0 ? ks + rot : ks + rot - (k1 - k0);
+      if (((k0 + k) * 64) % p.head_dim == p.head_dim - 64) {
+#pragma unroll
+        for (int i = 0; i < ACH; i++) {
+          const int j = threadIdx.x + NT * i, r = j >> 3, sl = j & 7, c = sl ^ ((r >> 1) & 7);
+          lds_u32x4_t* pa = (lds_u32x4_t*)(stage + r * kRow + 16 * sl);
+          *pa = inv_rope4(*pa, p.cos_t + prow[i] + 4 * c, p.sin_t + prow[i] + 4 * c);
+        }
+        lds_barrier();
+      }
+    }
+  });
+
+  store_tile<F, YDT>((smla_attn::lds_u8_t*)lds_g, p, sp, g, t0, n0, acc);
+}
+
+// fp32 operands with K a multiple of 32 (the K loop of gemm_f32.h); forms of 64 x 64 and 128 x 128
+// outputs, two workgroups per CU.
+template <int FORM>
+struct FormF32;
+template <>
+struct FormF32<0> {
+  static constexpr int BM = 64, BN = 64, WM = 32, WN = 32, D = 4;
+};
+template <>
+struct FormF32<1> {
+  static constexpr int BM = 128, BN = 128, WM = 64, WN = 64, D = 2;
+};
+constexpr int kFormsF32 = 2;
+constexpr int kFormF32B[kFormsF32] = {64, 128}, kFormF32D[kFormsF32] = {FormF32<0>::D, FormF32<1>::D};
+
+template <int FORM, int YDT>
+__global__ __launch_bounds__(256) void gemm_f32_kernel(const RingArgs p) {
+  using namespace smla_gemm;
+  using F = FormF32<FORM>;
+  constexpr int BM = F::BM, BN = F::BN, WM = F::WM, WN = F::WN, D = F::D;
+  using L = Tile<BM, BN, WM, WN, D>;
+  static_assert(L::NW == 4 && L::MB * L::NB * 16 <= 64, "256 threads; a mask bit per accumulator");
+  extern __shared__ __align__(16) uint8_t lds_g[];
+  const TileId id = tile_id(p);
+  const int t0 = id.tm * BM, n0 = id.tn * BN;
+  const int nk = p.K / 32, k0 = nk * id.sp / p.splits, k1 = nk * (id.sp + 1) / p.splits;
+  const uint8_t* xk = p.x + (int64_t)t0 * p.ldx + (int64_t)id.g * p.K * 4 + (int64_t)k0 * kRow;
+  const uint8_t* wk = p.w + ((int64_t)id.g * p.N + n0) * (int64_t)p.K * 4 + (int64_t)k0 * kRow;
+  f32x16_t acc[L::MB][L::NB];
+  tile_loop_f32<BM, BN, WM, WN, D>((lds_u8_t*)lds_g, xk, p.ldx, p.T - 1 - t0, wk, (int64_t)p.K * 4, p.N - 1 - n0, k1 - k0,
+                                   acc);
+  store_tile<F, YDT>((lds_u8_t*)lds_g, p, id.sp, id.g, t0, n0, acc);
+  // nonfinite_fix: a sum that is infinite or NaN may be so only because an operand has no split; it
+  // is computed again as a chain of fp32 fmas (ended by the first NaN, which stays) and stored again,
+  // behind the first store
+  uint64_t bad = 0;
+#pragma unroll
+  for (int i = 0; i < L::MB * L::NB * 16; i++)
+    bad |= (uint64_t)!(__builtin_fabsf(acc[i / 16 / L::NB][i / 16 % L::NB][i % 16]) < SMLA_INF) << i;
+  if (__any(bad != 0)) {
+    wait_vm(0);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = wave % (BM / WM), wn = wave / (BM / WM);
+    while (bad) {
+      const int i = __builtin_ctzll(bad), blk = i / 16, r = i % 16;
+      bad &= bad - 1;
+      const int t = WM * wm + 32 * (blk / L::NB) + 4 * (lane >> 5) + 8 * (r >> 2) + (r & 3);
+      const int n = WN * wn + 32 * (blk % L::NB) + (lane & 31);
+      if (t0 + t >= p.T || n0 + n >= p.N) continue;
+      const float* xr = (const float*)(xk + (int64_t)t * p.ldx);
+      const float* wr = (const float*)wk + (int64_t)n * p.K;
+      float sum = 0.f;
+      for (int k = 0; k < (k1 - k0) * 32 && sum == sum; k++) sum = __builtin_fmaf(xr[k], wr[k], sum);
+      const int64_t o = id.sp * p.split_stride + (int64_t)id.g * p.N + (int64_t)(t0 + t) * p.ldy + n0 + n;
+      if constexpr (YDT == SMLA_BF16) ((uint16_t*)p.y)[o] = bf16_rne(sum);
+      else ((float*)p.y)[o] = sum;
+    }
+  }
 }
 
 // y[i] = part[0][i] + part[1][i] + ... in split order; V elements per thread
@@ -417,6 +502,34 @@ RingPlan ring_plan(int64_t T, int64_t G, int64_t N, int64_t K, bool may_split) {
   return best;
 }
 
+// fp32 operands: the same with its own step times (32 k; the vector ALUs' splits and the MFMAs keep
+// two co-resident workgroups of either form as long as one after the other)
+bool f32_takes(int64_t ldx, int64_t K) {
+  return K % 32 == 0 && K / 32 >= kFormF32D[1] && ldx * 4 * 128 < (1ll << 31) && K * 4 * 128 < (1ll << 31);
+}
+
+RingPlan f32_plan(int64_t T, int64_t G, int64_t N, int64_t K, bool may_split) {
+  constexpr double kIdle[kFormsF32] = {0.5, 1.2}, kBusy[kFormsF32] = {0.6, 1.42};
+  constexpr double kEnds = 2.5, kReduce = 2.0, kHbm = 4.8e6, kPartial = 8 / 4.3e6;
+  const int64_t cus = smla_num_cus(), nk = K / 32;
+  const double in = 4.0 * K * G * (N + T) / kHbm;
+  RingPlan best{1, 1};
+  double bt = 1e30;
+  for (int f = 0; f < kFormsF32; f++) {
+    const int64_t tiles = (T + kFormF32B[f] - 1) / kFormF32B[f] * G * ((N + kFormF32B[f] - 1) / kFormF32B[f]);
+    for (int s = 1; s <= (may_split ? kMaxSplits : 1) && nk / s >= kFormF32D[f]; s++) {
+      const int64_t rest = tiles * s % cus;
+      double t = (double)(tiles * s / cus) * kBusy[f];
+      if (rest > 0) t += kIdle[f] + (kBusy[f] - kIdle[f]) * (double)rest / (double)cus;
+      t *= (double)((nk + s - 1) / s);
+      t = kEnds + (t > in ? t : in);
+      if (s > 1) t += kReduce + s * (double)T * G * N * kPartial;
+      if (t < bt) bt = t, best = {f, s};
+    }
+  }
+  return best;
+}
+
 template <int FORM>
 int launch_ring(const RingArgs& a, int64_t wgs, bool rope, int y_dtype, hipStream_t st) {
   using F = Form<FORM>;
@@ -433,13 +546,24 @@ int launch_ring(const RingArgs& a, int64_t wgs, bool rope, int y_dtype, hipStrea
   return SMLA_OK;
 }
 
+template <int FORM>
+int launch_f32(const RingArgs& a, int64_t wgs, int y_dtype, hipStream_t st) {
+  using F = FormF32<FORM>;
+  using L = smla_gemm::Tile<F::BM, F::BN, F::WM, F::WN, F::D>;
+  auto kern = y_dtype == SMLA_BF16 ? gemm_f32_kernel<FORM, SMLA_BF16> : gemm_f32_kernel<FORM, SMLA_F32>;
+  static_assert(L::LDS <= 64 * 1024, "no raised LDS limit");
+  hipLaunchKernelGGL(kern, dim3((unsigned)wgs), dim3(L::NW * 64), L::LDS, st, a);
+  SMLA_HIP_CHECK_LAUNCH();
+  return SMLA_OK;
+}
+
 }  // namespace
 
 bool gemm_tiled_takes(int64_t G, int64_t K) { return ring_takes(G * K, K); }
 
 int64_t gemm_tiled_workspace(int64_t T, int64_t G, int64_t N, int64_t K, bool f32_operands) {
-  if (f32_operands || !ring_takes(G * K, K)) return 0;
-  const RingPlan p = ring_plan(T, G, N, K, true);
+  if (f32_operands ? !f32_takes(G * K, K) : !ring_takes(G * K, K)) return 0;
+  const RingPlan p = f32_operands ? f32_plan(T, G, N, K, true) : ring_plan(T, G, N, K, true);
   return p.splits > 1 ? p.splits * T * G * N * (int64_t)sizeof(float) : 0;
 }
 
@@ -452,22 +576,23 @@ int launch_gemm_tiled(const void* x, int64_t ldx, bool f32_operands, const void*
                       int64_t K, const int32_t* pos, const float* cos_t, const float* sin_t, int64_t head_dim,
                       void* y, int y_dtype, void* ws, size_t ws_bytes, hipStream_t st) {
   const int64_t ldy = G * N;
-  if (!f32_operands && ring_takes(ldx, K) && (!pos || head_dim % 64 == 0)) {
-    const int64_t need = gemm_tiled_workspace(T, G, N, K, false);
+  if (f32_operands ? f32_takes(ldx, K) : ring_takes(ldx, K) && (!pos || head_dim % 64 == 0)) {
+    const int64_t need = gemm_tiled_workspace(T, G, N, K, f32_operands);
     const bool split = need > 0 && ws && ws_bytes >= (size_t)need;
-    const RingPlan p = ring_plan(T, G, N, K, split);
-    const int bm = kFormBM[p.form], bn = kFormBN[p.form];
+    const RingPlan p = f32_operands ? f32_plan(T, G, N, K, split) : ring_plan(T, G, N, K, split);
+    const int bm = f32_operands ? kFormF32B[p.form] : kFormBM[p.form], bn = f32_operands ? bm : kFormBN[p.form];
     const int64_t nt = (T + bm - 1) / bm, nn = (N + bn - 1) / bn, wgs = nt * nn * G * p.splits;
     if (wgs > 0x7fffffff) return SMLA_E_UNSUPPORTED;
-    RingArgs a{(const uint8_t*)x, (const uint8_t*)w, ldx * 2, (int)T, (int)N, (int)K, (int)G, (int)nt, (int)nn, p.splits,
-               pos, cos_t, sin_t, (int)head_dim, (uint8_t*)(p.splits > 1 ? ws : y), ldy, T * ldy, 0, 0};
+    RingArgs a{(const uint8_t*)x, (const uint8_t*)w, ldx * (f32_operands ? 4 : 2), (int)T, (int)N, (int)K, (int)G, (int)nt,
+               (int)nn, p.splits, pos, cos_t, sin_t, (int)head_dim, (uint8_t*)(p.splits > 1 ? ws : y), ldy, T * ldy, 0, 0};
     const int odt = p.splits > 1 ? SMLA_F32 : y_dtype;
     // rows of x 64 KB apart fall in the same sets of an L2, which the 4 token tiles of a group would
     // then all want at once: they start 4 steps apart (8 groups of [4096, 4096] x [1024, 4096]^T 281 ->
     // 262 us; with closer rows, which it does not help, a rotation costs up to 3 %)
-    a.rot = p.form == 3 && a.ldx % 65536 == 0 ? 4 : 0;
+    a.rot = !f32_operands && p.form == 3 && a.ldx % 65536 == 0 ? 4 : 0;
     a.vec = N % (odt == SMLA_BF16 ? 8 : 4) == 0 && ((uintptr_t)a.y & 15) == 0;
-    const int rc = p.form == 0   ? launch_ring<0>(a, wgs, pos != nullptr, odt, st)
+    const int rc = f32_operands  ? (p.form == 0 ? launch_f32<0>(a, wgs, odt, st) : launch_f32<1>(a, wgs, odt, st))
+                   : p.form == 0 ? launch_ring<0>(a, wgs, pos != nullptr, odt, st)
                    : p.form == 1 ? launch_ring<1>(a, wgs, pos != nullptr, odt, st)
                    : p.form == 2 ? launch_ring<2>(a, wgs, pos != nullptr, odt, st)
                                  : launch_ring<3>(a, wgs, pos != nullptr, odt, st);

@@ -1,0 +1,160 @@
+// The K loop of the tiled fp32 product (gemm.hip): one workgroup's BM x BN tile of x . w^T, both
+// operands K-contiguous fp32, on the bf16 matrix cores.
+//
+// An fp32 value is the sum of three bf16 values, x = h + m + l, each the top 8 significant bits of what
+// is left: exact while the lowest bit of x is a bf16 (|x| >= 2^-110; below, bits under 2^-133 are lost).
+// x w = hh + (hm + mh) + (hl + lh + mm) up to terms of 2^-23 |x w| on average: the products of bf16
+// values are exact in fp32 and v_mfma_f32_32x32x16_bf16 adds 16 k of one of them per accumulator
+// rounding, against one rounding per k (or two) of a chain of fp32 fmas.  Distance from float64
+// (relative, 2-norm; uniform operands): 1.0e-6 for K = 4096 and 4.9e-7 for K = 1024 in one chain, 6.4e-7
+// and 3.5e-7 in two splits; the fp32 MFMAs 1.1e-6 and 5.9e-7.  An operand that the split cannot carry
+// (infinite or NaN) makes the sum non-finite, and every non-finite sum is recomputed as an fp32 fma
+// chain (nonfinite_fix), so infinities and NaN come out as fp32 arithmetic gives them.
+//
+// Six bf16 MFMAs carry 16 k in 192 cycles per 32 x 32 block where the fp32 MFMAs take 512.  [2046, 4096] x
+// [2048, 4096]^T: 394 us with fp32 MFMAs and register staging, 184 us here (186 TFLOP/s; the fp32 MFMA
+// peak is 157); [1, 8192] x [4096, 8192]^T 710 -> 43 us.
+//
+// What bounds it is the vector ALU work of the splits (11 instructions per pair of values, done by
+// every wave that reads them) beside the MFMAs: either takes about 55 % of the cycles, and they
+// overlap only in part (rounding the parts instead of truncating them, 1.5 times the MFMAs per split,
+// two waves per SIMD: all within 4 % of the same time).  The splits of the next 16 k are therefore interleaved with the MFMAs of the current ones, and
+// the raw values of the 16 k after those are read from LDS meanwhile (two register sets of each).
+#pragma once
+
+#include "gemm_tile.h"
+
+namespace smla_gemm {
+
+struct Split3 {
+  bf16x8_t h, m, l;
+};
+
+// the high halves of a (low word) and b (high word): both truncated to bf16
+__device__ inline uint32_t top_halves(float a, float b) {
+  return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
+}
+__device__ inline float below_top(float a) { return a - __uint_as_float(__float_as_uint(a) & 0xffff0000u); }
+
+__device__ inline Split3 split3(u32x4_t lo, u32x4_t hi) {
+  u32x4_t h, m, l;
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    const float a = __uint_as_float(j < 2 ? lo[2 * j] : hi[2 * j - 4]);
+    const float b = __uint_as_float(j < 2 ? lo[2 * j + 1] : hi[2 * j - 3]);
+    const float a1 = below_top(a), b1 = below_top(b);
+    h[j] = top_halves(a, b);
+    m[j] = top_halves(a1, b1);
+    l[j] = top_halves(below_top(a1), below_top(b1));
+  }
+  return {as_bf16x8(h), as_bf16x8(m), as_bf16x8(l)};
+}
+
+// acc[mb][nb] = rows 0 .. BM-1 of x times rows 0 .. BN-1 of w over nk >= D steps of 32 k; arguments and
+// accumulator layout as tile_loop's.  Rows of 128 bytes (32 k) as there; the ring is one step further
+// ahead: step s + 1 is read from LDS while step s is multiplied.
+template <int BM, int BN, int WM, int WN, int D>
+__device__ __attribute__((always_inline)) inline void tile_loop_f32(lds_u8_t* lds, const uint8_t* __restrict__ xk,
+                                                                    int64_t ldx, int tmax,
+                                                                    const uint8_t* __restrict__ wk, int64_t ldw,
+                                                                    int nmax, int nk,
+                                                                    f32x16_t (&acc)[WM / 32][WN / 32]) {
+  using L = Tile<BM, BN, WM, WN, D>;
+  constexpr int MB = L::MB, NB = L::NB, NR = MB + NB;
+  const uint32_t lds_base = (uint32_t)(uintptr_t)lds;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave % (BM / WM), wn = wave / (BM / WM);
+  uint32_t off[L::CP];
+#pragma unroll
+  for (int i = 0; i < L::CP; i++) {
+    const int q = wave * L::CP + i;
+    const bool isx = q < BM / 8;
+    const int r = 8 * (isx ? q : q - BM / 8) + (lane >> 3);
+    const int c = (lane & 7) ^ ((r >> 1) & 7);
+    off[i] = (isx ? (uint32_t)min(r, tmax) * (uint32_t)ldx : (uint32_t)min(r, nmax) * (uint32_t)ldw) + 16 * c;
+  }
+  auto copy = [&](int ks) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < L::CP; i++) {
+      const int q = wave * L::CP + i;
+      dma16_s((q < BM / 8 ? xk : wk) + (int64_t)ks * kRow, off[i], lds_base + (ks % D) * L::STAGE + q * 1024);
+    }
+  };
+  // a fragment is 8 k of a row, k 16 kk + 8 (lane / 32) ..: chunks 4 kk + 2 (lane / 32) and the next
+  const int r32 = lane & 31, kh = lane >> 5, sw = (r32 >> 1) & 7;
+  const uint32_t xrow = (WM * wm + r32) * kRow, wrow = BM * kRow + (WN * wn + r32) * kRow;
+  u32x4_t raw[2][NR][2];
+  Split3 sp[2][NR];
+  auto read = [&](int ks, auto kk_) __attribute__((always_inline)) {
+    constexpr int kk = decltype(kk_)::value;
+    const lds_u8_t* st = lds + (ks % D) * L::STAGE;
+#pragma unroll
+    for (int i = 0; i < NR; i++)
+#pragma unroll
+      for (int e = 0; e < 2; e++)
+        raw[kk][i][e] = *(const lds_u32x4_t*)(st + (i < MB ? xrow + 32 * kRow * i : wrow + 32 * kRow * (i - MB)) +
+                                              16 * ((4 * kk + 2 * kh + e) ^ sw));
+  };
+  auto split = [&](auto kk_) __attribute__((always_inline)) {
+    constexpr int kk = decltype(kk_)::value;
+#pragma unroll
+    for (int i = 0; i < NR; i++) sp[kk][i] = split3(raw[kk][i][0], raw[kk][i][1]);
+  };
+  // the MFMAs of sub-step kk, small products first, the blocks alternating so that an accumulator
+  // is not wanted again at once
+  auto mul = [&](auto kk_) __attribute__((always_inline)) {
+    constexpr int kk = decltype(kk_)::value;
+#pragma unroll
+    for (int p = 0; p < 6; p++)
+#pragma unroll
+      for (int j = 0; j < MB * NB; j++) {
+        const Split3 &a = sp[kk][j / NB], &b = sp[kk][MB + j % NB];
+        const bf16x8_t u = p == 0 ? a.m : p == 1 ? a.l : p == 3 ? a.m : a.h;
+        const bf16x8_t v = p == 0 ? b.m : p == 2 ? b.l : p == 4 ? b.m : b.h;
+        acc[j / NB][j % NB] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(u, v, acc[j / NB][j % NB], 0, 0, 0);
+      }
+  };
+  auto pin = [&]() __attribute__((always_inline)) {
+    constexpr int V = (NR * 44 + 6 * MB * NB - 1) / (6 * MB * NB);
+#pragma unroll
+    for (int j = 0; j < 6 * MB * NB; j++) {
+      __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);  // MFMA
+      __builtin_amdgcn_sched_group_barrier(0x2, V, 0);  // VALU
+    }
+  };
+#pragma unroll
+  for (int m = 0; m < MB; m++)
+#pragma unroll
+    for (int n = 0; n < NB; n++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) acc[m][n][r] = 0.f;
+#pragma unroll
+  for (int s = 0; s < D; s++) copy(s);
+  wait_vm((D - 1) * L::CP);
+  lds_barrier();
+  read(0, Int<0>{});
+  read(0, Int<1>{});
+  split(Int<0>{});
+  auto step = [&](int ks, auto more_, auto next_) __attribute__((always_inline)) {
+    constexpr int more = decltype(more_)::value, next = decltype(next_)::value;
+    if constexpr (next) {
+      wait_vm(more ? (D - 2) * L::CP : 0);  // this wave's copies of step ks + 1
+      lds_barrier();                         // everyone's; and step ks is in every wave's registers
+      if constexpr (more) copy(ks + D);
+      read(ks + 1, Int<0>{});
+    }
+    mul(Int<0>{});
+    split(Int<1>{});
+    pin();
+    if constexpr (next) read(ks + 1, Int<1>{});
+    mul(Int<1>{});
+    if constexpr (next) split(Int<0>{});
+    pin();
+  };
+  int ks = 0;
+  for (; ks < nk - D; ks++) step(ks, Int<1>{}, Int<1>{});
+  for (; ks < nk - 1; ks++) step(ks, Int<0>{}, Int<1>{});
+  step(ks, Int<0>{}, Int<0>{});
+}
+
+}  // namespace smla_gemm

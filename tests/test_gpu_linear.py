@@ -104,6 +104,52 @@ def test_linear_tile_forms(dev, T, G, N, K, out_dtype):
         assert bool(((y[:, i * N:(i + 1) * N].double() - ref).abs() <= tol).all())
 
 
+@pytest.mark.parametrize("T,G,N,K", [
+    (1, 1, 1024, 4096),      # 64 x 64 tiles, eight splits
+    (70, 1, 333, 512),       # odd N: element-wise stores
+    (129, 2, 136, 64),       # two steps of 32 k: 128 x 128 tiles, one token past the first
+    (65, 3, 90, 160),        # five steps, three groups
+    (700, 1, 2050, 1056),    # 128 x 128 tiles, ragged
+])
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
+def test_linear_fp32_tiles(dev, T, G, N, K, out_dtype):
+    """fp32 operands on the bf16 matrix cores (three bf16 parts per value), by the bound of an fp32
+    dot product."""
+    from smla import ops
+    announce(f"linear fp32 T={T} G={G} N={N} K={K} out={out_dtype}")
+    g = torch.Generator().manual_seed(T + N + K)
+    x = torch.randn(T, G * K, generator=g) * torch.exp2(torch.randint(-20, 20, (T, 1), generator=g).float())
+    w = torch.randn(G * N, K, generator=g) * 0.05
+    y = ops.linear_op(x.to(dev), w.to(dev), G, out_dtype)
+    _check_linear(y.float(), x, w, G, out_dtype)
+
+
+@pytest.mark.parametrize("T,N,K", [(40, 130, 4096), (300, 600, 96)])    # with and without splits
+def test_linear_fp32_special_values(dev, T, N, K):
+    """Infinities, NaN, values whose bf16 rounding overflows and subnormals come out as fp32 arithmetic
+    gives them: the same places infinite and NaN, the rest within the fp32 bound plus what the split
+    leaves of an operand below 2^-110, at most 2^-133 (the last bit of a subnormal bf16)."""
+    from smla import ops
+    announce(f"linear fp32 special values T={T} N={N} K={K}")
+    g = torch.Generator().manual_seed(T)
+    x, w = torch.randn(T, K, generator=g), torch.randn(N, K, generator=g) * 0.05
+    x[0, 3], x[1, 5], x[2, 7], x[3, 9] = float("inf"), float("nan"), 3.4028234e38, -3.4e38
+    x[4] *= 1e-36
+    x[5] *= 1e-40
+    w[4, 3] = 0.0                                   # inf * 0
+    w[6, 11], x[6, 11] = float("-inf"), 2.0
+    y = ops.linear_op(x.to(dev), w.to(dev), 1, torch.float32).cpu()
+    ref = x.double() @ w.double().t()
+    assert torch.equal(torch.isnan(y), torch.isnan(ref))
+    inf = torch.isinf(ref)
+    assert torch.equal(torch.isinf(y), inf) and torch.equal(y[inf].double(), ref[inf])
+    ok = torch.isfinite(ref)
+    xf, wf = torch.nan_to_num(x.double(), 0, 0, 0), torch.nan_to_num(w.double(), 0, 0, 0)
+    tol = (K + 8) * 2.0 ** -23 * (xf.abs() @ wf.abs().t()) \
+        + 2.0 ** -133 * (xf.abs().sum(1)[:, None] + wf.abs().sum(1)[None]) + K * 2.0 ** -149
+    assert bool(((y.double() - ref).abs()[ok] <= tol[ok]).all())
+
+
 @pytest.mark.parametrize("T,G,N,K", [(9, 1, 64, 1536), (17, 2, 48, 1024), (32, 1, 512, 4096), (100, 1, 1024, 4096)])
 def test_linear_without_workspace(dev, T, G, N, K):
     """smla_linear (no workspace): 9 to 32 rows whose GEMM would split K run the weight-streaming
