@@ -236,7 +236,9 @@ constexpr int kMaxSplits = 8;
 struct RingArgs {
   const uint8_t* x;
   const uint8_t* w;
-  int64_t ldx;  // bytes
+  const uint8_t* w2;  // the second group's weights (else group g's follow group g - 1's)
+  int64_t ldx;        // bytes
+  int64_t xg;         // bytes between the groups' slices of a row of x
   int T, N, K, G, nt, nn, splits;
   const int32_t* pos;
   const float* cos_t;
@@ -336,6 +338,10 @@ __device__ inline TileId tile_id(const RingArgs& p) {
   return t;
 }
 
+__device__ inline const uint8_t* group_weights(const RingArgs& p, int g, int es) {
+  return p.w2 && g > 0 ? p.w2 : p.w + (int64_t)g * p.N * (int64_t)p.K * es;
+}
+
 template <int FORM, int YDT, bool ROPE>
 __global__ __launch_bounds__((Form<FORM>::BM / Form<FORM>::WM) * (Form<FORM>::BN / Form<FORM>::WN) * 64) void
 gemm_ring_kernel(const RingArgs p) {
@@ -347,8 +353,8 @@ gemm_ring_kernel(const RingArgs p) {
   const TileId id = tile_id(p);
   const int sp = id.sp, g = id.g, t0 = id.tm * BM, n0 = id.tn * BN;
   const int nk = p.K / 64, k0 = nk * sp / p.splits, k1 = nk * (sp + 1) / p.splits;
-  const uint8_t* xk = p.x + (int64_t)t0 * p.ldx + (int64_t)g * p.K * 2 + (int64_t)k0 * kRow;
-  const uint8_t* wk = p.w + ((int64_t)g * p.N + n0) * (int64_t)p.K * 2 + (int64_t)k0 * kRow;
+  const uint8_t* xk = p.x + (int64_t)t0 * p.ldx + g * p.xg + (int64_t)k0 * kRow;
+  const uint8_t* wk = group_weights(p, g, 2) + (int64_t)n0 * p.K * 2 + (int64_t)k0 * kRow;
 
   const int rot = id.in_group * p.rot % (k1 - k0);
   // ROPE: the chunks of x this thread rotates in a step that holds a head's last 64 dims: chunk
@@ -406,8 +412,8 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const RingArgs p) {
   const TileId id = tile_id(p);
   const int t0 = id.tm * BM, n0 = id.tn * BN;
   const int nk = p.K / 32, k0 = nk * id.sp / p.splits, k1 = nk * (id.sp + 1) / p.splits;
-  const uint8_t* xk = p.x + (int64_t)t0 * p.ldx + (int64_t)id.g * p.K * 4 + (int64_t)k0 * kRow;
-  const uint8_t* wk = p.w + ((int64_t)id.g * p.N + n0) * (int64_t)p.K * 4 + (int64_t)k0 * kRow;
+  const uint8_t* xk = p.x + (int64_t)t0 * p.ldx + id.g * p.xg + (int64_t)k0 * kRow;
+  const uint8_t* wk = group_weights(p, id.g, 4) + (int64_t)n0 * p.K * 4 + (int64_t)k0 * kRow;
   f32x16_t acc[L::MB][L::NB];
   tile_loop_f32<BM, BN, WM, WN, D>((lds_u8_t*)lds_g, xk, p.ldx, p.T - 1 - t0, wk, (int64_t)p.K * 4, p.N - 1 - n0, k1 - k0,
                                    acc);
@@ -571,10 +577,11 @@ int64_t gemm_tiled_workspace(int64_t T, int64_t G, int64_t N, int64_t K, bool f3
 // x and w both bf16 (f32_operands false) or both fp32; y bf16 or fp32.  With pos (bf16 only), inverse RoPE
 // of the last 64 dims of every head_dim-wide head of x on load.  16-byte aligned rows (K % 8 for
 // bf16, K % 4 for fp32).  ws: gemm_tiled_workspace bytes for the partial sums of a split K range, or
-// less (null): the plan without splits.  Returns SMLA_OK or a hipError_t.
+// less (null): the plan without splits.  With w2, G = 2 groups of weights w and w2 that both multiply
+// the same x [T, K] (shapes the ring kernels take, else SMLA_E_UNSUPPORTED).  Returns SMLA_OK or a hipError_t.
 int launch_gemm_tiled(const void* x, int64_t ldx, bool f32_operands, const void* w, int64_t T, int64_t G, int64_t N,
                       int64_t K, const int32_t* pos, const float* cos_t, const float* sin_t, int64_t head_dim,
-                      void* y, int y_dtype, void* ws, size_t ws_bytes, hipStream_t st) {
+                      void* y, int y_dtype, void* ws, size_t ws_bytes, hipStream_t st, const void* w2) {
   const int64_t ldy = G * N;
   if (f32_operands ? f32_takes(ldx, K) : ring_takes(ldx, K) && (!pos || head_dim % 64 == 0)) {
     const int64_t need = gemm_tiled_workspace(T, G, N, K, f32_operands);
@@ -583,7 +590,8 @@ int launch_gemm_tiled(const void* x, int64_t ldx, bool f32_operands, const void*
     const int bm = f32_operands ? kFormF32B[p.form] : kFormBM[p.form], bn = f32_operands ? bm : kFormBN[p.form];
     const int64_t nt = (T + bm - 1) / bm, nn = (N + bn - 1) / bn, wgs = nt * nn * G * p.splits;
     if (wgs > 0x7fffffff) return SMLA_E_UNSUPPORTED;
-    RingArgs a{(const uint8_t*)x, (const uint8_t*)w, ldx * (f32_operands ? 4 : 2), (int)T, (int)N, (int)K, (int)G, (int)nt,
+    const int64_t es = f32_operands ? 4 : 2;
+    RingArgs a{(const uint8_t*)x, (const uint8_t*)w, (const uint8_t*)w2, ldx * es, w2 ? 0 : K * es, (int)T, (int)N, (int)K, (int)G, (int)nt,
                (int)nn, p.splits, pos, cos_t, sin_t, (int)head_dim, (uint8_t*)(p.splits > 1 ? ws : y), ldy, T * ldy, 0, 0};
     const int odt = p.splits > 1 ? SMLA_F32 : y_dtype;
     // rows of x 64 KB apart fall in the same sets of an L2, which the 4 token tiles of a group would
@@ -606,6 +614,7 @@ int launch_gemm_tiled(const void* x, int64_t ldx, bool f32_operands, const void*
     SMLA_HIP_CHECK_LAUNCH();
     return SMLA_OK;
   }
+  if (w2) return SMLA_E_UNSUPPORTED;
   const int64_t ntn = (N + kBN - 1) / kBN;
   const dim3 grid((unsigned)(ntn * G), (unsigned)((T + kBM - 1) / kBM)), blk(256);
 #define SMLA_GEMM(BF, YD, RP)                                                                                   \

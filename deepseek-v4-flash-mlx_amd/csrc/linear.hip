@@ -413,6 +413,22 @@ extern "C" int smla_linear(const void* x, int x_dtype, const void* w, int w_dtyp
   return smla_linear_ws(x, x_dtype, w, w_dtype, T, G, N, K, y, y_dtype, nullptr, 0, stream);
 }
 
+extern "C" int smla_linear_pair_ws(const void* x, int x_dtype, const void* w0, const void* w1, int w_dtype, int64_t T,
+                                   int64_t N, int64_t K, void* y, int y_dtype, void* workspace,
+                                   size_t workspace_bytes, void* stream) {
+  if (!w1) return SMLA_E_NULL;
+  int rc = check_linear(x, x_dtype, w0, w_dtype, T, 2, N, K, y, y_dtype);
+  if (rc) return rc;
+  if (((uintptr_t)w1 & 15) || K % (x_dtype == SMLA_BF16 ? 8 : 4) != 0) return SMLA_E_UNSUPPORTED;
+  return launch_gemm_tiled(x, K, x_dtype == SMLA_F32, w0, T, 2, N, K, nullptr, nullptr, nullptr, 0, y, y_dtype,
+                           workspace, workspace_bytes, (hipStream_t)stream, w1);
+}
+
+extern "C" size_t smla_linear_pair_workspace(int64_t T, int64_t N, int64_t K, int x_dtype) {
+  if (T <= 0 || N <= 0 || K <= 0) return 0;
+  return (size_t)gemm_tiled_workspace(T, 2, N, K, x_dtype == SMLA_F32);
+}
+
 extern "C" size_t smla_linear_workspace(int64_t T, int64_t G, int64_t N, int64_t K, int x_dtype) {
   if (T <= 0 || G <= 0 || N <= 0 || K <= 0 || decode_runs(x_dtype, T, G, N, K, true, true)) return 0;
   return (size_t)gemm_tiled_workspace(T, G, N, K, x_dtype == SMLA_F32);

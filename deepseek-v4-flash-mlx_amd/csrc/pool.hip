@@ -218,7 +218,7 @@ constexpr int kMaxRatio = 8;
 __global__ __launch_bounds__(kPoolThreads) void gated_pool_kernel(
     const float* __restrict__ kv, const float* __restrict__ score, const float* __restrict__ ape,
     const float* __restrict__ norm_w, const float* __restrict__ cos_t, const float* __restrict__ sin_t, int64_t N,
-    int d, int ratio, int rd, float eps, int sim, float* __restrict__ out) {
+    int d, int ratio, int rd, float eps, int sim, int64_t ld, int64_t ldb, float* __restrict__ out) {
   __shared__ float red[kPoolThreads / 64];
   __shared__ float xch[2 * kPoolThreads];
   const int64_t G = N / ratio;
@@ -233,8 +233,8 @@ __global__ __launch_bounds__(kPoolThreads) void gated_pool_kernel(
   float v0[2 * kMaxRatio], s0[2 * kMaxRatio], v1[2 * kMaxRatio], s1[2 * kMaxRatio];
   int ns = 0;
   auto slot = [&](int64_t row, int64_t off, int j) __attribute__((always_inline)) {
-    const f32x2_t kvv = *(const f32x2_t*)(kv + row * two_d + off + c0);
-    const f32x2_t sc = *(const f32x2_t*)(score + row * two_d + off + c0);
+    const f32x2_t kvv = *(const f32x2_t*)(kv + b * ldb + row * ld + off + c0);
+    const f32x2_t sc = *(const f32x2_t*)(score + b * ldb + row * ld + off + c0);
     const f32x2_t ap = *(const f32x2_t*)(ape + j * two_d + off + c0);
     v0[ns] = kvv[0];
     v1[ns] = kvv[1];
@@ -243,8 +243,8 @@ __global__ __launch_bounds__(kPoolThreads) void gated_pool_kernel(
     ns++;
   };
   if (g > 0)
-    for (int j = 0; j < ratio; j++) slot(b * N + (g - 1) * ratio + j, 0, j);
-  for (int j = 0; j < ratio; j++) slot(b * N + g * ratio + j, d, j);
+    for (int j = 0; j < ratio; j++) slot((g - 1) * ratio + j, 0, j);
+  for (int j = 0; j < ratio; j++) slot(g * ratio + j, d, j);
   float pooled[2];
   pooled[0] = softmax_pool<2 * kMaxRatio>(v0, s0, ns);
   pooled[1] = softmax_pool<2 * kMaxRatio>(v1, s1, ns);
@@ -453,6 +453,12 @@ static int check_pool_dims(int64_t d, int64_t ratio, int64_t rd, int sim) {
 extern "C" int smla_gated_pool(const float* kv, const float* score, const float* ape, const float* norm_w,
                                const float* cos_t, const float* sin_t, int64_t B, int64_t N, int64_t d, int64_t ratio,
                                int64_t rd, float eps, int sim, float* out, void* stream) {
+  return smla_gated_pool_ld(kv, score, 0, 0, ape, norm_w, cos_t, sin_t, B, N, d, ratio, rd, eps, sim, out, stream);
+}
+
+extern "C" int smla_gated_pool_ld(const float* kv, const float* score, int64_t ld, int64_t ld_batch, const float* ape,
+                                  const float* norm_w, const float* cos_t, const float* sin_t, int64_t B, int64_t N,
+                                  int64_t d, int64_t ratio, int64_t rd, float eps, int sim, float* out, void* stream) {
   if (!kv || !score || !ape || !norm_w || !cos_t || !sin_t || !out) return SMLA_E_NULL;
   if (B <= 0 || N <= 0) return SMLA_E_SHAPE;
   int rc = check_pool_dims(d, ratio, rd, sim);
@@ -460,10 +466,14 @@ extern "C" int smla_gated_pool(const float* kv, const float* score, const float*
   if (N % ratio != 0) return SMLA_E_SHAPE;
   // the kernel reads two adjacent channels of kv, score and ape in one 8-byte load
   if ((((uintptr_t)kv | (uintptr_t)score | (uintptr_t)ape) & 7) != 0) return SMLA_E_UNSUPPORTED;
+  if (ld == 0) ld = 2 * d;
+  if (ld_batch == 0) ld_batch = N * ld;
+  if (ld < 2 * d || ld_batch < 0) return SMLA_E_SHAPE;
+  if (ld % 2 != 0 || ld_batch % 2 != 0) return SMLA_E_UNSUPPORTED;
   int64_t rows = B * (N / ratio);
   if (rows <= 0) return SMLA_OK;
   hipLaunchKernelGGL(gated_pool_kernel, dim3((unsigned)rows), dim3((unsigned)(d / 2)), 0, (hipStream_t)stream, kv,
-                     score, ape, norm_w, cos_t, sin_t, N, (int)d, (int)ratio, (int)rd, eps, sim, out);
+                     score, ape, norm_w, cos_t, sin_t, N, (int)d, (int)ratio, (int)rd, eps, sim, ld, ld_batch, out);
   SMLA_HIP_CHECK_LAUNCH();
   return SMLA_OK;
 }

@@ -296,10 +296,11 @@ __device__ inline void store_from_f32(void* p, int64_t i, int dtype, float v) {
 // tiled MFMA GEMM (gemm.hip): y [T, G*N] = grouped x [T, G*K] (row stride ldx) times w [G*N, K]^T,
 // operands both bf16 or both fp32 (f32_operands), y bf16 or fp32; with pos, inverse RoPE of the
 // last 64 dims of every head_dim-wide head of x (bf16) as it is loaded.  With gemm_tiled_workspace
-// bytes of workspace, few tiles split their K range; with less they do not.
+// bytes of workspace, few tiles split their K range; with less they do not.  With w2, G = 2 and both
+// weights multiply the same x (SMLA_E_UNSUPPORTED for shapes only gemm_kernel takes).
 int launch_gemm_tiled(const void* x, int64_t ldx, bool f32_operands, const void* w, int64_t T, int64_t G, int64_t N,
                       int64_t K, const int32_t* pos, const float* cos_t, const float* sin_t, int64_t head_dim,
-                      void* y, int y_dtype, void* ws, size_t ws_bytes, hipStream_t st);
+                      void* y, int y_dtype, void* ws, size_t ws_bytes, hipStream_t st, const void* w2 = nullptr);
 // whether bf16 operands run its ring kernel; bytes of the partial sums its plan splits K into (0: none)
 bool gemm_tiled_takes(int64_t G, int64_t K);
 int64_t gemm_tiled_workspace(int64_t T, int64_t G, int64_t N, int64_t K, bool f32_operands);

@@ -50,6 +50,8 @@ _SIGNATURES = {
     "smla_block_mean_pool": (_int, [_vp, _int, _i64, _i64, _i64, _i64, _vp, _int, _vp]),
     "smla_gated_pool": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _f32,
                                _int, _vp, _vp]),
+    "smla_gated_pool_ld": (_int, [_vp, _vp, _i64, _i64, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _f32,
+                                  _int, _vp, _vp]),
     "smla_ring_step": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64,
                               _f32, _int, _vp, _i64, _i64, _vp]),
     "smla_ring_step_kv": (_int, [_vp] * 9 + [_i64] * 5 + [_f32, _int, _vp, _i64, _i64, _vp, _i64, _vp, _vp, _vp,
@@ -65,6 +67,8 @@ _SIGNATURES = {
     "smla_linear": (_int, [_vp, _int, _vp, _int, _i64, _i64, _i64, _i64, _vp, _int, _vp]),
     "smla_linear_workspace": (_sz, [_i64, _i64, _i64, _i64, _int]),
     "smla_linear_ws": (_int, [_vp, _int, _vp, _int, _i64, _i64, _i64, _i64, _vp, _int, _vp, _sz, _vp]),
+    "smla_linear_pair_workspace": (_sz, [_i64, _i64, _i64, _int]),
+    "smla_linear_pair_ws": (_int, [_vp, _int, _vp, _vp, _int, _i64, _i64, _i64, _vp, _int, _vp, _sz, _vp]),
     "smla_o_proj_workspace": (_sz, [_i64] * 6),
     "smla_o_proj_ws": (_int, [_vp, _int, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _vp, _vp, _int,
                               _i64, _vp, _vp, _int, _vp, _sz, _vp]),

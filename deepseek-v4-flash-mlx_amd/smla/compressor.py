@@ -57,16 +57,20 @@ def compressor_prefill(x, wkv, wgate, ape, norm_w, head_dim=512, ratio=4, rope_h
 
 
 def project_pair(x, wkv, wgate):
-    """(x @ wkv^T, x @ wgate^T) as fp32 [b, s, 2*head_dim] each, from one ``smla_linear`` call over
-    the stacked weights: fp32 operands unless x and both weights are bf16."""
+    """(x @ wkv^T, x @ wgate^T) as fp32 [b, s, 2*head_dim] each, from one launch: fp32 operands unless
+    x and both weights are bf16.  The two weights are read where they are when they match (shape,
+    dtype, alignment) and the tiled GEMM takes them; else they are stacked first."""
     b, s, dim = x.shape
-    wcat = torch.cat([wkv, wgate], dim=0)
-    if x.dtype == torch.bfloat16 and wcat.dtype == torch.bfloat16:
-        y = ops.linear_op(x.reshape(b * s, dim), wcat, 1, torch.float32)
-    else:
-        y = ops.linear_op(x.float().reshape(b * s, dim), wcat.float(), 1, torch.float32)
-    y = y.reshape(b, s, -1)
+    dt = torch.bfloat16 if x.dtype == wkv.dtype == wgate.dtype == torch.bfloat16 else torch.float32
+    x = x.to(dt).reshape(b * s, dim)
     n = wkv.shape[0]
+    if (b * s > 8 and dim % 64 == 0 and 128 <= dim <= 1 << 20 and wkv.dim() == 2 and wkv.shape == wgate.shape
+            and wkv.shape[1] == dim and all(w.dtype == dt and w.is_contiguous() and w.data_ptr() % 16 == 0
+                                            for w in (wkv, wgate)) and x.data_ptr() % 16 == 0):
+        y = ops.linear_pair_op(x, wkv, wgate)
+    else:
+        y = ops.linear_op(x, torch.cat([wkv, wgate], dim=0).to(dt), 1, torch.float32)
+    y = y.reshape(b, s, -1)
     return y[..., :n], y[..., n:]
 
 

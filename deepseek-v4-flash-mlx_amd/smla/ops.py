@@ -302,7 +302,13 @@ def gated_pool_op(kv: torch.Tensor, score: torch.Tensor, ape: torch.Tensor, norm
     """kv, score [B,N,2d] fp32 (N % ratio == 0) -> [B,N//ratio,d] fp32.  sim: 0 none, 1 fp8 of the
     non-rope channels, 2 Hadamard + fp4 of all channels (``_lib.SIM_*``)."""
     _on_gpu(kv, score, ape, norm_w, cos_t, sin_t)
-    kv, score = kv.float().contiguous(), score.float().contiguous()
+    # slices of one wider projection (unit column stride, the same even row and sequence strides, 8-byte
+    # aligned) pass as they are; anything else is packed
+    sliced = (kv.dtype == score.dtype == torch.float32 and kv.shape == score.shape and kv.stride() == score.stride()
+              and kv.stride(2) == 1 and kv.stride(1) >= kv.shape[2] and kv.stride(1) % 2 == 0 and kv.stride(0) % 2 == 0
+              and (kv.shape[0] == 1 or kv.stride(0) > 0) and (kv.data_ptr() | score.data_ptr()) % 8 == 0)
+    if not sliced:
+        kv, score = kv.float().contiguous(), score.float().contiguous()
     ape, norm_w = ape.float().contiguous(), norm_w.float().contiguous()
     cos_t, sin_t = cos_t.float().contiguous(), sin_t.float().contiguous()
     B, N, two_d = kv.shape
@@ -310,8 +316,9 @@ def gated_pool_op(kv: torch.Tensor, score: torch.Tensor, ape: torch.Tensor, norm
     if cos_t.shape[0] < N:
         raise ValueError("rotation tables must cover every token position")
     out = torch.empty(B, N // ratio, d, dtype=torch.float32, device=kv.device)
-    _lib.call("smla_gated_pool", _p(kv), _p(score), _p(ape), _p(norm_w), _p(cos_t), _p(sin_t), B, N, d,
-              ratio, rope_head_dim, float(eps), int(sim), _p(out), _stream(kv))
+    # the batch stride of a single sequence is not used (0: the dense one)
+    _lib.call("smla_gated_pool_ld", _p(kv), _p(score), kv.stride(1), kv.stride(0) if B > 1 else 0, _p(ape), _p(norm_w),
+              _p(cos_t), _p(sin_t), B, N, d, ratio, rope_head_dim, float(eps), int(sim), _p(out), _stream(kv))
     return out
 
 
@@ -434,6 +441,31 @@ def linear_op(x: torch.Tensor, w: torch.Tensor, groups: int, out_dtype: torch.dt
 @linear_op.register_fake
 def _(x, w, groups, out_dtype):
     return x.new_empty(x.shape[0], w.shape[0], dtype=out_dtype)
+
+
+@torch.library.custom_op("smla::linear_pair", mutates_args=(), device_types="cuda")
+def linear_pair_op(x: torch.Tensor, w0: torch.Tensor, w1: torch.Tensor) -> torch.Tensor:
+    """x [T, K], w0 and w1 [N, K] (all bf16 or all fp32; K a multiple of 64 from 128) -> fp32 [T, 2N] =
+    [x @ w0^T, x @ w1^T], one launch of the tiled GEMM."""
+    _on_gpu(x, w0, w1)
+    if w0.shape != w1.shape or x.dim() != 2 or w0.dim() != 2 or x.shape[1] != w0.shape[1]:
+        raise ValueError("linear_pair: x [T, K] and w0, w1 [N, K] do not agree")
+    if not x.dtype == w0.dtype == w1.dtype:
+        raise TypeError("linear_pair: x, w0 and w1 share a dtype")
+    x, w0, w1 = x.contiguous(), w0.contiguous(), w1.contiguous()
+    T, K = x.shape
+    N = w0.shape[0]
+    y = torch.empty(T, 2 * N, dtype=torch.float32, device=x.device)
+    wsb = _lib.lib().smla_linear_pair_workspace(T, N, K, dtype_code(x))
+    ws = torch.empty(wsb, dtype=torch.uint8, device=x.device) if wsb else None
+    _lib.call("smla_linear_pair_ws", _p(x), dtype_code(x), _p(w0), _p(w1), dtype_code(w0), T, N, K, _p(y), _lib.F32,
+              _p(ws), wsb, _stream(x))
+    return y
+
+
+@linear_pair_op.register_fake
+def _(x, w0, w1):
+    return x.new_empty(x.shape[0], 2 * w0.shape[0], dtype=torch.float32)
 
 
 @torch.library.custom_op("smla::rope_", mutates_args=("x",), device_types="cuda")

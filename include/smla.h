@@ -24,6 +24,7 @@
  *   smla_index_decode         oracle/decode_engine.py:110-114  indexer scores + widx + cidx (fused)
  *   smla_block_mean_pool      (none: block mean of the 32K decode workload)
  *   smla_gated_pool           ref_torch/compressor.py:41-49    pooling + RMSNorm + RoPE of compressor_prefill
+ *   smla_gated_pool_ld        ref_torch/compressor.py:41-49    (the same over slices of wider rows)
  *   smla_ring_step            oracle/decode_engine.py:96-105   decode compressor ring step and cache append
  *   smla_quant_fp8_pow2       v4mlx/compressor.py:11-20        act_quant_sim (stored form: codes + pow2 scales)
  *   smla_row_epilogue         oracle/decode_engine.py:78-83    q/kv row norms, RoPE, fp8 sim, window-cache write
@@ -36,6 +37,7 @@
  *                             v4mlx/norm_rope.py:46-62         (MLX twin, cos/sin tables)
  *   smla_linear               v4mlx/mla.py:16-18               linear(x, W) (and the grouped form of mla.py:49-53)
  *   smla_linear_ws            v4mlx/mla.py:16-18               (the same, with a workspace)
+ *   smla_linear_pair_ws       ref_torch/compressor.py:28-29    kv and score projections in one launch
  *   smla_o_proj, _ws          oracle/decode_engine.py:118-119  inverse RoPE of o's rope dims + o_grouped
  *                             v4mlx/mla.py:42-56               o_grouped(o, wo_a, wo_b)
  */
@@ -319,6 +321,12 @@ int smla_gated_pool(const float* kv, const float* score, const float* ape, const
                     const float* cos_t, const float* sin_t, int64_t B, int64_t N, int64_t d,
                     int64_t ratio, int64_t rd, float eps, int sim, float* out, void* stream);
 
+/* smla_gated_pool of kv and score that are slices of wider rows: row n of sequence b starts ld_batch
+ * b + ld n elements in (0: dense, ld = 2d and ld_batch = N ld; even, SMLA_E_UNSUPPORTED otherwise). */
+int smla_gated_pool_ld(const float* kv, const float* score, int64_t ld, int64_t ld_batch, const float* ape,
+                       const float* norm_w, const float* cos_t, const float* sin_t, int64_t B, int64_t N,
+                       int64_t d, int64_t ratio, int64_t rd, float eps, int sim, float* out, void* stream);
+
 /* smla_ring_step: one decode token of the compressor ring (oracle/decode_engine.py:96-105) for
  * B sequences at positions pos[b]:
  *   ring_kv, ring_sc [B, 2*ratio, 2d] fp32 (updated);  kv_p, score_p: B rows of 2d fp32
@@ -448,6 +456,15 @@ size_t smla_linear_workspace(int64_t T, int64_t G, int64_t N, int64_t K, int x_d
 int smla_linear_ws(const void* x, int x_dtype, const void* w, int w_dtype, int64_t T, int64_t G,
                    int64_t N, int64_t K, void* y, int y_dtype, void* workspace, size_t workspace_bytes,
                    void* stream);
+
+/* Two weights on the same x: y [T, 2N] = [x w0^T, x w1^T], w0 and w1 [N, K] (the compressor's kv and
+ * score projections, ref_torch/compressor.py:28-29), in the tiled GEMM's one launch.  K a multiple of
+ * 64 from 128 (BF16) or of 32 from 64 (F32), else SMLA_E_UNSUPPORTED; other limits as smla_linear's.
+ * workspace: smla_linear_pair_workspace bytes or less, as in smla_linear_ws. */
+size_t smla_linear_pair_workspace(int64_t T, int64_t N, int64_t K, int x_dtype);
+int smla_linear_pair_ws(const void* x, int x_dtype, const void* w0, const void* w1, int w_dtype, int64_t T,
+                        int64_t N, int64_t K, void* y, int y_dtype, void* workspace, size_t workspace_bytes,
+                        void* stream);
 
 /* smla_o_proj: the attention output path of oracle/decode_engine.py:118-119 for T tokens:
  *   o [T, heads, head_dim] BF16; when pos != NULL the last rd dims of every head are rotated back

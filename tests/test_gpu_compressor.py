@@ -179,3 +179,44 @@ def test_quant_fp8_bit_exact(dev):
     rc_b, rs_b = ofp8.quantize_e4m3_pow2(x.to(torch.bfloat16).float().numpy(), 64)
     np.testing.assert_array_equal(codes_b.cpu().numpy(), rc_b)
     np.testing.assert_array_equal(scales_b.cpu().numpy(), rs_b)
+
+
+@pytest.mark.parametrize("B,N,d", [(1, 12, 512), (3, 20, 128)])
+def test_gated_pool_of_slices(dev, B, N, d):
+    """kv and score as slices of one wider projection (read where they are) give the packed call's rows
+    bit for bit; so do forms that are packed first (odd strides, repeated sequences)."""
+    from smla import norm_rope as snr
+    from smla import ops
+    announce(f"gated pool slices B={B} N={N} d={d}")
+    g = torch.Generator(device=dev).manual_seed(B + N)
+    ape, nw = torch.randn(4, 2 * d, generator=g, device=dev), torch.rand(d, generator=g, device=dev)
+    cos_t, sin_t = snr.rope_tables(64, 64, device=dev)
+    pool = lambda kv, sc: ops.gated_pool_op(kv, sc, ape, nw, cos_t, sin_t, 4, 64, 1e-6, 0)  # noqa: E731
+    for width, lo in ((4 * d, 0), (4 * d + 6, 2), (4 * d + 3, 0), (4 * d, 1)):
+        y = torch.randn(B, N + 3, width + 2, generator=g, device=dev)
+        kv, sc = y[:, 1:N + 1, lo:lo + 2 * d], y[:, 1:N + 1, lo + 2 * d:lo + 4 * d]
+        assert torch.equal(pool(kv, sc), pool(kv.contiguous(), sc.contiguous()))
+    one = torch.randn(1, N, 4 * d, generator=g, device=dev).expand(3, N, 4 * d)
+    got = pool(one[..., :2 * d], one[..., 2 * d:])
+    assert torch.equal(got, pool(one[..., :2 * d].contiguous(), one[..., 2 * d:].contiguous()))
+
+
+@pytest.mark.parametrize("s,dim,n,xdt,wdt,gdt", [
+    (300, 4096, 1024, torch.bfloat16, torch.bfloat16, torch.bfloat16),     # two weights, one launch
+    (37, 512, 256, torch.float32, torch.float32, torch.float32),
+    (37, 512, 250, torch.float32, torch.float32, torch.float32),
+    (37, 512, 256, torch.bfloat16, torch.bfloat16, torch.float32),         # mixed types: stacked, fp32
+    (5, 512, 256, torch.bfloat16, torch.bfloat16, torch.bfloat16),         # few rows: stacked
+    (40, 72, 256, torch.bfloat16, torch.bfloat16, torch.bfloat16),         # a K tail: stacked
+])
+def test_project_pair(dev, s, dim, n, xdt, wdt, gdt):
+    from smla import compressor as scomp
+    announce(f"project_pair s={s} dim={dim} n={n} {xdt} {wdt} {gdt}")
+    g = torch.Generator(device=dev).manual_seed(s + dim)
+    x = torch.randn(2, s, dim, generator=g, device=dev).to(xdt)
+    wkv = (torch.randn(n, dim, generator=g, device=dev) * 0.05).to(wdt)
+    wgate = (torch.randn(n, dim, generator=g, device=dev) * 0.05).to(gdt)
+    for got, w in zip(scomp.project_pair(x, wkv, wgate), (wkv, wgate)):
+        assert got.dtype == torch.float32 and got.shape == (2, s, n)
+        ref, mag = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+        assert bool(((got.double() - ref).abs() <= (dim + 8) * 2.0 ** -23 * mag).all())   # a dim-term fp32 sum
