@@ -227,14 +227,14 @@ __global__ __launch_bounds__(256) void indexer_kernel(const void* __restrict__ q
 // (h = lane again) and the key n = lane mod 16; register j of lane l holds head 16 (j / 4) + 4 (l / 16)
 // + j mod 4.  The head chain walks the 16-lane rows: after the four heads of row g, every row takes
 // row g's sum (two lane swaps).
-template <int KDT, int QDT, int KT = 32>
+template <int DI, int KDT, int QDT, int KT = 32>
 __global__ __launch_bounds__(256) void indexer_mfma_kernel(const void* __restrict__ q, const void* __restrict__ keys,
                                                        const uint8_t* __restrict__ kbs,
                                                        const float* __restrict__ kscale,
                                                        const float* __restrict__ weights,
                                                        const int32_t* __restrict__ nvis, int64_t S, int64_t N,
                                                        float* __restrict__ scores) {
-  constexpr int DI = 64;
+  static_assert(DI == 64 || DI == 128, "rows of 64 or 128");
   static_assert(KT == 32 || KT == 16, "key tiles of 32 or 16");
   constexpr int KEYS = 4 * KT;  // keys per workgroup: 4 waves x one tile of KT keys
   {
@@ -249,23 +249,27 @@ __global__ __launch_bounds__(256) void indexer_mfma_kernel(const void* __restric
   const int64_t kb = chunk * KEYS + wave * KT;  // first key of this wave's tile
 
   // the row of key kb + lane mod KT in its storage type
-  constexpr int KW = KDT == kFp4 ? 2 : KDT == SMLA_FP8_E4M3 ? 4 : (KDT == SMLA_BF16 ? 8 : 16);
+  constexpr int KW = DI / 64 * (KDT == kFp4 ? 2 : KDT == SMLA_FP8_E4M3 ? 4 : (KDT == SMLA_BF16 ? 8 : 16));
   u32x4_t kr[KW];
-  uint32_t ksb = 0;  // fp4: the row's two scale bytes
+  uint32_t ksb = 0;  // fp4: the row's DI / 32 scale bytes (2-byte aligned)
   {
     const int64_t n = kb + (lane & (KT - 1));
     const int64_t row = b * N + (n < N ? n : N - 1);
-    const u32x4_t* pk = (const u32x4_t*)((const uint8_t*)keys + row * DI * KW / 4);
+    const u32x4_t* pk = (const u32x4_t*)((const uint8_t*)keys + row * KW * 16);
 #pragma unroll
     for (int v = 0; v < KW; v++) kr[v] = pk[v];
-    if constexpr (KDT == kFp4) ksb = ((const uint16_t*)kbs)[row];
+    if constexpr (KDT == kFp4) {
+      const uint16_t* pb = (const uint16_t*)kbs + row * (DI / 64);
+      ksb = pb[0];
+      if constexpr (DI == 128) ksb |= (uint32_t)pb[1] << 16;
+    }
   }
   // The row's q block (64 heads), its head weights and the key's scale come in once per workgroup
   // through LDS: each wave loading the whole q block itself moved 8 KB per wave through L2 (16 MB
   // per decode step), and the compiler placed each of those loads next to its first MFMA, a round
   // trip per 16 bytes inside the chain; the weights and the scale were loaded after the chain.  q
   // rows sit at a stride of QW + 1 16-byte words, so the 64 lanes' row reads spread over the banks.
-  constexpr int QW = QDT == SMLA_BF16 ? 8 : 16;  // 16-byte words per head row
+  constexpr int QW = DI / 64 * (QDT == SMLA_BF16 ? 8 : 16);  // 16-byte words per head row
   constexpr int QV = 64 * QW / 256;              // words of the q block per thread
   __shared__ u32x4_t q_s[64 * (QW + 1)];
   __shared__ float w_s[64];
@@ -296,24 +300,27 @@ __global__ __launch_bounds__(256) void indexer_mfma_kernel(const void* __restric
   }
   const int64_t nv = nvis ? (int64_t)nvl : N;
   __syncthreads();
+  if (kb >= nv) {  // no key of the wave's tile is visible (wave-uniform; no barrier follows)
+    const int64_t n = kb + lane;
+    if (lane < KT && n < N) scores[bs * N + n] = -SMLA_INF;
+    return;
+  }
   u32x4_t qw[QW];  // head `lane`'s q row, read whole before the chain starts
 #pragma unroll
   for (int v = 0; v < QW; v++) qw[v] = q_s[lane * (QW + 1) + v];
 #pragma unroll
   for (int v = 0; v < QW; v++) asm volatile("" : "+v"(qw[v]));
   auto wrow = [&](int h) -> float { return w_s[h]; };
-  float qf[DI];
-#pragma unroll
-  for (int v = 0; v < QW; v++)
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      if constexpr (QDT == SMLA_BF16) {
-        qf[8 * v + 2 * j] = __uint_as_float(qw[v][j] << 16);
-        qf[8 * v + 2 * j + 1] = __uint_as_float(qw[v][j] & 0xffff0000u);
-      } else {
-        qf[4 * v + j] = __uint_as_float(qw[v][j]);
-      }
+  // q[lane][d] for a constant d, converted where it is used (beside a 64-cycle MFMA): an array of 128
+  // floats ahead of the chain would cost a second wave its registers
+  auto qval = [&](int d) __attribute__((always_inline)) -> float {
+    if constexpr (QDT == SMLA_BF16) {
+      const uint32_t w = qw[d / 8][d % 8 / 2];
+      return __uint_as_float(d & 1 ? w & 0xffff0000u : w << 16);
+    } else {
+      return __uint_as_float(qw[d / 4][d % 4]);
     }
+  };
   // 16 values of the key row starting at d0 = 16 db, as fp32 (fold: see fp4_block16)
   auto block16 = [&](int db, float (&o)[16], auto fold) {
     const u32x4_t(&row)[KW] = kr;
@@ -353,21 +360,23 @@ __global__ __launch_bounds__(256) void indexer_mfma_kernel(const void* __restric
   for (int r = 0; r < KT; r++) acc[r] = 0.f;
   auto run = [&](auto fold) {
 #pragma unroll
-    for (int db = 0; db < 4; db++) {
+    for (int db = 0; db < DI / 16; db++) {
       float x[16];
       block16(db, x, fold);
 #pragma unroll
       for (int dd = 0; dd < 16; dd++) {
         if constexpr (KT == 32)
-          acc = __builtin_amdgcn_mfma_f32_32x32x1f32(qf[16 * db + dd], x[dd], acc, 0, 0, 0);
+          acc = __builtin_amdgcn_mfma_f32_32x32x1f32(qval(16 * db + dd), x[dd], acc, 0, 0, 0);
         else
-          acc = __builtin_amdgcn_mfma_f32_16x16x1f32(qf[16 * db + dd], x[dd], acc, 0, 0, 0);
+          acc = __builtin_amdgcn_mfma_f32_16x16x1f32(qval(16 * db + dd), x[dd], acc, 0, 0, 0);
       }
     }
   };
   if constexpr (KDT == kFp4) {
     // the folded conversion when every scale byte of the wave's keys allows it (wave-uniform)
-    const bool fold = fp4_scale_in_range(ksb & 0xffu) && fp4_scale_in_range(ksb >> 8);
+    bool fold = true;
+#pragma unroll
+    for (int v = 0; v < DI / 32; v++) fold = fold && fp4_scale_in_range((ksb >> (8 * v)) & 0xffu);
     if (__all(fold)) run(std::true_type{});
     else run(std::false_type{});
   } else {
@@ -454,13 +463,13 @@ __global__ __launch_bounds__(256) void indexer_wide_kernel(const void* __restric
 template <int DI, int KDT>
 int launch_k(const void* q, int q_dtype, const void* keys, const uint8_t* kbs, const float* kscale, const float* w,
              const int32_t* nvis, int64_t B, int64_t S, int64_t Hi, int64_t N, float* scores, hipStream_t st) {
-  if (Hi == 64 && DI == 64) {
+  if constexpr (DI == 64 || DI == 128) if (Hi == 64) {
     // 128 keys per workgroup (a 64-head x 32-key tile per wave), or 64 (16-key tiles) when 128-key
     // workgroups would leave CUs idle
     const bool k16 = (N + 127) / 128 * B * S < smla_num_cus();
     const dim3 grid((unsigned)(k16 ? (N + 63) / 64 : (N + 127) / 128), (unsigned)(B * S));
 #define SMLA_IDX_MFMA(QT, KTT)                                                                                  \
-  hipLaunchKernelGGL((indexer_mfma_kernel<KDT, QT, KTT>), grid, dim3(256), 0, st, q, keys, kbs, kscale, w, nvis, S, \
+  hipLaunchKernelGGL((indexer_mfma_kernel<DI, KDT, QT, KTT>), grid, dim3(256), 0, st, q, keys, kbs, kscale, w, nvis, S, \
                      N, scores)
     if (q_dtype == SMLA_BF16) {
       if (k16) SMLA_IDX_MFMA(SMLA_BF16, 16); else SMLA_IDX_MFMA(SMLA_BF16, 32);
@@ -468,7 +477,10 @@ int launch_k(const void* q, int q_dtype, const void* keys, const uint8_t* kbs, c
       if (k16) SMLA_IDX_MFMA(SMLA_F32, 16); else SMLA_IDX_MFMA(SMLA_F32, 32);
     }
 #undef SMLA_IDX_MFMA
-  } else if (Hi <= 64) {
+    SMLA_HIP_CHECK_LAUNCH();
+    return SMLA_OK;
+  }
+  if (Hi <= 64) {
     dim3 grid((unsigned)((N + kKeys - 1) / kKeys), (unsigned)(B * S));
     const int hpw = heads_per_wave(Hi);
     const int threads = (int)(((Hi + hpw - 1) / hpw) * 64);

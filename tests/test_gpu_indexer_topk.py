@@ -109,6 +109,21 @@ def test_indexer_fp4_bit_exact(dev, qdt, use_scale, Hi, Di, N, edges):
         _same(out[b], ref)
 
 
+@pytest.mark.parametrize("qdt,kdt,use_scale,N", [
+    ("bf16", "fp8", True, 1000), ("f32", "f32", False, 130), ("f32", "bf16", True, 65),   # 16-key tiles
+    ("bf16", "fp8", False, 8200), ("f32", "f32", True, 8193), ("bf16", "bf16", False, 8192),  # 32-key tiles
+])
+def test_indexer_64x128_bit_exact(dev, qdt, kdt, use_scale, N):
+    """64 heads of 128 dims: the matrix-core chains."""
+    test_indexer_bit_exact(dev, qdt, kdt, use_scale, 64, 128, N)
+
+
+@pytest.mark.parametrize("qdt,use_scale,N", [("bf16", True, 300), ("f32", False, 1000), ("bf16", False, 8200),
+                                             ("f32", True, 8192)])
+def test_indexer_64x128_fp4_bit_exact(dev, qdt, use_scale, N):
+    test_indexer_fp4_bit_exact(dev, qdt, use_scale, 64, 128, N, True)
+
+
 def test_indexer_key_path_end_to_end(dev):
     """fp32 compressed keys -> Hadamard + fp4 on the GPU (smla_rotate_fp4, stored form) -> fp4
     scores -> top-2048, against the oracle's rotate_fp4 -> score -> top-k on the same keys; the
