@@ -228,7 +228,7 @@ __global__ __launch_bounds__(256) void indexer_kernel(const void* __restrict__ q
 // + j mod 4.  The head chain walks the 16-lane rows: after the four heads of row g, every row takes
 // row g's sum (two lane swaps).
 template <int DI, int KDT, int QDT, int KT = 32>
-__global__ __launch_bounds__(256) void indexer_mfma_kernel(const void* __restrict__ q, const void* __restrict__ keys,
+__global__ __launch_bounds__(256, DI == 128 && QDT == SMLA_BF16 && KDT != SMLA_F32 ? 3 : 1) void indexer_mfma_kernel(const void* __restrict__ q, const void* __restrict__ keys,
                                                        const uint8_t* __restrict__ kbs,
                                                        const float* __restrict__ kscale,
                                                        const float* __restrict__ weights,
