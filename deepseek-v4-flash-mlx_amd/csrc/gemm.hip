@@ -445,6 +445,97 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const RingArgs p) {
   }
 }
 
+// The q up projection of a prompt with its per-head epilogue (oracle/decode_engine.py:78-80): a tile is
+// 128 tokens x one head of 512, so the head's RMS norm (weightless, v4mlx/mla.py:26-28) and the RoPE of
+// its last 64 dims run on the accumulators and bf16 leaves.  As two launches the fp32 projection went
+// out and came back (1.07 GB for 4096 tokens x 64 heads).  Two stages of (128 + 512) x 64 k fill the 160 KB
+// of LDS.  4096 tokens, K 1024: 287 us, against 283 of fp32 product and 277 of epilogue; about 190 of them
+// are the K loop (1.46 us a step, 80 KB of operands per CU), the rest the 268 MB of rows, which leave when
+// the tiles end together.
+struct HeadForm {
+  static constexpr int BM = 128, BN = 512, WM = 64, WN = 128, D = 2;
+};
+
+__global__ __launch_bounds__(512) void gemm_heads_kernel(const RingArgs p, int64_t n_pos, float eps) {
+  using namespace smla_gemm;
+  using F = HeadForm;
+  using L = Tile<F::BM, F::BN, F::WM, F::WN, F::D>;
+  extern __shared__ __align__(16) uint8_t lds_g[];
+  lds_u8_t* lds = (lds_u8_t*)lds_g;
+  const TileId id = tile_id(p);
+  const int t0 = id.tm * F::BM, n0 = id.tn * F::BN;
+  f32x16_t acc[L::MB][L::NB];
+  tile_loop<F::BM, F::BN, F::WM, F::WN, F::D>(lds, p.x + (int64_t)t0 * p.ldx, p.ldx, p.T - 1 - t0,
+                                              p.w + (int64_t)n0 * p.K * 2, (int64_t)p.K * 2, F::BN - 1, p.K / 64, 0, acc,
+                                              [](int, lds_u8_t*) {});
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = wave % 2, wn = wave / 2;
+  // sums of squares: a row's 512 values sit in the 32 lanes of a half wave of four waves; the waves' sums
+  // and then the rows' factors go through LDS past the region the stores use
+  smla_attn::lds_f32_t* ss = (smla_attn::lds_f32_t*)(lds + 8 * F::WM * F::WN * 2);  // [4][128], then [128]
+  static_assert(8 * F::WM * F::WN * 2 + 5 * 128 * 4 <= L::LDS, "the sums fit behind the staged rows");
+  // the tile's rotations (128 rows of 32 cos and 32 sin) come in beside the sums, two 16-byte pieces of
+  // each per thread, and are read from LDS (one wave gathering them itself: 443 against 369 us, profiled)
+  f32x4_t rot[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; i++) {
+    const int e = threadIdx.x + 512 * i;  // row e / 8, piece e mod 8
+    int64_t ps = p.pos[min(t0 + (e >> 3), p.T - 1)];
+    ps = ps < 0 ? 0 : ps >= n_pos ? n_pos - 1 : ps;
+    rot[0][i] = *(const f32x4_t*)(p.cos_t + ps * 32 + 4 * (e & 7));
+    rot[1][i] = *(const f32x4_t*)(p.sin_t + ps * 32 + 4 * (e & 7));
+  }
+  lds_barrier();  // every wave has read its last fragments
+#pragma unroll
+  for (int mb = 0; mb < L::MB; mb++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      float q = 0.f;
+#pragma unroll
+      for (int nb = 0; nb < L::NB; nb++) q = __builtin_fmaf(acc[mb][nb][r], acc[mb][nb][r], q);
+      q += dpp_f<0xB1>(q);
+      q += dpp_f<0x4E>(q);
+      q += dpp_f<0x141>(q);
+      q += dpp_f<0x140>(q);
+      const auto h = __builtin_amdgcn_permlane16_swap(__float_as_uint(q), __float_as_uint(q), false, false);
+      q = __uint_as_float(h[0]) + __uint_as_float(h[1]);
+      if ((lane & 31) == 0) ss[128 * wn + 64 * wm + 32 * mb + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)] = q;
+    }
+  smla_attn::lds_f32x4_t* cs = (smla_attn::lds_f32x4_t*)lds;  // cos then sin, [128][32]
+#pragma unroll
+  for (int i = 0; i < 2; i++) {
+    cs[threadIdx.x + 512 * i] = rot[0][i];
+    cs[1024 + threadIdx.x + 512 * i] = rot[1][i];
+  }
+  lds_barrier();
+  if (threadIdx.x < 128) {
+    const int i = threadIdx.x;
+    ss[512 + i] = rsqrtf(((ss[i] + ss[128 + i]) + (ss[256 + i] + ss[384 + i])) / 512.f + eps);
+  }
+  lds_barrier();
+#pragma unroll
+  for (int mb = 0; mb < L::MB; mb++)
+#pragma unroll
+    for (int q4 = 0; q4 < 4; q4++) {
+      const int row = 64 * wm + 32 * mb + 8 * q4 + 4 * (lane >> 5);
+      const f32x4_t inv = *(smla_attn::lds_f32x4_t*)(ss + 512 + row);
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+#pragma unroll
+        for (int nb = 0; nb < L::NB; nb++) acc[mb][nb][4 * q4 + j] *= inv[j];
+        if (wn == 3) {  // uniform: this wave holds dims 384 .. 511; pair i sits in lanes 2 i and 2 i + 1
+          const smla_attn::lds_f32_t* cr = (const smla_attn::lds_f32_t*)lds + 32 * (row + j);
+#pragma unroll
+          for (int nb = 2; nb < 4; nb++) {
+            const int i = 16 * (nb - 2) + ((lane & 31) >> 1);
+            const float v = acc[mb][nb][4 * q4 + j], u = dpp_f<0xB1>(v), c = cr[i], s = cr[4096 + i];
+            acc[mb][nb][4 * q4 + j] = v * c + u * (lane & 1 ? s : -s);
+          }
+        }
+      }
+    }
+  store_tile<F, SMLA_BF16>(lds, p, 0, 0, t0, n0, acc);
+}
+
 // y[i] = part[0][i] + part[1][i] + ... in split order; V elements per thread
 template <int YDT, int V>
 __global__ __launch_bounds__(256) void gemm_reduce_kernel(const float* __restrict__ part, int splits, int64_t n,
@@ -631,6 +722,24 @@ int launch_gemm_tiled(const void* x, int64_t ldx, bool f32_operands, const void*
     else SMLA_GEMM(true, SMLA_F32, false);
   }
 #undef SMLA_GEMM
+  SMLA_HIP_CHECK_LAUNCH();
+  return SMLA_OK;
+}
+
+// out [T, heads, 512] bf16 = per-head RMS norm (eps) and RoPE of the last 64 dims (at pos) of x [T, K] times
+// w [heads * 512, K]^T, bf16 operands.  K a multiple of 64 from 128.  Returns SMLA_OK or a hipError_t.
+int launch_gemm_heads(const void* x, const void* w, int64_t T, int64_t heads, int64_t K, const int32_t* pos,
+                      const float* cos_t, const float* sin_t, int64_t n_pos, float eps, void* out, hipStream_t st) {
+  using F = HeadForm;
+  using L = smla_gemm::Tile<F::BM, F::BN, F::WM, F::WN, F::D>;
+  if (K % 64 != 0 || K / 64 < F::D || K * 2 * F::BN >= (1ll << 31) || heads * 512 > 0x7fffffff) return SMLA_E_UNSUPPORTED;
+  const int64_t nt = (T + F::BM - 1) / F::BM, wgs = nt * heads;
+  if (wgs > 0x7fffffff) return SMLA_E_UNSUPPORTED;
+  RingArgs a{(const uint8_t*)x, (const uint8_t*)w, nullptr, K * 2, 0, (int)T, (int)(heads * 512), (int)K, 1, (int)nt,
+             (int)heads, 1, pos, cos_t, sin_t, 512, (uint8_t*)out, heads * 512, 0, 1, 0};
+  static std::atomic<uint64_t> lds_attr{0};
+  if (hipError_t e = smla_set_dynamic_lds((const void*)gemm_heads_kernel, L::LDS, lds_attr); e != hipSuccess) return (int)e;
+  hipLaunchKernelGGL(gemm_heads_kernel, dim3((unsigned)wgs), dim3(L::NW * 64), L::LDS, st, a, n_pos, eps);
   SMLA_HIP_CHECK_LAUNCH();
   return SMLA_OK;
 }

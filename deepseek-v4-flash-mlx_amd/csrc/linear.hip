@@ -434,6 +434,16 @@ extern "C" size_t smla_linear_workspace(int64_t T, int64_t G, int64_t N, int64_t
   return (size_t)gemm_tiled_workspace(T, G, N, K, x_dtype == SMLA_F32);
 }
 
+extern "C" int smla_q_up(const void* x, const void* w, int64_t T, int64_t heads, int64_t K, const int32_t* pos,
+                         const float* cos_t, const float* sin_t, int64_t n_pos, float eps, void* out, void* stream) {
+  int rc = check_linear(x, SMLA_BF16, w, SMLA_BF16, T, 1, heads > 0 ? heads * 512 : 0, K, out, SMLA_BF16);
+  if (rc) return rc;
+  rc = check_rope_args(pos, cos_t, sin_t, n_pos, heads, 512, 64);
+  if (rc) return rc;
+  if (!(eps >= 0.f)) return SMLA_E_RANGE;
+  return launch_gemm_heads(x, w, T, heads, K, pos, cos_t, sin_t, n_pos, eps, out, (hipStream_t)stream);
+}
+
 extern "C" int smla_rope(void* x, int x_dtype, int64_t T, int64_t heads, int64_t head_dim, int64_t rd,
                          const int32_t* pos, const float* cos_t, const float* sin_t, int64_t n_pos, int inverse,
                          void* stream) {

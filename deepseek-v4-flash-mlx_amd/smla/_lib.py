@@ -69,6 +69,7 @@ _SIGNATURES = {
     "smla_linear_ws": (_int, [_vp, _int, _vp, _int, _i64, _i64, _i64, _i64, _vp, _int, _vp, _sz, _vp]),
     "smla_linear_pair_workspace": (_sz, [_i64, _i64, _i64, _int]),
     "smla_linear_pair_ws": (_int, [_vp, _int, _vp, _vp, _int, _i64, _i64, _i64, _vp, _int, _vp, _sz, _vp]),
+    "smla_q_up": (_int, [_vp, _vp, _i64, _i64, _i64, _vp, _vp, _vp, _i64, _f32, _vp, _vp]),
     "smla_o_proj_workspace": (_sz, [_i64] * 6),
     "smla_o_proj_ws": (_int, [_vp, _int, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _vp, _vp, _int,
                               _i64, _vp, _vp, _int, _vp, _sz, _vp]),

@@ -598,6 +598,26 @@ def row_epilogue(x, norm_w, pos, cos_t, sin_t, rd, sim, out, rows_per_pos=1, cac
     return out
 
 
+def q_up(x, w, pos, cos_t, sin_t, out, eps=1e-6):
+    """``smla_q_up``: x [T, K] bf16 times w [heads*512, K]^T, per-head RMS norm and RoPE of the last 64
+    dims at pos [T] (int32; cos/sin [n_pos, 32] fp32), into out [T, heads, 512] bf16.  Stream-ordered;
+    returns out."""
+    _on_gpu(x, w, pos, cos_t, sin_t, out)
+    if x.dim() != 2 or w.dim() != 2 or w.shape[1] != x.shape[1] or w.shape[0] % 512:
+        raise ValueError("q_up: expected x [T, K] and w [heads*512, K]")
+    T, heads = x.shape[0], w.shape[0] // 512
+    if tuple(out.shape) != (T, heads, 512) or not x.dtype == w.dtype == out.dtype == torch.bfloat16:
+        raise ValueError(f"q_up: bf16 operands and out [{T}, {heads}, 512]")
+    if pos.dtype != torch.int32 or tuple(pos.shape) != (T,) or tuple(cos_t.shape) != tuple(sin_t.shape) or \
+            cos_t.dim() != 2 or cos_t.shape[1] != 32 or not cos_t.dtype == sin_t.dtype == torch.float32:
+        raise ValueError("q_up: pos [T] int32 and fp32 cos/sin tables [n_pos, 32]")
+    if not all(t.is_contiguous() for t in (x, w, pos, cos_t, sin_t, out)):
+        raise ValueError("q_up: contiguous tensors")
+    _lib.call("smla_q_up", _p(x), _p(w), T, heads, x.shape[1], _p(pos), _p(cos_t), _p(sin_t), cos_t.shape[0],
+              float(eps), _p(out), _stream(x))
+    return out
+
+
 def row_epilogue_ids(x, norm_w, pos, cos_t, sin_t, rd, sim, out, rows_per_pos, ids_pos, window, ratio, n_raw,
                      ncomp, T, ids, comp32=None, comp_out=None, cache_rows=0, eps=1e-6):
     """``smla_row_epilogue_ids``: ``row_epilogue(x, norm_w, pos, cos_t, sin_t, rd, sim, out,

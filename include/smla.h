@@ -38,6 +38,7 @@
  *   smla_linear               v4mlx/mla.py:16-18               linear(x, W) (and the grouped form of mla.py:49-53)
  *   smla_linear_ws            v4mlx/mla.py:16-18               (the same, with a workspace)
  *   smla_linear_pair_ws       ref_torch/compressor.py:28-29    kv and score projections in one launch
+ *   smla_q_up                 oracle/decode_engine.py:78-80    q_up, per-head norm and RoPE of a prompt
  *   smla_o_proj, _ws          oracle/decode_engine.py:118-119  inverse RoPE of o's rope dims + o_grouped
  *                             v4mlx/mla.py:42-56               o_grouped(o, wo_a, wo_b)
  */
@@ -465,6 +466,15 @@ size_t smla_linear_pair_workspace(int64_t T, int64_t N, int64_t K, int x_dtype);
 int smla_linear_pair_ws(const void* x, int x_dtype, const void* w0, const void* w1, int w_dtype, int64_t T,
                         int64_t N, int64_t K, void* y, int y_dtype, void* workspace, size_t workspace_bytes,
                         void* stream);
+
+/* smla_q_up: a prompt's q up projection with its per-head epilogue, oracle/decode_engine.py:78-80:
+ * out [T, heads, 512] BF16 = x [T, K] w^T (w [heads*512, K], both BF16), every head RMS-normed without
+ * weights (v4mlx/mla.py:26-28, eps), its last 64 dims rotated to position pos[t] in [0, n_pos) (cos/sin
+ * [n_pos, 32], ref_torch/norm_rope.py:53-62): smla_linear with an fp32 result followed by
+ * smla_row_epilogue, in one launch without the fp32 rows.  K a multiple of 64 from 128
+ * (SMLA_E_UNSUPPORTED otherwise), 16-byte aligned pointers. */
+int smla_q_up(const void* x, const void* w, int64_t T, int64_t heads, int64_t K, const int32_t* pos,
+              const float* cos_t, const float* sin_t, int64_t n_pos, float eps, void* out, void* stream);
 
 /* smla_o_proj: the attention output path of oracle/decode_engine.py:118-119 for T tokens:
  *   o [T, heads, head_dim] BF16; when pos != NULL the last rd dims of every head are rotated back

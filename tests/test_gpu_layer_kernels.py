@@ -176,3 +176,30 @@ def test_row_epilogue_ids_equals_separate_calls(dev):
     assert torch.equal(i0, i1)
     assert torch.equal(c0.view(torch.int16), c1.view(torch.int16))
     assert q0.float().abs().sum() > 0 and c0.float().abs().sum() > 0 and (i0 >= 0).any()
+
+
+@pytest.mark.parametrize("T,heads,K", [(1, 2, 128), (127, 3, 192), (129, 2, 1024), (300, 64, 1024)])
+def test_q_up(dev, T, heads, K):
+    """smla_q_up against float64: the product of the bf16 operands, the per-head RMS norm and the
+    rotation, within half a bf16 ulp of the result plus the fp32 error of a K-term sum and its norm."""
+    from smla import norm_rope as snr
+    from smla import ops
+    announce(f"q_up T={T} heads={heads} K={K}")
+    g = torch.Generator(device=dev).manual_seed(T + K)
+    x = torch.randn(T, K, generator=g, device=dev).to(torch.bfloat16)
+    w = (torch.randn(heads * 512, K, generator=g, device=dev) * 0.05).to(torch.bfloat16)
+    pos = torch.randint(0, 4096, (T,), generator=g, device=dev, dtype=torch.int32)
+    cos_t, sin_t = snr.rope_tables(64, 4096, device=dev)
+    out = torch.empty(T, heads, 512, dtype=torch.bfloat16, device=dev)
+    ops.q_up(x, w, pos, cos_t, sin_t, out)
+    ref = (x.double() @ w.double().t()).view(T, heads, 512)
+    mag = (x.double().abs() @ w.double().abs().t()).view(T, heads, 512)
+    inv = torch.rsqrt(ref.square().mean(-1, keepdim=True) + 1e-6)
+    ref, mag = ref * inv, mag * inv
+    c, s = cos_t[pos.long()].double()[:, None], sin_t[pos.long()].double()[:, None]
+    a, b = ref[..., 448::2].clone(), ref[..., 449::2].clone()
+    ref[..., 448::2], ref[..., 449::2] = a * c - b * s, a * s + b * c
+    ma, mb = mag[..., 448::2].clone(), mag[..., 449::2].clone()
+    mag[..., 448::2] = mag[..., 449::2] = ma + mb       # |cos|, |sin| <= 1
+    tol = ref.abs() * 2.0 ** -8 + (K + 8) * 2.0 ** -23 * mag
+    assert bool(((out.double() - ref).abs() <= tol).all())
