@@ -131,4 +131,6 @@ def check(fn_name, status):
 
 
 def call(fn_name, *args):
-    check(fn_name, getattr(lib(), fn_name)(*args))
+    status = getattr(_LIB or lib(), fn_name)(*args)
+    if status != 0:
+        check(fn_name, status)

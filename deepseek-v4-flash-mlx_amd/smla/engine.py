@@ -160,20 +160,25 @@ class DecodeLayer:
         """``q_path`` and ``index_list`` of one decode step, with the per-head q epilogue and the id
         build in one launch (``smla_row_epilogue_ids``): the same q and ids.  Runs after the ring
         step, whose emitted row the id build copies."""
-        rows = qa_f.shape[0]
-        qa = torch.empty(rows, qa_f.shape[1], dtype=torch.bfloat16, device=qa_f.device)
+        return self._q_ids_from(self._q_proj(qa_f), pos, scores, k)
+
+    def _q_proj(self, qa_f):
+        """``decode_engine.py:78``: the fp32 q projection [rows * 64, 512] from the q_down projection."""
+        qa = torch.empty(qa_f.shape[0], qa_f.shape[1], dtype=torch.bfloat16, device=qa_f.device)
         ops.row_epilogue(qa_f, self.q_a_norm, None, None, None, 0, _lib.SIM_NONE, qa)
-        q = torch.empty(rows, N_HEADS, HEAD_DIM, dtype=torch.bfloat16, device=qa_f.device)
+        return _proj(qa, self.w.wq_b).view(-1, HEAD_DIM)
+
+    def _q_ids_from(self, q_f, pos, scores, k):
+        q = torch.empty(q_f.shape[0] // N_HEADS, N_HEADS, HEAD_DIM, dtype=torch.bfloat16, device=q_f.device)
         comp = (self.comp32, self.comp) if self.ring_ratio else (None, None)
         take_all = scores is None or not self.ring_ratio
         T = WINDOW + (self.ncap if take_all else 0)
         # on the indexer-scores path this launch still builds the window ids (T = 128), because it
         # also makes the bf16 copy of a compressed row the ring emitted; _select then writes the
         # step's list (window + top-k) and those ids are not used
-        ids = torch.empty(self.B, T, dtype=torch.int32, device=qa_f.device)
-        ops.row_epilogue_ids(_proj(qa, self.w.wq_b).view(rows * N_HEADS, HEAD_DIM), None, pos, self.cos_t,
-                             self.sin_t, ROPE_HD, _lib.SIM_NONE, q, N_HEADS, pos, WINDOW, self.ring_ratio,
-                             WINDOW, self.ncap, T, ids, comp32=comp[0], comp_out=comp[1])
+        ids = torch.empty(self.B, T, dtype=torch.int32, device=q_f.device)
+        ops.row_epilogue_ids(q_f, None, pos, self.cos_t, self.sin_t, ROPE_HD, _lib.SIM_NONE, q, N_HEADS, pos, WINDOW,
+                             self.ring_ratio, WINDOW, self.ncap, T, ids, comp32=comp[0], comp_out=comp[1])
         if take_all:
             return q, ids
         return q, self._select(pos, scores, k)
@@ -246,11 +251,20 @@ class DecodeLayer:
         if pos.shape != (self.B,):
             raise ValueError(f"pos must be [{self.B}]")
         pos = pos.to(torch.int32).contiguous()
-        if not torch.cuda.is_current_stream_capturing():
-            lo, hi = torch.aminmax(pos)
+        # the positions come to the host for the check while the projections, which change no state,
+        # already run: the device is not left idle between the check and the first launch
+        capturing = torch.cuda.is_current_stream_capturing()
+        if not capturing:
+            host_pos = pos.to("cpu", non_blocking=True)
+            arrived = torch.cuda.Event()
+            arrived.record(torch.cuda.current_stream(pos.device))
+        y = _proj(xn, self.w_in)                     # [B, sum of the projection widths] fp32
+        q_f = self._q_proj(y[:, :self.cuts[1]])
+        if not capturing:
+            arrived.synchronize()
+            lo, hi = torch.aminmax(host_pos)
             if int(lo) < 0 or int(hi) >= self.max_pos:
                 raise ValueError(f"positions must lie in [0, {self.max_pos}); got {int(lo)}..{int(hi)}")
-        y = _proj(xn, self.w_in)                     # [B, sum of the projection widths] fp32
         c = self.cuts
         if self.ring_ratio:
             # the kv row's epilogue and the ring step in one launch (kv_append + ring_step)
@@ -259,7 +273,7 @@ class DecodeLayer:
                              cache_rows=WINDOW)
         else:
             self.kv_append(y[:, c[1]:c[2]], pos)
-        q, ids = self.q_and_ids(y[:, c[0]:c[1]], pos, scores, k)
+        q, ids = self._q_ids_from(q_f, pos, scores, k)
         o = _sa.sparse_attn_two_source(q[:, None], self.raw, self.comp, self.w.sinks.float(), ids[:, None],
                                        HEAD_DIM ** -0.5, dv=HEAD_DIM)
         return mla.o_project(o[:, 0].contiguous(), pos, self.cos_t, self.sin_t, self.w.wo_a, self.w.wo_b)

@@ -21,6 +21,8 @@ def linear(x, W):
     ops._on_gpu(x, W)
     if x.dtype != W.dtype or x.dtype not in (torch.bfloat16, torch.float32):
         raise ValueError(f"linear: x ({x.dtype}) and W ({W.dtype}) must both be bf16 or both fp32")
+    if x.dim() == 2:
+        return ops.linear_op(x, W, 1, x.dtype)
     lead = x.shape[:-1]
     return ops.linear_op(x.reshape(-1, x.shape[-1]), W, 1, x.dtype).reshape(*lead, W.shape[0])
 

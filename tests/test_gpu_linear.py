@@ -302,3 +302,39 @@ def test_apply_rotary_emb_mirror(dev, shape, dt, inverse):
     got = snr.apply_rotary_emb(x.to(dev), cis.to(dev), inverse=inverse).cpu()
     ref = onr.apply_rotary_emb(x, cis, inverse=inverse)
     assert got.dtype == x.dtype and torch.equal(got, ref)
+
+
+def test_ops_eager_route(dev):
+    """Plain CUDA tensors skip the registered op and give its result; whatever needs the op (a
+    differentiated input, forward-mode level, functorch transform, fake tensors, a tracer, a CPU
+    tensor) still reaches it."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    from smla import ops
+    announce("ops eager route")
+    x = torch.randn(4, 512, device=dev).to(torch.bfloat16)
+    w = torch.randn(64, 512, device=dev).to(torch.bfloat16)
+    args = (x, w, 1, torch.float32)
+    seen = []
+
+    def probe(a):
+        seen.append(ops._eager((a, w, 1, torch.float32)))
+        return a
+
+    assert ops._eager(args)
+    assert torch.equal(ops.linear_op(*args), ops.linear_op.op(*args))
+    leaf = x.clone().requires_grad_()
+    probe(leaf)
+    assert ops.linear_op(leaf, w, 1, torch.float32).requires_grad
+    torch.func.vmap(probe)(x[None])
+    with torch.autograd.forward_ad.dual_level():
+        probe(x)
+    with FakeTensorMode() as mode:
+        fake = mode.from_tensor(x)
+        probe(fake)
+        assert ops.linear_op(fake, mode.from_tensor(w), 1, torch.float32).shape == (4, 64)
+    torch.jit.trace(probe, (x,), check_trace=False)
+    probe(x.cpu())
+    assert len(seen) >= 6 and not any(seen)
+    with torch.no_grad():
+        assert ops._eager((leaf, w, 1, torch.float32))
