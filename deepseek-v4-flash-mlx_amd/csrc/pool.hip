@@ -127,8 +127,8 @@ __device__ inline void epilogue_rotation(EpiOperands& e, int d, int rd, const fl
   }
 }
 
-__device__ inline void pool_epilogue(float v0, float v1, int d, int rd, float eps, int sim, const EpiOperands& e,
-                                     float* red, float* xch, float* dst) {
+__device__ inline f32x2_t epilogue_values(float v0, float v1, int d, int rd, float eps, int sim,
+                                          const EpiOperands& e, float* red, float* xch) {
   const int t = threadIdx.x;
   const int c0 = 2 * t;
   float ss = block_sum(v0 * v0 + v1 * v1, red);
@@ -195,8 +195,14 @@ __device__ inline void pool_epilogue(float v0, float v1, int d, int rd, float ep
     y0 = e2m1_to_f32(f32_to_e2m1(fminf(fmaxf(y0 * si, -6.f), 6.f))) * s;
     y1 = e2m1_to_f32(f32_to_e2m1(fminf(fmaxf(y1 * si, -6.f), 6.f))) * s;
   }
-  dst[c0] = y0;
-  dst[c0 + 1] = y1;
+  return f32x2_t{y0, y1};
+}
+
+__device__ inline void pool_epilogue(float v0, float v1, int d, int rd, float eps, int sim, const EpiOperands& e,
+                                     float* red, float* xch, float* dst) {
+  const f32x2_t y = epilogue_values(v0, v1, d, rd, eps, sim, e, red, xch);
+  dst[2 * threadIdx.x] = y[0];
+  dst[2 * threadIdx.x + 1] = y[1];
 }
 
 // slot-weighted pooling for one channel over `ns` (value, score) pairs held in registers
@@ -215,15 +221,13 @@ __device__ inline float softmax_pool(const float* v, const float* s, int ns) {
 
 constexpr int kMaxRatio = 8;
 
-__global__ __launch_bounds__(kPoolThreads) void gated_pool_kernel(
-    const float* __restrict__ kv, const float* __restrict__ score, const float* __restrict__ ape,
-    const float* __restrict__ norm_w, const float* __restrict__ cos_t, const float* __restrict__ sin_t, int64_t N,
-    int d, int ratio, int rd, float eps, int sim, int64_t ld, int64_t ldb, float* __restrict__ out) {
+// pooled row g of sequence b, run by one workgroup of d/2 threads: this thread's two channels
+__device__ __attribute__((always_inline)) inline f32x2_t gated_pool_body(
+    int64_t b, int64_t g, const float* __restrict__ kv, const float* __restrict__ score, const float* __restrict__ ape,
+    const float* __restrict__ norm_w, const float* __restrict__ cos_t, const float* __restrict__ sin_t, int d, int ratio,
+    int rd, float eps, int sim, int64_t ld, int64_t ldb) {
   __shared__ float red[kPoolThreads / 64];
   __shared__ float xch[2 * kPoolThreads];
-  const int64_t G = N / ratio;
-  const int64_t bg = blockIdx.x;
-  const int64_t b = bg / G, g = bg % G;
   const int t = threadIdx.x;
   const int64_t two_d = 2 * (int64_t)d;
   // channels c0 = 2t and c0 + 1 of every slot in one 8-byte load each (kv, score, ape)
@@ -245,11 +249,18 @@ __global__ __launch_bounds__(kPoolThreads) void gated_pool_kernel(
   if (g > 0)
     for (int j = 0; j < ratio; j++) slot((g - 1) * ratio + j, 0, j);
   for (int j = 0; j < ratio; j++) slot(g * ratio + j, d, j);
-  float pooled[2];
-  pooled[0] = softmax_pool<2 * kMaxRatio>(v0, s0, ns);
-  pooled[1] = softmax_pool<2 * kMaxRatio>(v1, s1, ns);
-  pool_epilogue(pooled[0], pooled[1], d, rd, eps, sim, eo, red, xch,
-                out + bg * (int64_t)d);
+  const float p0 = softmax_pool<2 * kMaxRatio>(v0, s0, ns), p1 = softmax_pool<2 * kMaxRatio>(v1, s1, ns);
+  return epilogue_values(p0, p1, d, rd, eps, sim, eo, red, xch);
+}
+
+__global__ __launch_bounds__(kPoolThreads) void gated_pool_kernel(
+    const float* __restrict__ kv, const float* __restrict__ score, const float* __restrict__ ape,
+    const float* __restrict__ norm_w, const float* __restrict__ cos_t, const float* __restrict__ sin_t, int64_t N,
+    int d, int ratio, int rd, float eps, int sim, int64_t ld, int64_t ldb, float* __restrict__ out) {
+  const int64_t G = N / ratio;
+  const int64_t bg = blockIdx.x;
+  const f32x2_t y = gated_pool_body(bg / G, bg % G, kv, score, ape, norm_w, cos_t, sin_t, d, ratio, rd, eps, sim, ld, ldb);
+  *(f32x2_t*)(out + bg * (int64_t)d + 2 * threadIdx.x) = y;
 }
 
 // the ring step of sequence b, run by one workgroup of d/2 threads
@@ -590,6 +601,128 @@ __global__ __launch_bounds__(256) void q_ids_kernel(
     const int64_t i = blk - rows;
     decode_ids_body(i % nx, i / nx, pos, window, ratio, n_raw, ncomp, T, ids, comp32, comp_out, comp_d);
   }
+}
+
+// Everything a prompt's projections feed besides the q up projection, in one launch (workgroups of 256
+// threads, 512-wide rows; oracle/decode_engine.py:78,81-95 for positions 0 .. S-1 of B sequences):
+//   pool  B * (S/4): a compressed row (gated pool, RMSNorm, RoPE, fp8 round trip) into the fp32 cache
+//         and its bf16 copy;
+//   kv    B * S: a window row (RMSNorm, RoPE, fp8 round trip) into the prompt's buffer and, for the last
+//         `ring_rows` positions, the window ring (oracle/v4_fast.py:93-94); and the row's position;
+//   q_a   B * S: the RMSNorm of the q down projection;
+//   ring  B: the compressor ring from the last whole group and the remainder (decode_engine.py:90-95).
+// They read nothing but the projections.  As separate calls they were some 18 launches (slices packed,
+// tables of positions, caches copied, ring slots filled), which is what a prompt of a few hundred
+// tokens spent its time on.
+struct PromptRows {
+  const float *qa, *kv, *kvp, *scp;  // the projections' slices; kvp null: no compressor
+  int64_t ld, B, S;
+  int dq;
+  const float *qa_norm, *kv_norm, *cos_t, *sin_t;
+  uint16_t *qa_out, *win, *raw;
+  int64_t ring_rows;
+  const float *ape, *c_norm, *c_cos, *c_sin;
+  float* comp32;
+  uint16_t* comp;
+  int64_t ncap;
+  float *ring_kv, *ring_sc;
+  int32_t* pos;
+  float eps;
+};
+
+__global__ __launch_bounds__(256) void prompt_rows_kernel(const PromptRows p) {
+  constexpr int d = 512, rd = 64, ratio = 4;
+  __shared__ float red[4];
+  __shared__ float xch[512];
+  const int t = threadIdx.x;
+  int64_t i = blockIdx.x;
+  const int64_t groups = p.kvp ? p.S / ratio : 0, rows = p.B * p.S;
+  if (i < p.B * groups) {
+    const int64_t b = i / groups, g = i % groups;
+    const f32x2_t y = gated_pool_body(b, g, p.kvp, p.scp, p.ape, p.c_norm, p.c_cos, p.c_sin, d, ratio, rd, p.eps,
+                                      SMLA_SIM_FP8, p.ld, p.S * p.ld);
+    const int64_t o = (b * p.ncap + g) * d + 2 * t;
+    *(f32x2_t*)(p.comp32 + o) = y;
+    *(uint32_t*)(p.comp + o) = pack_bf16x2(y[0], y[1]);
+    return;
+  }
+  i -= p.B * groups;
+  if (i < rows) {
+    const int64_t b = i / p.S, s = i % p.S;
+    const f32x2_t v = *(const f32x2_t*)(p.kv + i * p.ld + 2 * t);
+    EpiOperands eo = epilogue_weights(p.kv_norm);
+    epilogue_rotation(eo, d, rd, p.cos_t, p.sin_t, s);
+    const f32x2_t y = epilogue_values(v[0], v[1], d, rd, p.eps, SMLA_SIM_FP8, eo, red, xch);
+    const uint32_t w = pack_bf16x2(y[0], y[1]);
+    *(uint32_t*)(p.win + i * d + 2 * t) = w;
+    if (s >= p.S - p.ring_rows) *(uint32_t*)(p.raw + (b * p.ring_rows + s % p.ring_rows) * d + 2 * t) = w;
+    if (t == 0) p.pos[i] = (int32_t)s;
+    return;
+  }
+  i -= rows;
+  if (i < rows) {
+    // 4 channels per thread and round: dq <= 1024
+    const float* x = p.qa + i * p.ld;
+    const int c = 4 * t;
+    f32x2_t a = {0.f, 0.f}, q = {0.f, 0.f};
+    if (c < p.dq) {
+      a = *(const f32x2_t*)(x + c);
+      q = *(const f32x2_t*)(x + c + 2);
+    }
+    const float ss = block_sum(a[0] * a[0] + a[1] * a[1] + q[0] * q[0] + q[1] * q[1], red);
+    const float inv = rsqrtf(ss / (float)p.dq + p.eps);
+    if (c < p.dq) {
+      const f32x4_t w = *(const f32x4_t*)(p.qa_norm + c);
+      *(u32x2_t*)(p.qa_out + i * p.dq + c) = (u32x2_t){pack_bf16x2(w[0] * (a[0] * inv), w[1] * (a[1] * inv)),
+                                                      pack_bf16x2(w[2] * (q[0] * inv), w[3] * (q[1] * inv))};
+    }
+    return;
+  }
+  // the ring of sequence b: slots 0 .. 3 the last whole group, 4 .. the remainder, else kv 0 and score -inf
+  const int64_t b = i - rows, cut = p.S - p.S % ratio;
+  for (int slot = 0; slot < 2 * ratio; slot++) {
+    const int64_t s = slot < ratio ? cut - ratio + slot : cut + slot - ratio;
+    const bool live = slot < ratio ? cut >= ratio : s < p.S;
+    for (int c = 2 * t; c < 2 * d; c += 512) {
+      f32x2_t k = {0.f, 0.f}, sc = {-SMLA_INF, -SMLA_INF};
+      if (live) {
+        k = *(const f32x2_t*)(p.kvp + (b * p.S + s) * p.ld + c);
+        const f32x2_t v = *(const f32x2_t*)(p.scp + (b * p.S + s) * p.ld + c);
+        const f32x2_t ap = *(const f32x2_t*)(p.ape + (slot % ratio) * 2 * d + c);
+        sc = f32x2_t{v[0] + ap[0], v[1] + ap[1]};
+      }
+      const int64_t o = (b * 2 * ratio + slot) * 2 * d + c;
+      *(f32x2_t*)(p.ring_kv + o) = k;
+      *(f32x2_t*)(p.ring_sc + o) = sc;
+    }
+  }
+}
+
+extern "C" int smla_prompt_rows(const float* qa, const float* kv, const float* kvp, const float* scp, int64_t ld,
+                                int64_t B, int64_t S, int64_t dq, const float* qa_norm, const float* kv_norm,
+                                const float* cos_t, const float* sin_t, int64_t n_pos, void* qa_out, void* win,
+                                void* raw, int64_t ring_rows, const float* ape, const float* c_norm, const float* c_cos,
+                                const float* c_sin, int64_t c_n_pos, float* comp32, void* comp, int64_t ncap,
+                                float* ring_kv, float* ring_sc, int32_t* pos, float eps, void* stream) {
+  if (!qa || !kv || !qa_norm || !kv_norm || !cos_t || !sin_t || !qa_out || !win || !raw || !pos) return SMLA_E_NULL;
+  const bool c = kvp != nullptr;
+  if (c && (!scp || !ape || !c_norm || !c_cos || !c_sin || !comp32 || !comp || !ring_kv || !ring_sc)) return SMLA_E_NULL;
+  if (B <= 0 || S <= 0 || dq <= 0 || ring_rows <= 0 || ld <= 0 || S > n_pos || (c && (ncap < S / 4 || S > c_n_pos)))
+    return SMLA_E_SHAPE;
+  if (!(eps >= 0.f)) return SMLA_E_RANGE;
+  const uintptr_t even = (uintptr_t)qa | (uintptr_t)kv | (uintptr_t)kvp | (uintptr_t)scp | (uintptr_t)ape |
+                         (uintptr_t)comp32 | (uintptr_t)ring_kv | (uintptr_t)ring_sc | (uintptr_t)qa_out;
+  if (dq > 1024 || dq % 4 != 0 || ld % 2 != 0 || (even & 7) || ((uintptr_t)qa_norm & 15) ||
+      (((uintptr_t)win | (uintptr_t)raw | (uintptr_t)comp) & 3))
+    return SMLA_E_UNSUPPORTED;
+  const int64_t blocks = 2 * B * S + (c ? B * (S / 4) + B : 0);
+  if (B > (int64_t)INT32_MAX / S || blocks > (int64_t)INT32_MAX) return SMLA_E_UNSUPPORTED;
+  const PromptRows a{qa, kv, kvp, scp, ld, B, S, (int)dq, qa_norm, kv_norm, cos_t, sin_t, (uint16_t*)qa_out,
+                     (uint16_t*)win, (uint16_t*)raw, ring_rows, ape, c_norm, c_cos, c_sin, comp32, (uint16_t*)comp,
+                     ncap, ring_kv, ring_sc, pos, eps};
+  hipLaunchKernelGGL(prompt_rows_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, a);
+  SMLA_HIP_CHECK_LAUNCH();
+  return SMLA_OK;
 }
 
 static int check_ring_step(const float* ring_kv, const float* ring_sc, const float* kv_p, const float* score_p,

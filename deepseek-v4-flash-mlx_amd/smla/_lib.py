@@ -61,6 +61,8 @@ _SIGNATURES = {
                                  _int, _i64, _vp]),
     "smla_row_epilogue_ids": (_int, [_vp, _i64, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _i64, _i64, _f32, _int, _vp,
                                      _int, _i64, _vp, _i64, _i64, _i64, _i64, _i64, _vp, _i64, _vp, _vp, _i64, _vp]),
+    "smla_prompt_rows": (_int, [_vp] * 4 + [_i64] * 4 + [_vp] * 4 + [_i64] + [_vp] * 3 + [_i64] + [_vp] * 4
+                         + [_i64, _vp, _vp, _i64, _vp, _vp, _vp, _f32, _vp]),
     "smla_decode_ids": (_int, [_vp, _i64, _i64, _i64, _i64, _i64, _vp, _i64, _vp, _vp, _i64, _vp]),
     "smla_rotate_fp4": (_int, [_vp, _int, _i64, _i64, _int, _vp, _vp, _vp, _vp]),
     "smla_rope": (_int, [_vp, _int, _i64, _i64, _i64, _i64, _vp, _vp, _vp, _i64, _int, _vp]),

@@ -117,7 +117,12 @@ class DecodeLayer:
         rows = qa_f.shape[0]
         qa = torch.empty(rows, qa_f.shape[1], dtype=torch.bfloat16, device=qa_f.device)
         ops.row_epilogue(qa_f, self.q_a_norm, None, None, None, 0, _lib.SIM_NONE, qa)
-        q = torch.empty(rows, N_HEADS, HEAD_DIM, dtype=torch.bfloat16, device=qa_f.device)
+        return self._q_up(qa, pos)
+
+    def _q_up(self, qa, pos):
+        """``decode_engine.py:79-80``: q [rows, 64, 512] bf16 from the normed q down projection."""
+        rows = qa.shape[0]
+        q = torch.empty(rows, N_HEADS, HEAD_DIM, dtype=torch.bfloat16, device=qa.device)
         # from 192 tokens the projection's tiles of 128 tokens x one head fill the device and take the
         # epilogue with them (31 against 21 + 15 us at 192 tokens, 287 against 283 + 277 at 4096)
         wq_b = self.w.wq_b
@@ -208,33 +213,16 @@ class DecodeLayer:
         B, S, dim = xn.shape
         if not 0 < S <= self.max_pos:
             raise ValueError(f"the prompt length must lie in 1..{self.max_pos}")
-        dev = xn.device
-        pos = torch.arange(S, dtype=torch.int32, device=dev).repeat(B)      # position of each (b, s) row
         y = _proj(xn.reshape(B * S, dim), self.w_in)                        # [B*S, projection widths] fp32
-        c = self.cuts
-        q = self.q_path(y[:, c[0]:c[1]], pos)                               # [B*S, 64, 512]
-        win = torch.empty(B, S, HEAD_DIM, dtype=torch.bfloat16, device=dev)    # the prompt's window rows
-        for b in range(B):                                                  # window rows 0..S-1
-            ops.row_epilogue(y[b * S:(b + 1) * S, c[1]:c[2]], self.kv_a_norm, pos[:S], self.cos_t, self.sin_t,
-                             ROPE_HD, _lib.SIM_FP8, win[b])
-        T = WINDOW
-        if self.ring_ratio:
-            kvp = y[:, c[2]:c[3]].reshape(B, S, -1)
-            scp = y[:, c[3]:c[4]].reshape(B, S, -1)
-            cut = S - S % 4
-            if cut >= 4:
-                comp = ops.gated_pool_op(kvp[:, :cut], scp[:, :cut], self.ring.ape, self.ring.norm_w, self.ring.cos_t,
-                                         self.ring.sin_t, 4, ROPE_HD, 1e-6, _lib.SIM_FP8)
-                self.comp32[:, :cut // 4] = comp
-                self.comp[:, :cut // 4] = comp.to(torch.bfloat16)
-            self.ring.init_from_prefill(kvp, scp)
-            T += S // 4
+        # the norms, the prompt's window rows and their ring, the compressed rows, the ring: one launch
+        comp = dict(ring=self.ring, comp32=self.comp32, comp=self.comp) if self.ring_ratio else {}
+        qa, win, pos = ops.prompt_rows(y, self.cuts, B, S, self.q_a_norm, self.kv_a_norm, self.cos_t, self.sin_t,
+                                       self.raw, **comp)
+        q = self._q_up(qa, pos)                                             # [B*S, 64, 512]
         # every position's window and visible compressed rows, computed in the kernel (smla_prefill_attn)
         o = _sa.prefill_attn(q.view(B, S, N_HEADS, HEAD_DIM), win, self.comp if self.ring_ratio else None,
                              self.w.sinks.float(), HEAD_DIM ** -0.5, q_pos0=0, window=WINDOW, ratio=self.ring_ratio,
                              dv=HEAD_DIM)
-        lo = max(0, S - WINDOW)                     # the positions the ring keeps, each at its row p % 128
-        self.raw[:, torch.arange(lo, S, device=dev) % WINDOW] = win[:, lo:]
         out = mla.o_project(o.view(B * S, N_HEADS, HEAD_DIM), pos, self.cos_t, self.sin_t, self.w.wo_a, self.w.wo_b)
         return out.view(B, S, -1)
 

@@ -699,6 +699,41 @@ def q_up(x, w, pos, cos_t, sin_t, out, eps=1e-6):
     return out
 
 
+def prompt_rows(y, cuts, B, S, qa_norm, kv_norm, cos_t, sin_t, raw, ring=None, comp32=None, comp=None, eps=1e-6):
+    """``smla_prompt_rows`` on y [B*S, cuts[-1]] fp32, the projections [q_down; kv (; kv_c; gate_c)] side by
+    side (column bounds cuts), with raw [B, rows, 512] bf16 and, for a layer with a compressor, its
+    ``compressor.Ring`` and the caches comp32 / comp [B, ncap, 512].  Writes raw, the caches and the ring;
+    returns (qa [B*S, dq] bf16, win [B, S, 512] bf16, pos [B*S] int32).  Stream-ordered."""
+    _on_gpu(y, qa_norm, kv_norm, cos_t, sin_t, raw, comp32, comp)
+    dq = cuts[1]
+    wide = [dq, 512] + ([1024, 1024] if ring is not None else [])
+    if y.dim() != 2 or y.dtype != torch.float32 or not y.is_contiguous() or y.shape[0] != B * S or \
+            [b - a for a, b in zip(cuts, cuts[1:])] != wide or y.shape[1] != cuts[-1]:
+        raise ValueError(f"prompt_rows: y must be contiguous fp32 [{B * S}, {sum(wide)}]")
+    f32 = [(qa_norm, (dq,)), (kv_norm, (512,)), (cos_t, (cos_t.shape[0], 32)), (sin_t, tuple(cos_t.shape))]
+    if ring is not None:
+        n = ring.cos_t.shape[0]
+        f32 += [(ring.ape, (4, 1024)), (ring.norm_w, (512,)), (ring.cos_t, (n, 32)), (ring.sin_t, (n, 32)),
+                (ring.ring_kv, (B, 8, 1024)), (ring.ring_sc, (B, 8, 1024)), (comp32, (B, comp32.shape[1], 512))]
+    if any(t.dtype != torch.float32 or tuple(t.shape) != s or not t.is_contiguous() for t, s in f32):
+        raise ValueError("prompt_rows: norms, tables, ring and comp32 must be contiguous fp32 of their shapes")
+    bf16 = [(raw, (B, raw.shape[1], 512))] + ([(comp, tuple(comp32.shape))] if ring is not None else [])
+    if any(t.dtype != torch.bfloat16 or tuple(t.shape) != s or not t.is_contiguous() for t, s in bf16):
+        raise ValueError("prompt_rows: raw and comp must be contiguous bf16 of their shapes")
+    qa = torch.empty(B * S, dq, dtype=torch.bfloat16, device=y.device)
+    win = torch.empty(B, S, 512, dtype=torch.bfloat16, device=y.device)
+    pos = torch.empty(B * S, dtype=torch.int32, device=y.device)
+    at = [y.data_ptr() + 4 * c for c in cuts]
+    c = ring is not None
+    _lib.call("smla_prompt_rows", at[0], at[1], at[2] if c else None, at[3] if c else None, y.shape[1], B, S, dq,
+              _p(qa_norm), _p(kv_norm), _p(cos_t), _p(sin_t), cos_t.shape[0], _p(qa), _p(win), _p(raw), raw.shape[1],
+              _p(ring.ape) if c else None, _p(ring.norm_w) if c else None, _p(ring.cos_t) if c else None,
+              _p(ring.sin_t) if c else None, ring.cos_t.shape[0] if c else 0, _p(comp32), _p(comp),
+              comp32.shape[1] if c else 0, _p(ring.ring_kv) if c else None, _p(ring.ring_sc) if c else None, _p(pos),
+              float(eps), _stream(y))
+    return qa, win, pos
+
+
 def row_epilogue_ids(x, norm_w, pos, cos_t, sin_t, rd, sim, out, rows_per_pos, ids_pos, window, ratio, n_raw,
                      ncomp, T, ids, comp32=None, comp_out=None, cache_rows=0, eps=1e-6):
     """``smla_row_epilogue_ids``: ``row_epilogue(x, norm_w, pos, cos_t, sin_t, rd, sim, out,

@@ -30,6 +30,7 @@
  *   smla_row_epilogue         oracle/decode_engine.py:78-83    q/kv row norms, RoPE, fp8 sim, window-cache write
  *   smla_ring_step_kv         oracle/decode_engine.py:81-84,96-105  kv window append + ring step in one launch
  *   smla_row_epilogue_ids     oracle/decode_engine.py:78-80,110-114  per-head q epilogue + decode ids in one launch
+ *   smla_prompt_rows          oracle/decode_engine.py:78,81-95  a prompt's norms, window rows, pooled rows, ring
  *   smla_decode_ids           oracle/decode_engine.py:110-114  decode id list (window + visible compressed rows)
  *   smla_rotate_fp4           v4mlx/qat.py:8-31                hadamard_rotate, fp4_act_quant (and stored form)
  *                             v4mlx/compressor.py:57-59        the indexer compressor's key transform
@@ -388,6 +389,24 @@ int smla_ring_step_kv(float* ring_kv, float* ring_sc, const float* kv_p, const f
                       const float* kv_x, int64_t ld_kv, const float* kv_norm, const float* kv_cos,
                       const float* kv_sin, int64_t kv_n_pos, int64_t kv_rd, float kv_eps, int kv_sim,
                       void* kv_cache, int kv_cache_dtype, int64_t kv_cache_rows, void* stream);
+
+/* smla_prompt_rows: what the projections of a prompt at positions 0 .. S-1 of B sequences feed besides
+ * the q up projection, in one launch (oracle/decode_engine.py:78,81-95).  qa [B*S, dq], kv [B*S, 512] and
+ * kvp / scp [B*S, 1024] (NULL: a layer without compressor) are fp32 slices of rows ld elements apart.
+ *   qa_out [B*S, dq] BF16: RMSNorm(qa) with qa_norm [dq] (dq <= 1024, a multiple of 4);
+ *   win [B*S, 512] BF16: the kv rows, RMSNorm with kv_norm, RoPE of the last 64 channels (cos/sin [n_pos,
+ *     32]) and fp8 round trip; the last min(S, ring_rows) of a sequence also at row s mod ring_rows of
+ *     raw [B, ring_rows, 512] BF16; pos [B*S] int32 = s;
+ *   comp32 / comp [B, ncap, 512] fp32 / BF16: rows 0 .. S/4 - 1 as smla_gated_pool (d 512, ratio 4, sim
+ *     SMLA_SIM_FP8; ape [4, 1024], c_norm, c_cos / c_sin [c_n_pos, 32]) gives them;
+ *   ring_kv, ring_sc [B, 8, 1024] fp32: the ring after the prompt (decode_engine.py:90-95).
+ * S <= n_pos, c_n_pos; S/4 <= ncap.  Buffers must not overlap the projections. */
+int smla_prompt_rows(const float* qa, const float* kv, const float* kvp, const float* scp, int64_t ld, int64_t B,
+                     int64_t S, int64_t dq, const float* qa_norm, const float* kv_norm, const float* cos_t,
+                     const float* sin_t, int64_t n_pos, void* qa_out, void* win, void* raw, int64_t ring_rows,
+                     const float* ape, const float* c_norm, const float* c_cos, const float* c_sin,
+                     int64_t c_n_pos, float* comp32, void* comp, int64_t ncap, float* ring_kv, float* ring_sc,
+                     int32_t* pos, float eps, void* stream);
 
 /* smla_decode_ids: the decode id list of oracle/decode_engine.py:110-114 for B sequences at
  * positions pos [B]: ids [B, T] int32 (T >= window), columns 0..window-1 = the raw rows of

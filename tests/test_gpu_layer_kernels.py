@@ -203,3 +203,50 @@ def test_q_up(dev, T, heads, K):
     mag[..., 448::2] = mag[..., 449::2] = ma + mb       # |cos|, |sin| <= 1
     tol = ref.abs() * 2.0 ** -8 + (K + 8) * 2.0 ** -23 * mag
     assert bool(((out.double() - ref).abs() <= tol).all())
+
+
+@pytest.mark.parametrize("B,S,with_ring", [(1, 3, True), (2, 130, True), (2, 141, False), (3, 128, True)])
+def test_prompt_rows(dev, B, S, with_ring):
+    """smla_prompt_rows equals the separate calls: row epilogues of the kv rows, the gated pool, the
+    ring's initialisation and positions bit for bit; the q_a norm (another summation order) within half a
+    bf16 ulp plus the fp32 error of its sum."""
+    from smla import _lib, ops
+    from smla import compressor as scomp
+    from smla import norm_rope as snr
+    announce(f"prompt_rows B={B} S={S} ring={with_ring}")
+    g = torch.Generator(device=dev).manual_seed(B * S)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev)  # noqa: E731
+    cuts = [0, 1024, 1536] + ([2560, 3584] if with_ring else [])
+    y = rnd(B * S, cuts[-1])
+    qa_norm, kv_norm, nw, ape = 1 + 0.1 * rnd(1024), 1 + 0.1 * rnd(512), 1 + 0.1 * rnd(512), rnd(4, 1024)
+    cos_t, sin_t = snr.rope_tables(64, 512, device=dev)
+    ncap = S // 4 + 2
+    ring = lambda: scomp.Ring(B, 512, ape, nw, max_pos=512, device=dev)  # noqa: E731
+    r0, r1 = ring(), ring()
+    r0.ring_kv.normal_(generator=g)                       # stale contents are overwritten
+    raw = rnd(B, 128, 512).to(torch.bfloat16)
+    raw_ref = raw.clone()
+    comp32, comp = rnd(B, ncap, 512), rnd(B, ncap, 512).to(torch.bfloat16)
+    comp32_ref, comp_ref = comp32.clone(), comp.clone()
+    extra = dict(ring=r0, comp32=comp32, comp=comp) if with_ring else {}
+    qa, win, pos = ops.prompt_rows(y, cuts, B, S, qa_norm, kv_norm, cos_t, sin_t, raw, **extra)
+    assert torch.equal(pos, torch.arange(S, dtype=torch.int32, device=dev).repeat(B))
+    ref = torch.empty_like(win)
+    ops.row_epilogue(y[:, 1024:1536], kv_norm, pos, cos_t, sin_t, 64, _lib.SIM_FP8, ref.view(B * S, 512))
+    assert torch.equal(win, ref)
+    last = torch.arange(max(0, S - 128), S, device=dev)
+    raw_ref[:, last % 128] = ref[:, last]
+    assert torch.equal(raw, raw_ref)
+    if with_ring:
+        kvp, scp = y[:, 1536:2560].reshape(B, S, -1), y[:, 2560:].reshape(B, S, -1)
+        r1.init_from_prefill(kvp, scp)
+        assert torch.equal(r0.ring_kv, r1.ring_kv) and torch.equal(r0.ring_sc, r1.ring_sc)
+        cut = S - S % 4
+        if cut:
+            comp32_ref[:, :cut // 4] = ops.gated_pool_op(kvp[:, :cut], scp[:, :cut], ape, nw, r1.cos_t, r1.sin_t, 4, 64,
+                                                         1e-6, _lib.SIM_FP8)
+            comp_ref[:, :cut // 4] = comp32_ref[:, :cut // 4].to(torch.bfloat16)
+        assert torch.equal(comp32, comp32_ref) and torch.equal(comp, comp_ref)
+    x = y[:, :1024].double()
+    want = x * torch.rsqrt(x.square().mean(-1, keepdim=True) + 1e-6) * qa_norm.double()
+    assert bool(((qa.double() - want).abs() <= want.abs() * (2.0 ** -8 + 1024 * 2.0 ** -24)).all())
