@@ -53,8 +53,7 @@ __device__ inline float sub_rn_g(float a, float b) {
 }
 
 // inverse RoPE of 4 (x0, x1) bf16 pairs held in one 16-byte chunk, pairs p0 .. p0+3 at one position
-__device__ inline u32x4_t inv_rope4(u32x4_t v, const float* __restrict__ cs, const float* __restrict__ sn) {
-  const f32x4_t c = *(const f32x4_t*)cs, s = *(const f32x4_t*)sn;
+__device__ inline u32x4_t inv_rope4(u32x4_t v, f32x4_t c, f32x4_t s) {
 #pragma unroll
   for (int j = 0; j < 4; j++) {
     const float x0 = __uint_as_float(v[j] << 16), x1 = __uint_as_float(v[j] & 0xffff0000u);
@@ -120,7 +119,7 @@ __global__ __launch_bounds__(256) void gemm_kernel(const uint8_t* __restrict__ x
     if constexpr (ROPE) {
       if ((ks * KSTEP) % head_dim == head_dim - 64) {
 #pragma unroll
-        for (int i = 0; i < kChunks; i++) ra[i] = inv_rope4(ra[i], csp[i], snp[i]);
+        for (int i = 0; i < kChunks; i++) ra[i] = inv_rope4(ra[i], *(const f32x4_t*)csp[i], *(const f32x4_t*)snp[i]);
       }
     }
 #pragma unroll
@@ -243,7 +242,7 @@ struct RingArgs {
   const int32_t* pos;
   const float* cos_t;
   const float* sin_t;
-  int head_dim;
+  uint32_t head_steps, head_magic;  // ROPE: K steps of 64 per head, ceil(2^32 / head_steps)
   uint8_t* y;
   int64_t ldy, split_stride;  // elements
   int vec;                    // rows and groups of y start at multiples of 16 bytes
@@ -357,26 +356,38 @@ gemm_ring_kernel(const RingArgs p) {
   const uint8_t* wk = group_weights(p, g, 2) + (int64_t)n0 * p.K * 2 + (int64_t)k0 * kRow;
 
   const int rot = id.in_group * p.rot % (k1 - k0);
-  // ROPE: the chunks of x this thread rotates in a step that holds a head's last 64 dims: chunk
-  // tid + i threads (row j / 8, slot j mod 8, 4 (x0, x1) pairs from pair 4 c, c = slot ^ ((row / 2) mod
-  // 8)); offsets of their rows in the cos / sin tables (32 pairs per position)
+  // ROPE: the chunks of x this thread rotates in a step that holds a head's last 64 dims: chunk tid + i
+  // threads is row j / 8, slot j mod 8, 4 (x0, x1) pairs from pair 4 c, c = slot ^ ((row / 2) mod 8).  Their
+  // rotations are the same in every such step: loaded once, waited for once (with the first stage),
+  // because a wait for a load inside the loop drains the ring's copies with it (the output path of 300
+  // tokens 83 -> 81 us)
   constexpr int NT = L::NW * 64, ACH = BM * 8 / NT;
-  int prow[ACH] = {};
+  f32x4_t cs[ACH], sn[ACH];
   if constexpr (ROPE) {
 #pragma unroll
-    for (int i = 0; i < ACH; i++) prow[i] = p.pos[min(t0 + (((int)threadIdx.x + NT * i) >> 3), p.T - 1)] * 32;
+    for (int i = 0; i < ACH; i++) {
+      const int j = threadIdx.x + NT * i, c = (j & 7) ^ ((j >> 4) & 7);
+      const int64_t at = (int64_t)p.pos[min(t0 + (j >> 3), p.T - 1)] * 32 + 4 * c;
+      cs[i] = *(const f32x4_t*)(p.cos_t + at);
+      sn[i] = *(const f32x4_t*)(p.sin_t + at);
+    }
   }
   f32x16_t acc[L::MB][L::NB];
   tile_loop<BM, BN, WM, WN, D>((lds_u8_t*)lds_g, xk, p.ldx, p.T - 1 - t0, wk, (int64_t)p.K * 2, p.N - 1 - n0, k1 - k0,
-                               rot, acc, [&](int ks, lds_u8_t* stage) __attribute__((always_inline)) {
+                               rot, acc, [&](int ks, lds_u8_t* stage, auto first) __attribute__((always_inline)) {
     if constexpr (ROPE) {
-      const int k = ks + rot < k1 - k0 ? ks + rot : ks + rot - (k1 - k0);
-      if (((k0 + k) * 64) % p.head_dim == p.head_dim - 64) {
+      if constexpr (decltype(first)::value) {
+#pragma unroll
+        for (int i = 0; i < ACH; i++) asm volatile("" : "+v"(cs[i]), "+v"(sn[i]));
+      }
+      // step k of the row holds dims 64 (k mod head_steps) .. of a head (k < 2^16: the product is exact)
+      const uint32_t k = k0 + (ks + rot < k1 - k0 ? ks + rot : ks + rot - (k1 - k0));
+      if (p.head_steps == 1 || k - __umulhi(k, p.head_magic) * p.head_steps == p.head_steps - 1) {
 #pragma unroll
         for (int i = 0; i < ACH; i++) {
-          const int j = threadIdx.x + NT * i, r = j >> 3, sl = j & 7, c = sl ^ ((r >> 1) & 7);
-          lds_u32x4_t* pa = (lds_u32x4_t*)(stage + r * kRow + 16 * sl);
-          *pa = inv_rope4(*pa, p.cos_t + prow[i] + 4 * c, p.sin_t + prow[i] + 4 * c);
+          const int j = threadIdx.x + NT * i;
+          lds_u32x4_t* pa = (lds_u32x4_t*)(stage + (j >> 3) * kRow + 16 * (j & 7));
+          *pa = inv_rope4(*pa, cs[i], sn[i]);
         }
         lds_barrier();
       }
@@ -467,7 +478,7 @@ __global__ __launch_bounds__(512) void gemm_heads_kernel(const RingArgs p, int64
   f32x16_t acc[L::MB][L::NB];
   tile_loop<F::BM, F::BN, F::WM, F::WN, F::D>(lds, p.x + (int64_t)t0 * p.ldx, p.ldx, p.T - 1 - t0,
                                               p.w + (int64_t)n0 * p.K * 2, (int64_t)p.K * 2, F::BN - 1, p.K / 64, 0, acc,
-                                              [](int, lds_u8_t*) {});
+                                              [](int, lds_u8_t*, auto) {});
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = wave % 2, wn = wave / 2;
   // sums of squares: a row's 512 values sit in the 32 lanes of a half wave of four waves; the waves' sums
   // and then the rows' factors go through LDS past the region the stores use
@@ -682,8 +693,9 @@ int launch_gemm_tiled(const void* x, int64_t ldx, bool f32_operands, const void*
     const int64_t nt = (T + bm - 1) / bm, nn = (N + bn - 1) / bn, wgs = nt * nn * G * p.splits;
     if (wgs > 0x7fffffff) return SMLA_E_UNSUPPORTED;
     const int64_t es = f32_operands ? 4 : 2;
+    const uint32_t hs = pos ? (uint32_t)(head_dim / 64) : 1u;
     RingArgs a{(const uint8_t*)x, (const uint8_t*)w, (const uint8_t*)w2, ldx * es, w2 ? 0 : K * es, (int)T, (int)N, (int)K, (int)G, (int)nt,
-               (int)nn, p.splits, pos, cos_t, sin_t, (int)head_dim, (uint8_t*)(p.splits > 1 ? ws : y), ldy, T * ldy, 0, 0};
+               (int)nn, p.splits, pos, cos_t, sin_t, hs, hs > 1 ? (uint32_t)(((1ull << 32) + hs - 1) / hs) : 0u, (uint8_t*)(p.splits > 1 ? ws : y), ldy, T * ldy, 0, 0};
     const int odt = p.splits > 1 ? SMLA_F32 : y_dtype;
     // rows of x 64 KB apart fall in the same sets of an L2, which the 4 token tiles of a group would
     // then all want at once: they start 4 steps apart (8 groups of [4096, 4096] x [1024, 4096]^T 281 ->
@@ -736,7 +748,7 @@ int launch_gemm_heads(const void* x, const void* w, int64_t T, int64_t heads, in
   const int64_t nt = (T + F::BM - 1) / F::BM, wgs = nt * heads;
   if (wgs > 0x7fffffff) return SMLA_E_UNSUPPORTED;
   RingArgs a{(const uint8_t*)x, (const uint8_t*)w, nullptr, K * 2, 0, (int)T, (int)(heads * 512), (int)K, 1, (int)nt,
-             (int)heads, 1, pos, cos_t, sin_t, 512, (uint8_t*)out, heads * 512, 0, 1, 0};
+             (int)heads, 1, pos, cos_t, sin_t, 8, 0, (uint8_t*)out, heads * 512, 0, 1, 0};
   static std::atomic<uint64_t> lds_attr{0};
   if (hipError_t e = smla_set_dynamic_lds((const void*)gemm_heads_kernel, L::LDS, lds_attr); e != hipSuccess) return (int)e;
   hipLaunchKernelGGL(gemm_heads_kernel, dim3((unsigned)wgs), dim3(L::NW * 64), L::LDS, st, a, n_pos, eps);

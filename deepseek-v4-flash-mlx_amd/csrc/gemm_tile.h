@@ -55,8 +55,8 @@ struct Tile {
 // times rows 0 .. BN-1 of w (likewise), over nk >= D steps of 64 k.  Accumulator register r of block
 // (mb, nb) is row WM wm + 32 mb + 8 (r / 4) + 4 (lane / 32) + r mod 4 of x, row WN wn + 32 nb +
 // lane mod 32 of w, for wave wm + (BM / WM) wn.  BM ldx and BN ldw fit 31 bits.
-// The steps run from step rot (0 <= rot < nk) round to rot - 1.  landed(step, stage): run after the
-// stage of the step-th of them has landed and before it is read.
+// The steps run from step rot (0 <= rot < nk) round to rot - 1.  landed(step, stage, Int<first>): run after
+// the stage of the step-th of them has landed and before it is read.
 template <int BM, int BN, int WM, int WN, int D, class F>
 __device__ __attribute__((always_inline)) inline void tile_loop(lds_u8_t* lds, const uint8_t* __restrict__ xk,
                                                                 int64_t ldx, int tmax, const uint8_t* __restrict__ wk,
@@ -123,7 +123,7 @@ __device__ __attribute__((always_inline)) inline void tile_loop(lds_u8_t* lds, c
     if constexpr (next) {
       wait_vm(more ? (D - 2) * L::CP : 0);  // this wave's copies of step ks + 1
       lds_barrier();                         // everyone's; and step ks is in every wave's registers
-      landed(ks + 1, lds + ((ks + 1) % D) * L::STAGE);
+      landed(ks + 1, lds + ((ks + 1) % D) * L::STAGE, Int<0>{});
       sub(Int<1>{}, ks + 1, Int<0>{}, ks + D, Int<0>{}, Int<first ? Q3 : 0>{});
     } else {
       sub(Int<1>{}, 0, Int<-1>{}, 0, Int<0>{}, Int<0>{});
@@ -141,7 +141,7 @@ __device__ __attribute__((always_inline)) inline void tile_loop(lds_u8_t* lds, c
     for (int i = 0; i < (s < D - 1 ? L::CP : Q3); i++) copy(s, i);
   wait_vm((D - 2) * L::CP + Q3);
   lds_barrier();
-  landed(0, lds);
+  landed(0, lds, Int<1>{});
 #pragma unroll
   for (int i = 0; i < NR; i++) read(0, 0, 0, i);
   int ks = 0;

@@ -237,6 +237,27 @@ def test_o_proj_fused_rope_wide(dev, T):
     np.testing.assert_allclose(fused.cpu()[idx].double().numpy(), ref, rtol=1e-2, atol=2e-2 * np.abs(ref).max())
 
 
+@pytest.mark.parametrize("T", [40, 300])
+@pytest.mark.parametrize("H,D,G", [(8, 64, 1), (12, 192, 2), (4, 320, 2)])
+def test_o_proj_fused_rope_head_dims(dev, T, H, D, G):
+    """Heads of 1, 3 and 5 K steps of 64 (not only the layer's 8): the fused rotation finds each head's
+    last 64 dims, with and without a split K range."""
+    from smla import norm_rope as snr
+    from smla import ops
+    announce(f"o_proj T={T} heads={H} head_dim={D} groups={G}")
+    g = torch.Generator(device=dev).manual_seed(T + D)
+    o = torch.randn(T, H, D, generator=g, device=dev).to(torch.bfloat16)
+    wa = (torch.randn(G * 128, H * D // G, generator=g, device=dev) * 0.05).to(torch.bfloat16)
+    wb = (torch.randn(256, G * 128, generator=g, device=dev) * 0.05).to(torch.bfloat16)
+    pos = torch.randint(0, 4096, (T,), generator=g, device=dev, dtype=torch.int32)
+    cos_t, sin_t = snr.rope_tables(64, 4096, device=dev)
+    rot = o.clone()
+    ops.rope_op_(rot, pos, cos_t, sin_t, True)
+    assert not torch.equal(rot, o)
+    fused = ops.o_proj_op(o, pos, cos_t, sin_t, wa, wb, G, torch.float32)
+    assert torch.equal(fused, ops.o_proj_op(rot, None, None, None, wa, wb, G, torch.float32))
+
+
 def test_mla_mirror_routes(dev):
     """mla.linear / o_grouped / o_project run the weight-streaming kernels at decode shapes and the
     tiled GEMM beyond; both agree with the oracle."""
