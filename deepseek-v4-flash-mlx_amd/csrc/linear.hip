@@ -369,10 +369,13 @@ bool decode_form(int x_dtype, int64_t T, int64_t N, int64_t K) {
 // Whether a shape that the decode form can take runs on it.  From 9 rows on the tiled GEMM is faster
 // when its plan needs no workspace or has it ([12, 4096] x [1024, 4096]^T 7.4 against 9.4 us, [32, 1024]
 // x [32768, 1024]^T 12.6 against 32.7: the decode kernel re-reads x from L2 per 16 outputs), slower
-// when it would have to split K and cannot (16 against 8.6 us for [12, 4096] x [512, 4096]^T).
-bool decode_runs(int x_dtype, int64_t T, int64_t G, int64_t N, int64_t K, bool tiled_can, bool has_ws) {
+// when it would have to split K and cannot (16 against 8.6 us for [12, 4096] x [512, 4096]^T).  With RoPE
+// on load it takes over after 16 rows: its rotated steps stand in line with its MFMAs (the output path of
+// 16 tokens 43.1 against 41.9 us).
+bool decode_runs(int x_dtype, int64_t T, int64_t G, int64_t N, int64_t K, bool tiled_can, bool has_ws,
+                 bool rope = false) {
   if (!decode_form(x_dtype, T, N, K)) return false;
-  return T <= 8 || !tiled_can || !gemm_tiled_takes(G, K) || (gemm_tiled_workspace(T, G, N, K, false) > 0 && !has_ws);
+  return T <= (rope ? 16 : 8) || !tiled_can || !gemm_tiled_takes(G, K) || (gemm_tiled_workspace(T, G, N, K, false) > 0 && !has_ws);
 }
 
 int check_linear(const void* x, int x_dtype, const void* w, int w_dtype, int64_t T, int64_t G, int64_t N, int64_t K,
@@ -498,7 +501,8 @@ extern "C" int smla_o_proj_ws(const void* o, int o_dtype, const int32_t* pos, co
   if (rc) return rc;
   const bool rot64 = !pos || rd == 64;  // the tiled GEMM rotates exactly the last 64 dims of each head
   const bool dform = decode_runs(o_dtype, T, G, R, Kg, rot64,
-                                 workspace && workspace_bytes >= smla_linear_workspace(T, G, R, Kg, SMLA_BF16));
+                                 workspace && workspace_bytes >= smla_linear_workspace(T, G, R, Kg, SMLA_BF16),
+                                 pos != nullptr);
   if (pos) {
     rc = check_rope_args(pos, cos_t, sin_t, n_pos, heads, head_dim, rd);
     if (rc) return rc;
