@@ -1,4 +1,5 @@
-// Projections of the decode step: few tokens (at most 32) against a large bf16 weight, on MFMA.
+// Projections of the decode step: few tokens against a large bf16 weight, on MFMA (which calls: see
+// decode_form and decode_runs below; the others run the tiled kernels of gemm.hip).
 //
 //  * linear_kernel<TT, ROPE, YDT> : y[t, n] = sum_k x'[t, g*K + k] * W[n, k] for the rows n of
 //      group g = n / N (G groups of N rows; G = 1 is a plain linear).  With ROPE, x is the
@@ -366,16 +367,36 @@ bool decode_form(int x_dtype, int64_t T, int64_t N, int64_t K) {
   return x_dtype == SMLA_BF16 && T <= 32 && N % 16 == 0 && K % (64 * kLinWaves) == 0;
 }
 
-// Whether a shape that the decode form can take runs on it.  From 9 rows on the tiled GEMM is faster
-// when its plan needs no workspace or has it ([12, 4096] x [1024, 4096]^T 7.4 against 9.4 us, [32, 1024]
-// x [32768, 1024]^T 12.6 against 32.7: the decode kernel re-reads x from L2 per 16 outputs), slower
-// when it would have to split K and cannot (16 against 8.6 us for [12, 4096] x [512, 4096]^T).  With RoPE
-// on load it takes over after 16 rows: its rotated steps stand in line with its MFMAs (the output path of
-// 16 tokens 43.1 against 41.9 us).
+// Up to 32 rows, the decode kernels against the tiled GEMM.  A decode workgroup (16 outputs) reads all of x
+// from L2 and runs K / 8 of it per wave, so its time grows with the workgroups per CU, with the rows and
+// with K; the GEMM's 64-wide tiles split K over up to 8 workgroups, which costs a second launch and
+// leaves its time nearly the same from 9 to 32 rows.  Up to 8 rows (x in LDS) the decode kernels are faster
+// throughout.  Measured (us, decode / tiled, weights from HBM; W = workgroups = outputs / 16):
+//   9..16 rows   W  64  K 4096  8.9..10.2 /  8.3      W 512  K 2048  11.4..12.6 / 14.1..12.3
+//                W  96  K 4096  9.3..10.5 /  9.3      W 512  K 4096  19.4..21.3 / 24.1..21.4
+//                W 128  K 4096  9.4..10.5 /  9.8      W 512  K 8192  31.1..35.3 / 27.3
+//                W 160  K 8192 17.3..18.2 / 16.9      W 1024 K  512   9.0.. 9.7 /  6.1
+//                W 192  K 8192 18.0..18.4 / 20.1      W 1024 K 2048  20.7..22.1 / 18.9
+//                W 256  K 8192 18.2..19.1 / 20.4..19.1
+//   17..32 rows  W  64  K 2048  6.6.. 7.9 /  6.9      W 256  K 1024   4.9.. 5.6 /  7.3
+//                W 128  K 2048  6.9.. 8.3 /  8.0      W 512  K  512   6.3.. 6.9 /  5.4
+//                W 256  K 2048  7.3.. 8.6 /  9.7      W 256  K 4096  12.2..14.8 / 12.6
+bool decode_faster(int64_t T, int64_t G, int64_t N, int64_t K) {
+  const int64_t wgs = G * N / 16;
+  if (T <= 8) return true;
+  if (T <= 16) return wgs <= 512 && wgs * K <= 512 * 4096 && !(K >= 4096 && wgs <= 96 + (K - 4096) / 64);
+  return wgs <= 256 && K <= 2048 && !(K == 2048 && wgs <= 64);
+}
+
+// Whether a shape that the decode form can take runs on it: where it is faster, where the tiled GEMM does
+// not take the shape, or would have to split K without the workspace (16 against 8.6 us for [12, 4096] x
+// [512, 4096]^T).  With RoPE on load up to 16 rows stay: the GEMM's rotated steps stand in line with its
+// MFMAs (the output path of 16 tokens 43.1 against 41.9 us).
 bool decode_runs(int x_dtype, int64_t T, int64_t G, int64_t N, int64_t K, bool tiled_can, bool has_ws,
                  bool rope = false) {
   if (!decode_form(x_dtype, T, N, K)) return false;
-  return T <= (rope ? 16 : 8) || !tiled_can || !gemm_tiled_takes(G, K) || (gemm_tiled_workspace(T, G, N, K, false) > 0 && !has_ws);
+  return (rope && T <= 16) || decode_faster(T, G, N, K) || !tiled_can || !gemm_tiled_takes(G, K) ||
+         (gemm_tiled_workspace(T, G, N, K, false) > 0 && !has_ws);
 }
 
 int check_linear(const void* x, int x_dtype, const void* w, int w_dtype, int64_t T, int64_t G, int64_t N, int64_t K,

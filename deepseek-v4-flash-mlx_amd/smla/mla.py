@@ -2,9 +2,9 @@
 
 These dense GEMMs surround the sparse-attention core, with the reference's shapes: H=64 heads,
 head_dim 512, rope 64, 8 output groups of rank 1024.  Every product runs in libsmla's HIP kernels
-(``smla_linear`` / ``smla_o_proj``): up to 32 bf16 token rows (decode) the weight-streaming MFMA
-kernel, bound by reading the weights once; larger batches (prefill) the tiled MFMA GEMM, with the
-inverse RoPE of ``o_project`` fused into its operand load.  Every function refuses tensors that are
+(``smla_linear_ws`` / ``smla_o_proj_ws``): up to 8 bf16 token rows (decode), up to 32 where it is the
+faster form, the weight-streaming MFMA kernel, bound by reading the weights once; larger batches the
+tiled MFMA GEMM, with the inverse RoPE of ``o_project`` fused into its operand load.  Every function refuses tensors that are
 not on the GPU.
 """
 import torch

@@ -485,7 +485,7 @@ _YDT = {torch.float32: _lib.F32, torch.bfloat16: _lib.BF16}
 
 def _linear(x: torch.Tensor, w: torch.Tensor, groups: int, out_dtype: torch.dtype) -> torch.Tensor:
     """x [T, G*K], w [G*N, K] (both bf16 or both fp32) -> y [T, G*N]: y[:, gN:(g+1)N] = x[:, gK:(g+1)K] @ w_g^T
-    (the weight-streaming kernel up to 32 bf16 rows, the tiled MFMA GEMM otherwise)."""
+    (the weight-streaming kernel for few bf16 rows, the tiled MFMA GEMM otherwise)."""
     _on_gpu(x, w)
     x, w = x.contiguous(), w.contiguous()
     T = x.shape[0]
@@ -494,7 +494,7 @@ def _linear(x: torch.Tensor, w: torch.Tensor, groups: int, out_dtype: torch.dtyp
     if x.shape[1] != groups * K or w.shape[0] != groups * N:
         raise ValueError("linear: x [T, G*K] and w [G*N, K] do not agree")
     y = torch.empty(T, groups * N, dtype=out_dtype, device=x.device)
-    # no workspace up to 8 rows on the weight-streaming kernel (the library says 0 there)
+    # no workspace up to 8 rows, always on the weight-streaming kernel (the library says 0 there)
     wsb = 0 if T <= 8 and x.dtype == torch.bfloat16 and K % 512 == 0 and N % 16 == 0 else \
         _lib.lib().smla_linear_workspace(T, groups, N, K, dtype_code(x))
     ws = torch.empty(wsb, dtype=torch.uint8, device=x.device) if wsb else None

@@ -463,8 +463,8 @@ int smla_rope(void* x, int x_dtype, int64_t T, int64_t heads, int64_t head_dim, 
  *   x [T, G*K], w [G*N, K]: both BF16 or both F32; y [T, G*N] BF16 or F32; float32 accumulation.
  *   16-byte aligned pointers; K % 8 == 0 (BF16) or K % 4 == 0 (F32); any T >= 1.
  *   Decode shapes (BF16, T <= 8, N % 16 == 0, K % 512 == 0) stream w from HBM once (the bound), and
- *   so do up to 32 rows where the tiled GEMM would need a workspace it does not have (and up to 16
- *   with smla_o_proj's rotation); other shapes run a tiled MFMA GEMM. */
+ *   so do up to 32 rows where that is the faster form or the tiled GEMM would need a workspace it does
+ *   not have; other shapes run a tiled MFMA GEMM. */
 int smla_linear(const void* x, int x_dtype, const void* w, int w_dtype, int64_t T, int64_t G,
                 int64_t N, int64_t K, void* y, int y_dtype, void* stream);
 

@@ -105,6 +105,18 @@ def test_linear_tile_forms(dev, T, G, N, K, out_dtype):
 
 
 @pytest.mark.parametrize("T,G,N,K", [
+    # both sides of the lines between the weight-streaming kernels and the tiled GEMM
+    (16, 1, 8192, 512), (9, 1, 8208, 512),            # 512 and 513 workgroups of 16 outputs
+    (9, 2, 4096, 4096), (16, 1, 8192, 4608),          # 512 x 4096 and beyond
+    (12, 1, 1536, 4096), (12, 1, 1552, 4096),         # few outputs of a long K
+    (17, 1, 4096, 2048), (17, 1, 4112, 2048), (32, 1, 4096, 2560),
+    (32, 1, 1024, 2048), (32, 1, 1040, 2048),
+])
+def test_linear_few_rows(dev, T, G, N, K):
+    test_linear_tile_forms(dev, T, G, N, K, torch.float32)
+
+
+@pytest.mark.parametrize("T,G,N,K", [
     (1, 1, 1024, 4096),      # 64 x 64 tiles, eight splits
     (70, 1, 333, 512),       # odd N: element-wise stores
     (129, 2, 136, 64),       # two steps of 32 k: 128 x 128 tiles, one token past the first
@@ -150,7 +162,7 @@ def test_linear_fp32_special_values(dev, T, N, K):
     assert bool(((y.double() - ref).abs()[ok] <= tol[ok]).all())
 
 
-@pytest.mark.parametrize("T,G,N,K", [(9, 1, 64, 1536), (17, 2, 48, 1024), (32, 1, 512, 4096), (100, 1, 1024, 4096)])
+@pytest.mark.parametrize("T,G,N,K", [(9, 1, 64, 4096), (17, 2, 48, 4096), (32, 1, 512, 4096), (100, 1, 1024, 4096)])
 def test_linear_without_workspace(dev, T, G, N, K):
     """smla_linear (no workspace): 9 to 32 rows whose GEMM would split K run the weight-streaming
     kernel, more rows the GEMM without the split; both as exact as with a workspace."""
