@@ -7,9 +7,9 @@
 //   score = acc * kscale[n]   (or acc when kscale == NULL);  -inf for n >= nvis
 //
 // The order is fixed so that every score is reproducible bit for bit by the CPU oracle; the top-k
-// that follows can then be compared exactly.  Hi = Di = 64 (the decode shape) runs the dot-product
-// chains on the matrix cores (indexer_mfma_kernel: K = 1 fp32 MFMAs, each one rounding, so the
-// chain is the same sequence of fmas); other head counts run them on the vector ALUs
+// that follows can then be compared exactly.  64 heads of 64 or 128 dims (the decode and the indexer-key
+// shapes) run the dot-product chains on the matrix cores (indexer_mfma_kernel: K = 1 fp32 MFMAs, each
+// one rounding, so the chain is the same sequence of fmas); other shapes run them on the vector ALUs
 // (indexer_kernel: 64 keys per workgroup, one per lane, key row in VGPRs as fp32, waves splitting
 // the heads 16 at a time with q and w staged in LDS as fp32 and read as wave-wide broadcasts).
 // HBM traffic per query row: N * (Di * sizeof(key) + 4) bytes of keys and scales, N * 4 bytes of
@@ -206,8 +206,8 @@ __global__ __launch_bounds__(256) void indexer_kernel(const void* __restrict__ q
   if (n < N) scores[bs * N + n] = live ? (kscale ? acc * kscale[row] : acc) : -SMLA_INF;
 }
 
-// Hi = Di = 64 on the matrix cores.  v_mfma_f32_32x32x1_2b_f32 (K = 1) adds one product to each
-// accumulator with a single rounding, so a chain of 64 of them over d = 0..63 is, element for
+// Hi = 64, Di = 64 or 128 on the matrix cores.  v_mfma_f32_32x32x1_2b_f32 (K = 1) adds one product to
+// each accumulator with a single rounding, so a chain of Di of them over d = 0..Di-1 is, element for
 // element, the fma chain dot_h = fma(q[h,d], k[n,d], dot_h) of the definition above (bit for bit:
 // checked against fmaf over 6.7e7 operand triples, subnormal, cancelling and overflowing ones
 // included), at twice the rate of fp32 fma on the vector ALUs.  A wave computes a tile of 64 heads x
@@ -227,8 +227,14 @@ __global__ __launch_bounds__(256) void indexer_kernel(const void* __restrict__ q
 // (h = lane again) and the key n = lane mod 16; register j of lane l holds head 16 (j / 4) + 4 (l / 16)
 // + j mod 4.  The head chain walks the 16-lane rows: after the four heads of row g, every row takes
 // row g's sum (two lane swaps).
+//
+// Di = 128 doubles the chain and the registers of a key row, and q is converted where it is used: 1024
+// queries x 64 heads over 2048 fp4 keys with the top-k take 310 us at three waves per SIMD (bf16 q, keys
+// of at most 256 bytes; 321 at two, where fp32 q or keys stay) against 676 on the vector ALUs, which read
+// q from LDS.  Bound by the MFMA chain: 64 cycles a dependent step, tiles past nvis skip theirs.
 template <int DI, int KDT, int QDT, int KT = 32>
-__global__ __launch_bounds__(256, DI == 128 && QDT == SMLA_BF16 && KDT != SMLA_F32 ? 3 : 1) void indexer_mfma_kernel(const void* __restrict__ q, const void* __restrict__ keys,
+__global__ __launch_bounds__(256, DI == 128 && QDT == SMLA_BF16 && KDT != SMLA_F32 ? 3 : 1)
+void indexer_mfma_kernel(const void* __restrict__ q, const void* __restrict__ keys,
                                                        const uint8_t* __restrict__ kbs,
                                                        const float* __restrict__ kscale,
                                                        const float* __restrict__ weights,

@@ -26,8 +26,9 @@ positions), ratio-0 layers plain base 10000 (``decode_engine.py:47,73``).  Every
 ``smla_linear`` (projections, fp32 results), ``smla_row_epilogue`` (the norms, RoPE, the fp8 round
 trip and the window-ring write; in a step, ``smla_ring_step_kv`` runs it with the compressor ring
 step in one launch), ``smla_row_epilogue_ids`` (the per-head q epilogue with the id build),
-``smla_select_decode`` (the indexer top-k form), ``smla_sparse_attn``, ``smla_prefill_attn``
-(prompts) and ``smla_o_proj``.  Caches are device-resident and owned by the layer object: the
+``smla_select_decode`` (the indexer top-k form), ``smla_sparse_attn`` and ``smla_o_proj``; a prompt's
+``smla_q_up`` (the q up projection with its per-head epilogue), ``smla_prompt_rows`` (what the other
+projections feed, in one launch) and ``smla_prefill_attn``.  Caches are device-resident and owned by the layer object: the
 window is a 128-row ring whatever ``max_pos`` is, the compressed cache holds ``max_pos // 4``
 rows (the reference's compressed list grows with the context the same way).
 """
