@@ -246,7 +246,6 @@ struct RingArgs {
   uint8_t* y;
   int64_t ldy, split_stride;  // elements
   int vec;                    // rows and groups of y start at multiples of 16 bytes
-  int rot;                    // K steps between the starts of neighbouring token tiles
 };
 
 // The tile's outputs from the accumulators (layout of tile_loop) to rows t0 .., columns n0 .. of group g
@@ -319,7 +318,7 @@ __device__ __attribute__((always_inline)) inline void store_tile(smla_attn::lds_
 // contiguous run of tiles, ordered in groups of 4 token tiles over all output tiles, so that the
 // tiles running together on an XCD share x and w rows in its L2.  Splits are outermost.
 struct TileId {
-  int sp, g, tm, tn, in_group;  // split, group, token tile, output tile; token tile within its 4
+  int sp, g, tm, tn;  // split, group, token tile, output tile
 };
 __device__ inline TileId tile_id(const RingArgs& p) {
   const uint32_t tot = gridDim.x, per = tot / kXcds, rem = tot % kXcds, xcd = blockIdx.x % kXcds;
@@ -331,8 +330,7 @@ __device__ inline TileId tile_id(const RingArgs& p) {
   TileId t;
   t.sp = sg / p.G;
   t.g = sg - t.sp * p.G;
-  t.in_group = in % gs;
-  t.tm = 4 * grp + t.in_group;
+  t.tm = 4 * grp + in % gs;
   t.tn = in / gs;
   return t;
 }
@@ -355,7 +353,6 @@ gemm_ring_kernel(const RingArgs p) {
   const uint8_t* xk = p.x + (int64_t)t0 * p.ldx + g * p.xg + (int64_t)k0 * kRow;
   const uint8_t* wk = group_weights(p, g, 2) + (int64_t)n0 * p.K * 2 + (int64_t)k0 * kRow;
 
-  const int rot = id.in_group * p.rot % (k1 - k0);
   // ROPE: the chunks of x this thread rotates in a step that holds a head's last 64 dims: chunk tid + i
   // threads is row j / 8, slot j mod 8, 4 (x0, x1) pairs from pair 4 c, c = slot ^ ((row / 2) mod 8).  Their
   // rotations are the same in every such step: loaded once, waited for once (with the first stage),
@@ -374,14 +371,14 @@ gemm_ring_kernel(const RingArgs p) {
   }
   f32x16_t acc[L::MB][L::NB];
   tile_loop<BM, BN, WM, WN, D>((lds_u8_t*)lds_g, xk, p.ldx, p.T - 1 - t0, wk, (int64_t)p.K * 2, p.N - 1 - n0, k1 - k0,
-                               rot, acc, [&](int ks, lds_u8_t* stage, auto first) __attribute__((always_inline)) {
+                               acc, [&](int ks, lds_u8_t* stage, auto first) __attribute__((always_inline)) {
     if constexpr (ROPE) {
       if constexpr (decltype(first)::value) {
 #pragma unroll
         for (int i = 0; i < ACH; i++) asm volatile("" : "+v"(cs[i]), "+v"(sn[i]));
       }
       // step k of the row holds dims 64 (k mod head_steps) .. of a head (k < 2^16: the product is exact)
-      const uint32_t k = k0 + (ks + rot < k1 - k0 ? ks + rot : ks + rot - (k1 - k0));
+      const uint32_t k = k0 + ks;
       if (p.head_steps == 1 || k - __umulhi(k, p.head_magic) * p.head_steps == p.head_steps - 1) {
 #pragma unroll
         for (int i = 0; i < ACH; i++) {
@@ -477,7 +474,7 @@ __global__ __launch_bounds__(512) void gemm_heads_kernel(const RingArgs p, int64
   const int t0 = id.tm * F::BM, n0 = id.tn * F::BN;
   f32x16_t acc[L::MB][L::NB];
   tile_loop<F::BM, F::BN, F::WM, F::WN, F::D>(lds, p.x + (int64_t)t0 * p.ldx, p.ldx, p.T - 1 - t0,
-                                              p.w + (int64_t)n0 * p.K * 2, (int64_t)p.K * 2, F::BN - 1, p.K / 64, 0, acc,
+                                              p.w + (int64_t)n0 * p.K * 2, (int64_t)p.K * 2, F::BN - 1, p.K / 64, acc,
                                               [](int, lds_u8_t*, auto) {});
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = wave % 2, wn = wave / 2;
   // sums of squares: a row's 512 values sit in the 32 lanes of a half wave of four waves; the waves' sums
@@ -695,12 +692,8 @@ int launch_gemm_tiled(const void* x, int64_t ldx, bool f32_operands, const void*
     const int64_t es = f32_operands ? 4 : 2;
     const uint32_t hs = pos ? (uint32_t)(head_dim / 64) : 1u;
     RingArgs a{(const uint8_t*)x, (const uint8_t*)w, (const uint8_t*)w2, ldx * es, w2 ? 0 : K * es, (int)T, (int)N, (int)K, (int)G, (int)nt,
-               (int)nn, p.splits, pos, cos_t, sin_t, hs, hs > 1 ? (uint32_t)(((1ull << 32) + hs - 1) / hs) : 0u, (uint8_t*)(p.splits > 1 ? ws : y), ldy, T * ldy, 0, 0};
+               (int)nn, p.splits, pos, cos_t, sin_t, hs, hs > 1 ? (uint32_t)(((1ull << 32) + hs - 1) / hs) : 0u, (uint8_t*)(p.splits > 1 ? ws : y), ldy, T * ldy, 0};
     const int odt = p.splits > 1 ? SMLA_F32 : y_dtype;
-    // rows of x 64 KB apart fall in the same sets of an L2, which the 4 token tiles of a group would
-    // then all want at once: they start 4 steps apart (8 groups of [4096, 4096] x [1024, 4096]^T 281 ->
-    // 262 us; with closer rows, which it does not help, a rotation costs up to 3 %)
-    a.rot = !f32_operands && p.form == 3 && a.ldx % 65536 == 0 ? 4 : 0;
     a.vec = N % (odt == SMLA_BF16 ? 8 : 4) == 0 && ((uintptr_t)a.y & 15) == 0;
     const int rc = f32_operands  ? (p.form == 0 ? launch_f32<0>(a, wgs, odt, st) : launch_f32<1>(a, wgs, odt, st))
                    : p.form == 0 ? launch_ring<0>(a, wgs, pos != nullptr, odt, st)
@@ -748,7 +741,7 @@ int launch_gemm_heads(const void* x, const void* w, int64_t T, int64_t heads, in
   const int64_t nt = (T + F::BM - 1) / F::BM, wgs = nt * heads;
   if (wgs > 0x7fffffff) return SMLA_E_UNSUPPORTED;
   RingArgs a{(const uint8_t*)x, (const uint8_t*)w, nullptr, K * 2, 0, (int)T, (int)(heads * 512), (int)K, 1, (int)nt,
-             (int)heads, 1, pos, cos_t, sin_t, 8, 0, (uint8_t*)out, heads * 512, 0, 1, 0};
+             (int)heads, 1, pos, cos_t, sin_t, 8, 0, (uint8_t*)out, heads * 512, 0, 1};
   static std::atomic<uint64_t> lds_attr{0};
   if (hipError_t e = smla_set_dynamic_lds((const void*)gemm_heads_kernel, L::LDS, lds_attr); e != hipSuccess) return (int)e;
   hipLaunchKernelGGL(gemm_heads_kernel, dim3((unsigned)wgs), dim3(L::NW * 64), L::LDS, st, a, n_pos, eps);

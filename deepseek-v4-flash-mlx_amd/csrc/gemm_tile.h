@@ -55,12 +55,14 @@ struct Tile {
 // times rows 0 .. BN-1 of w (likewise), over nk >= D steps of 64 k.  Accumulator register r of block
 // (mb, nb) is row WM wm + 32 mb + 8 (r / 4) + 4 (lane / 32) + r mod 4 of x, row WN wn + 32 nb +
 // lane mod 32 of w, for wave wm + (BM / WM) wn.  BM ldx and BN ldw fit 31 bits.
-// The steps run from step rot (0 <= rot < nk) round to rot - 1.  landed(step, stage, Int<first>): run after
-// the stage of the step-th of them has landed and before it is read.
+// An output is one chain of fp32 accumulations over k = 0, 16, 32 ..: tiles whose rows of x lie 64 KB apart
+// (the same sets of an L2) ran 4 steps apart once (8 groups of [4096, 4096] x [1024, 4096]^T 281 -> 262 us),
+// but a token's sums then depended on where it stands in the prompt.  landed(step, stage, Int<first>): run
+// after a step's stage has landed and before it is read.
 template <int BM, int BN, int WM, int WN, int D, class F>
 __device__ __attribute__((always_inline)) inline void tile_loop(lds_u8_t* lds, const uint8_t* __restrict__ xk,
                                                                 int64_t ldx, int tmax, const uint8_t* __restrict__ wk,
-                                                                int64_t ldw, int nmax, int nk, int rot,
+                                                                int64_t ldw, int nmax, int nk,
                                                                 f32x16_t (&acc)[WM / 32][WN / 32], F&& landed) {
   using L = Tile<BM, BN, WM, WN, D>;
   constexpr int NM = L::MB * L::NB, NR = L::MB + L::NB, RPM = (NR + NM - 1) / NM;
@@ -81,8 +83,7 @@ __device__ __attribute__((always_inline)) inline void tile_loop(lds_u8_t* lds, c
   }
   auto copy = [&](int ks, int i) __attribute__((always_inline)) {
     const int q = wave * L::CP + i;
-    const int k = ks + rot < nk ? ks + rot : ks + rot - nk;
-    dma16_s((q < BM / 8 ? xk : wk) + (int64_t)k * kRow, off[i], lds_base + (ks % D) * L::STAGE + q * 1024);
+    dma16_s((q < BM / 8 ? xk : wk) + (int64_t)ks * kRow, off[i], lds_base + (ks % D) * L::STAGE + q * 1024);
   };
   // fragments: row r, chunk 2 kk + lane / 32 at slot chunk ^ ((r / 2) mod 8); the blocks of 32 rows
   // share the swizzle

@@ -249,6 +249,23 @@ def test_o_proj_fused_rope_wide(dev, T):
     np.testing.assert_allclose(fused.cpu()[idx].double().numpy(), ref, rtol=1e-2, atol=2e-2 * np.abs(ref).max())
 
 
+@pytest.mark.parametrize("T", [520, 2048])
+def test_o_proj_token_anywhere(dev, T):
+    """One token's output has the same bits wherever it stands in a prompt (rows of o 64 KB apart, tiles
+    of 128 x 128 and 256 x 256): every output is one accumulation chain in k order."""
+    from smla import norm_rope as snr
+    from smla import ops
+    announce(f"o_proj T={T}, one token repeated")
+    g = torch.Generator(device=dev).manual_seed(T)
+    o = torch.randn(1, 64, 512, generator=g, device=dev).to(torch.bfloat16).expand(T, -1, -1).contiguous()
+    wa = (torch.randn(8192, 4096, generator=g, device=dev) * 0.02).to(torch.bfloat16)
+    wb = (torch.randn(4096, 8192, generator=g, device=dev) * 0.02).to(torch.bfloat16)
+    cos_t, sin_t = snr.rope_tables(64, 4096, device=dev)
+    pos = torch.full((T,), 1234, dtype=torch.int32, device=dev)
+    y = ops.o_proj_op(o, pos, cos_t, sin_t, wa, wb, 8, torch.float32)
+    assert torch.equal(y, y[:1].expand(T, -1))
+
+
 @pytest.mark.parametrize("T", [40, 300])
 @pytest.mark.parametrize("H,D,G", [(8, 64, 1), (12, 192, 2), (4, 320, 2)])
 def test_o_proj_fused_rope_head_dims(dev, T, H, D, G):
