@@ -478,7 +478,11 @@ __global__ __launch_bounds__(512) void gemm_heads_kernel(const RingArgs p, int64
                                               [](int, lds_u8_t*, auto) {});
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = wave % 2, wn = wave / 2;
   // sums of squares: a row's 512 values sit in the 32 lanes of a half wave of four waves; the waves' sums
-  // and then the rows' factors go through LDS past the region the stores use
+  // and then the rows' factors go through LDS past the region the stores use.  The epilogue is
+  // row_epilogue_kernel's to the bit, so that a prompt's rows do not depend on its length: a thread there
+  // holds channels 2t and 2t + 1 and a wave the 128 channels of a wave here, so pairs are summed first,
+  // then threads 32, 16 (blocks of 32 channels), 8, 4, 2, 1 apart (16, 8, 4, 2 lanes here; row_ror:8 and :4
+  // where the values repeat every 8 lanes), then the waves in order
   smla_attn::lds_f32_t* ss = (smla_attn::lds_f32_t*)(lds + 8 * F::WM * F::WN * 2);  // [4][128], then [128]
   static_assert(8 * F::WM * F::WN * 2 + 5 * 128 * 4 <= L::LDS, "the sums fit behind the staged rows");
   // the tile's rotations (128 rows of 32 cos and 32 sin) come in beside the sums, two 16-byte pieces of
@@ -497,15 +501,18 @@ __global__ __launch_bounds__(512) void gemm_heads_kernel(const RingArgs p, int64
   for (int mb = 0; mb < L::MB; mb++)
 #pragma unroll
     for (int r = 0; r < 16; r++) {
-      float q = 0.f;
+      float pr[4];
 #pragma unroll
-      for (int nb = 0; nb < L::NB; nb++) q = __builtin_fmaf(acc[mb][nb][r], acc[mb][nb][r], q);
-      q += dpp_f<0xB1>(q);
-      q += dpp_f<0x4E>(q);
-      q += dpp_f<0x141>(q);
-      q += dpp_f<0x140>(q);
+      for (int nb = 0; nb < L::NB; nb++) {
+        const float v0 = dpp_f<0xA0>(acc[mb][nb][r]), v1 = dpp_f<0xF5>(acc[mb][nb][r]);
+        pr[nb] = __builtin_fmaf(v0, v0, mul_rn_g(v1, v1));
+      }
+      float q = (pr[0] + pr[2]) + (pr[1] + pr[3]);
       const auto h = __builtin_amdgcn_permlane16_swap(__float_as_uint(q), __float_as_uint(q), false, false);
       q = __uint_as_float(h[0]) + __uint_as_float(h[1]);
+      q += dpp_f<0x128>(q);
+      q += dpp_f<0x124>(q);
+      q += dpp_f<0x4E>(q);
       if ((lane & 31) == 0) ss[128 * wn + 64 * wm + 32 * mb + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)] = q;
     }
   smla_attn::lds_f32x4_t* cs = (smla_attn::lds_f32x4_t*)lds;  // cos then sin, [128][32]
@@ -517,7 +524,7 @@ __global__ __launch_bounds__(512) void gemm_heads_kernel(const RingArgs p, int64
   lds_barrier();
   if (threadIdx.x < 128) {
     const int i = threadIdx.x;
-    ss[512 + i] = rsqrtf(((ss[i] + ss[128 + i]) + (ss[256 + i] + ss[384 + i])) / 512.f + eps);
+    ss[512 + i] = rsqrtf((((ss[i] + ss[128 + i]) + ss[256 + i]) + ss[384 + i]) / 512.f + eps);
   }
   lds_barrier();
 #pragma unroll
@@ -535,8 +542,9 @@ __global__ __launch_bounds__(512) void gemm_heads_kernel(const RingArgs p, int64
 #pragma unroll
           for (int nb = 2; nb < 4; nb++) {
             const int i = 16 * (nb - 2) + ((lane & 31) >> 1);
-            const float v = acc[mb][nb][4 * q4 + j], u = dpp_f<0xB1>(v), c = cr[i], s = cr[4096 + i];
-            acc[mb][nb][4 * q4 + j] = v * c + u * (lane & 1 ? s : -s);
+            const float v = acc[mb][nb][4 * q4 + j], c = cr[i], s = cr[4096 + i];
+            const float y0 = dpp_f<0xA0>(v), y1 = dpp_f<0xF5>(v);  // y0 c - y1 s, y0 s + y1 c
+            acc[mb][nb][4 * q4 + j] = __builtin_fmaf(y0, lane & 1 ? s : c, mul_rn_g(y1, lane & 1 ? c : -s));
           }
         }
       }

@@ -632,7 +632,7 @@ struct PromptRows {
 
 __global__ __launch_bounds__(256) void prompt_rows_kernel(const PromptRows p) {
   constexpr int d = 512, rd = 64, ratio = 4;
-  __shared__ float red[4];
+  __shared__ float red[8];
   __shared__ float xch[512];
   const int t = threadIdx.x;
   int64_t i = blockIdx.x;
@@ -661,7 +661,9 @@ __global__ __launch_bounds__(256) void prompt_rows_kernel(const PromptRows p) {
   }
   i -= rows;
   if (i < rows) {
-    // 4 channels per thread and round: dq <= 1024
+    // 4 channels per thread: dq <= 1024.  The sum is row_epilogue_kernel's to the bit: a thread here is two
+    // threads there and half a wave here a wave there, so threads 16, 8 .. 1 apart first, then the
+    // thread's two pairs, then the half waves in order
     const float* x = p.qa + i * p.ld;
     const int c = 4 * t;
     f32x2_t a = {0.f, 0.f}, q = {0.f, 0.f};
@@ -669,7 +671,17 @@ __global__ __launch_bounds__(256) void prompt_rows_kernel(const PromptRows p) {
       a = *(const f32x2_t*)(x + c);
       q = *(const f32x2_t*)(x + c + 2);
     }
-    const float ss = block_sum(a[0] * a[0] + a[1] * a[1] + q[0] * q[0] + q[1] * q[1], red);
+    float s0 = a[0] * a[0] + a[1] * a[1], s1 = q[0] * q[0] + q[1] * q[1];
+#pragma unroll
+    for (int o = 16; o >= 1; o >>= 1) {
+      s0 += __shfl_xor(s0, o, 64);
+      s1 += __shfl_xor(s1, o, 64);
+    }
+    if ((t & 31) == 0) red[t >> 5] = s0 + s1;
+    __syncthreads();
+    float ss = 0.f;
+#pragma unroll
+    for (int h = 0; h < 8; h++) ss += red[h];
     const float inv = rsqrtf(ss / (float)p.dq + p.eps);
     if (c < p.dq) {
       const f32x4_t w = *(const f32x4_t*)(p.qa_norm + c);

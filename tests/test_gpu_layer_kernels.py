@@ -205,6 +205,45 @@ def test_q_up(dev, T, heads, K):
     assert bool(((out.double() - ref).abs() <= tol).all())
 
 
+@pytest.mark.parametrize("T,heads,K", [(1, 64, 128), (130, 3, 1024), (300, 64, 192)])
+def test_q_up_is_the_two_launches(dev, T, heads, K):
+    """smla_q_up equals smla_linear with an fp32 result followed by smla_row_epilogue bit for bit (a prompt's
+    rows do not depend on which of the two its length takes), and smla_prompt_rows' q_a norm equals
+    smla_row_epilogue's."""
+    from smla import _lib, ops
+    from smla import norm_rope as snr
+    announce(f"q_up against two launches T={T} heads={heads} K={K}")
+    g = torch.Generator(device=dev).manual_seed(T + K)
+    x = torch.randn(T, K, generator=g, device=dev).to(torch.bfloat16)
+    w = (torch.randn(heads * 512, K, generator=g, device=dev) * 0.05).to(torch.bfloat16)
+    pos = torch.randint(0, 4096, (T,), generator=g, device=dev, dtype=torch.int32)
+    cos_t, sin_t = snr.rope_tables(64, 4096, device=dev)
+    out, ref = (torch.empty(T, heads, 512, dtype=torch.bfloat16, device=dev) for _ in range(2))
+    ops.q_up(x, w, pos, cos_t, sin_t, out)
+    xr = x.repeat(1 if T > 32 else 40, 1)     # beyond the weight-streaming kernels, without workspace: one chain over K
+    y = torch.empty(xr.shape[0], heads * 512, device=dev)
+    _lib.call("smla_linear", xr.data_ptr(), _lib.BF16, w.data_ptr(), _lib.BF16, xr.shape[0], 1, heads * 512, K,
+              y.data_ptr(), _lib.F32, torch.cuda.current_stream().cuda_stream)
+    ops.row_epilogue(y[:T].view(T * heads, 512), None, pos, cos_t, sin_t, 64, _lib.SIM_NONE, ref, rows_per_pos=heads)
+    assert torch.equal(out, ref)
+
+
+@pytest.mark.parametrize("dq", [256, 1024])
+def test_prompt_rows_q_a_norm(dev, dq):
+    from smla import _lib, ops
+    from smla import norm_rope as snr
+    announce(f"prompt_rows q_a norm dq={dq}")
+    g = torch.Generator(device=dev).manual_seed(dq)
+    y = torch.randn(70, dq + 512, generator=g, device=dev)
+    qa_norm, kv_norm = 1 + 0.1 * torch.randn(dq, generator=g, device=dev), torch.ones(512, device=dev)
+    cos_t, sin_t = snr.rope_tables(64, 128, device=dev)
+    raw = torch.zeros(1, 128, 512, dtype=torch.bfloat16, device=dev)
+    qa, _, _ = ops.prompt_rows(y, [0, dq, dq + 512], 1, 70, qa_norm, kv_norm, cos_t, sin_t, raw)
+    ref = torch.empty_like(qa)
+    ops.row_epilogue(y[:, :dq], qa_norm, None, None, None, 0, _lib.SIM_NONE, ref)
+    assert torch.equal(qa, ref)
+
+
 @pytest.mark.parametrize("B,S,with_ring", [(1, 3, True), (2, 130, True), (2, 141, False), (3, 128, True)])
 def test_prompt_rows(dev, B, S, with_ring):
     """smla_prompt_rows equals the separate calls: row epilogues of the kv rows, the gated pool, the
