@@ -5,15 +5,22 @@
 // is left: exact while the lowest bit of x is a bf16 (|x| >= 2^-110; below, bits under 2^-133 are lost).
 // x w = hh + (hm + mh) + (hl + lh + mm) up to terms of 2^-23 |x w| on average: the products of bf16
 // values are exact in fp32 and v_mfma_f32_32x32x16_bf16 adds 16 k of one of them per accumulator
-// rounding, against one rounding per k (or two) of a chain of fp32 fmas.  Distance from float64
-// (relative, 2-norm; uniform operands): 1.0e-6 for K = 4096 and 4.9e-7 for K = 1024 in one chain, 6.4e-7
-// and 3.5e-7 in two splits; the fp32 MFMAs 1.1e-6 and 5.9e-7.  An operand that the split cannot carry
-// (infinite or NaN) makes the sum non-finite, and every non-finite sum is recomputed as an fp32 fma
-// chain (nonfinite_fix), so infinities and NaN come out as fp32 arithmetic gives them.
+// rounding, against one rounding per k (or two) of a chain of fp32 fmas.  hh has an accumulator, the five
+// small products share another, added once at the end: in one accumulator the 2^-16 of hl, lh and mm fall
+// below half its last place once it holds some thousand products, always with the same sign (1.05e-5 for
+// K = 4096 and operands of one sign).  Distance from float64 (relative, 2-norm), here / one chain of fp32
+// MFMAs:
+//   K             64                1024              4096              8192
+//   uniform 0..1  0.6 / 1.2e-7      0.8 / 4.3e-7      3.0 / 8.4e-7      4.2e-7 / 1.2e-6
+//   normal        0.8 / 1.4e-7      1.2 / 5.7e-7      4.0e-7 / 1.2e-6   5.7e-7 / 1.6e-6
+// An operand that the split cannot carry (infinite or NaN) makes the sum non-finite, and every
+// non-finite sum is recomputed as an fp32 fma chain (nonfinite_fix), so infinities and NaN come out as
+// fp32 arithmetic gives them.  The three-way split is that of G. Henry, P. Tang and A. Heinecke,
+// "Leveraging the bfloat16 artificial intelligence datatype for higher-precision computations" (2019).
 //
 // Six bf16 MFMAs carry 16 k in 192 cycles per 32 x 32 block where the fp32 MFMAs take 512.  [2046, 4096] x
-// [2048, 4096]^T: 394 us with fp32 MFMAs and register staging, 184 us here (186 TFLOP/s; the fp32 MFMA
-// peak is 157); [1, 8192] x [4096, 8192]^T 710 -> 43 us.
+// [2048, 4096]^T: 394 us with fp32 MFMAs and register staging, 188 us here (183 TFLOP/s; the fp32 MFMA
+// peak is 157; 184 us with one accumulator); [1, 8192] x [4096, 8192]^T 694 -> 45 us.
 //
 // What bounds it is the vector ALU work of the splits (11 instructions per pair of values, done by
 // every wave that reads them) beside the MFMAs: either takes about 55 % of the cycles, and they
@@ -100,8 +107,9 @@ __device__ __attribute__((always_inline)) inline void tile_loop_f32(lds_u8_t* ld
 #pragma unroll
     for (int i = 0; i < NR; i++) sp[kk][i] = split3(raw[kk][i][0], raw[kk][i][1]);
   };
-  // the MFMAs of sub-step kk, small products first, the blocks alternating so that an accumulator
-  // is not wanted again at once
+  // the MFMAs of sub-step kk: hh into acc, the others into low; the blocks alternate so that an
+  // accumulator is not wanted again at once
+  f32x16_t low[MB][NB];
   auto mul = [&](auto kk_) __attribute__((always_inline)) {
     constexpr int kk = decltype(kk_)::value;
 #pragma unroll
@@ -111,7 +119,8 @@ __device__ __attribute__((always_inline)) inline void tile_loop_f32(lds_u8_t* ld
         const Split3 &a = sp[kk][j / NB], &b = sp[kk][MB + j % NB];
         const bf16x8_t u = p == 0 ? a.m : p == 1 ? a.l : p == 3 ? a.m : a.h;
         const bf16x8_t v = p == 0 ? b.m : p == 2 ? b.l : p == 4 ? b.m : b.h;
-        acc[j / NB][j % NB] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(u, v, acc[j / NB][j % NB], 0, 0, 0);
+        f32x16_t& c = p == 5 ? acc[j / NB][j % NB] : low[j / NB][j % NB];
+        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(u, v, c, 0, 0, 0);
       }
   };
   auto pin = [&]() __attribute__((always_inline)) {
@@ -127,7 +136,7 @@ __device__ __attribute__((always_inline)) inline void tile_loop_f32(lds_u8_t* ld
 #pragma unroll
     for (int n = 0; n < NB; n++)
 #pragma unroll
-      for (int r = 0; r < 16; r++) acc[m][n][r] = 0.f;
+      for (int r = 0; r < 16; r++) acc[m][n][r] = low[m][n][r] = 0.f;
 #pragma unroll
   for (int s = 0; s < D; s++) copy(s);
   wait_vm((D - 1) * L::CP);
@@ -155,6 +164,10 @@ __device__ __attribute__((always_inline)) inline void tile_loop_f32(lds_u8_t* ld
   for (; ks < nk - D; ks++) step(ks, Int<1>{}, Int<1>{});
   for (; ks < nk - 1; ks++) step(ks, Int<0>{}, Int<1>{});
   step(ks, Int<0>{}, Int<0>{});
+#pragma unroll
+  for (int m = 0; m < MB; m++)
+#pragma unroll
+    for (int n = 0; n < NB; n++) acc[m][n] += low[m][n];
 }
 
 }  // namespace smla_gemm

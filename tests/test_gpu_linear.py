@@ -136,6 +136,24 @@ def test_linear_fp32_tiles(dev, T, G, N, K, out_dtype):
     _check_linear(y.float(), x, w, G, out_dtype)
 
 
+@pytest.mark.parametrize("T,N,K", [(64, 1024, 64), (300, 1024, 1024), (2046, 2048, 4096), (1024, 4096, 8192)])
+@pytest.mark.parametrize("sign", [1.0, -1.0])
+def test_linear_fp32_one_sign(dev, T, N, K, sign):
+    """Sums of one sign, where a term that falls below the accumulator's last place is lost every time and
+    not only now and then.  K / 16 roundings of partial sums that grow evenly, each off by at most
+    2^-24 of its partial sum, are 2^-24 sqrt(K / 48) of the result together (2-norm); the last addition
+    and the terms that three bf16 parts leave out are 2^-24 each.  All of it is noise: the mean is at most
+    the last two."""
+    from smla import ops
+    announce(f"linear fp32 one sign T={T} N={N} K={K}")
+    g = torch.Generator(device=dev).manual_seed(T + K)
+    x, w = torch.rand(T, K, generator=g, device=dev), torch.rand(N, K, generator=g, device=dev) * sign
+    ref = x.double() @ w.double().t()
+    err = (ops.linear_op(x, w, 1, torch.float32).double() - ref) / ref
+    assert err.square().mean().sqrt().item() <= 2.0 ** -24 * ((K / 48) ** 0.5 + 2)
+    assert abs(err.mean().item()) <= 2.0 ** -23
+
+
 @pytest.mark.parametrize("T,N,K", [(40, 130, 4096), (300, 600, 96)])    # with and without splits
 def test_linear_fp32_special_values(dev, T, N, K):
     """Infinities, NaN, values whose bf16 rounding overflows and subnormals come out as fp32 arithmetic
