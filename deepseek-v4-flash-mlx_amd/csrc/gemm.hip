@@ -426,9 +426,8 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const RingArgs p) {
   tile_loop_f32<BM, BN, WM, WN, D>((lds_u8_t*)lds_g, xk, p.ldx, p.T - 1 - t0, wk, (int64_t)p.K * 4, p.N - 1 - n0, k1 - k0,
                                    acc);
   store_tile<F, YDT>((lds_u8_t*)lds_g, p, id.sp, id.g, t0, n0, acc);
-  // nonfinite_fix: a sum that is infinite or NaN may be so only because an operand has no split; it
-  // is computed again as a chain of fp32 fmas (ended by the first NaN, which stays) and stored again,
-  // behind the first store
+  // a sum that is infinite or NaN may be so only because an operand has no split: it is taken from the
+  // fp32 MFMAs, a wave's block of 32 x 32 at a time, and stored again behind the first store
   uint64_t bad = 0;
 #pragma unroll
   for (int i = 0; i < L::MB * L::NB * 16; i++)
@@ -436,19 +435,20 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const RingArgs p) {
   if (__any(bad != 0)) {
     wait_vm(0);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = wave % (BM / WM), wn = wave / (BM / WM);
-    while (bad) {
-      const int i = __builtin_ctzll(bad), blk = i / 16, r = i % 16;
-      bad &= bad - 1;
-      const int t = WM * wm + 32 * (blk / L::NB) + 4 * (lane >> 5) + 8 * (r >> 2) + (r & 3);
-      const int n = WN * wn + 32 * (blk % L::NB) + (lane & 31);
-      if (t0 + t >= p.T || n0 + n >= p.N) continue;
-      const float* xr = (const float*)(xk + (int64_t)t * p.ldx);
-      const float* wr = (const float*)wk + (int64_t)n * p.K;
-      float sum = 0.f;
-      for (int k = 0; k < (k1 - k0) * 32 && sum == sum; k++) sum = __builtin_fmaf(xr[k], wr[k], sum);
-      const int64_t o = id.sp * p.split_stride + (int64_t)id.g * p.N + (int64_t)(t0 + t) * p.ldy + n0 + n;
-      if constexpr (YDT == SMLA_BF16) ((uint16_t*)p.y)[o] = bf16_rne(sum);
-      else ((float*)p.y)[o] = sum;
+#pragma unroll 1
+    for (int blk = 0; blk < L::MB * L::NB; blk++, bad >>= 16) {
+      if (!__any((bad & 0xffffu) != 0)) continue;
+      const f32x16_t f = block_f32<BM, BN, WM, WN>(xk, p.ldx, p.T - 1 - t0, wk, (int64_t)p.K * 4, p.N - 1 - n0, k1 - k0,
+                                                   blk / L::NB, blk % L::NB);
+      const int t = t0 + WM * wm + 32 * (blk / L::NB) + 4 * (lane >> 5), n = n0 + WN * wn + 32 * (blk % L::NB) + (lane & 31);
+      const int64_t o = id.sp * p.split_stride + (int64_t)id.g * p.N + n;
+#pragma unroll
+      for (int r = 0; r < 16; r++) {
+        const int tr = t + 8 * (r >> 2) + (r & 3);
+        if (!(bad >> r & 1) || tr >= p.T || n >= p.N) continue;
+        if constexpr (YDT == SMLA_BF16) ((uint16_t*)p.y)[o + (int64_t)tr * p.ldy] = bf16_rne(f[r]);
+        else ((float*)p.y)[o + (int64_t)tr * p.ldy] = f[r];
+      }
     }
   }
 }

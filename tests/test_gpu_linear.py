@@ -180,6 +180,32 @@ def test_linear_fp32_special_values(dev, T, N, K):
     assert bool(((y.double() - ref).abs()[ok] <= tol[ok]).all())
 
 
+@pytest.mark.parametrize("T,N,K", [(300, 600, 8192), (1024, 2048, 4096)])
+def test_linear_fp32_infinity_costs_no_cliff(dev, T, N, K):
+    """One infinite weight makes a column of the result non-finite, which the fp32 MFMAs compute again block
+    by block: that work is at most the product's own at a third of its rate (8 times with its start and
+    its loads' latency), not a serial chain per output (40 times and more)."""
+    from smla import ops
+    announce(f"linear fp32 with an infinity T={T} N={N} K={K}")
+    g = torch.Generator(device=dev).manual_seed(T)
+    x, w = torch.randn(T, K, generator=g, device=dev), torch.randn(N, K, generator=g, device=dev)
+    bad = w.clone()
+    bad[5, 0] = float("inf")
+
+    def us(weight):
+        ev = [torch.cuda.Event(enable_timing=True) for _ in range(6)]
+        ops.linear_op(x, weight, 1, torch.float32)
+        for e in ev:
+            e.record()
+            ops.linear_op(x, weight, 1, torch.float32)
+        torch.cuda.synchronize()
+        return min(a.elapsed_time(b) for a, b in zip(ev, ev[1:]))
+
+    y = ops.linear_op(x, bad, 1, torch.float32)
+    assert bool(torch.isinf(y[:, 5]).all()) and bool(torch.isfinite(y[:, :5]).all())
+    assert us(bad) <= 8 * us(w)
+
+
 @pytest.mark.parametrize("T,G,N,K", [(9, 1, 64, 4096), (17, 2, 48, 4096), (32, 1, 512, 4096), (100, 1, 1024, 4096)])
 def test_linear_without_workspace(dev, T, G, N, K):
     """smla_linear (no workspace): 9 to 32 rows whose GEMM would split K run the weight-streaming
