@@ -426,8 +426,8 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const RingArgs p) {
   tile_loop_f32<BM, BN, WM, WN, D>((lds_u8_t*)lds_g, xk, p.ldx, p.T - 1 - t0, wk, (int64_t)p.K * 4, p.N - 1 - n0, k1 - k0,
                                    acc);
   store_tile<F, YDT>((lds_u8_t*)lds_g, p, id.sp, id.g, t0, n0, acc);
-  // a sum that is infinite or NaN may be so only because an operand has no split: it is taken from the
-  // fp32 MFMAs, a wave's block of 32 x 32 at a time, and stored again behind the first store
+  // a sum that is infinite or NaN may be so only because an operand has no split, and every sum of a wave
+  // that met a value below 2^-110 may have lost some of it: they are taken from the fp32 MFMAs, a wave's block of 32 x 32 at a time, and stored again behind the first store
   uint64_t bad = 0;
 #pragma unroll
   for (int i = 0; i < L::MB * L::NB * 16; i++)

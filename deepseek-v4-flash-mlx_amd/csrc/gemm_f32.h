@@ -1,32 +1,33 @@
 // The K loop of the tiled fp32 product (gemm.hip): one workgroup's BM x BN tile of x . w^T, both
 // operands K-contiguous fp32, on the bf16 matrix cores.
 //
-// An fp32 value is the sum of three bf16 values, x = h + m + l, each the top 8 significant bits of what
-// is left: exact while the lowest bit of x is a bf16 (|x| >= 2^-110; below, bits under 2^-133 are lost).
-// x w = hh + (hm + mh) + (hl + lh + mm) up to terms of 2^-23 |x w| on average: the products of bf16
-// values are exact in fp32 and v_mfma_f32_32x32x16_bf16 adds 16 k of one of them per accumulator
-// rounding, against one rounding per k (or two) of a chain of fp32 fmas.  hh has an accumulator, the five
-// small products share another, added once at the end: in one accumulator the 2^-16 of hl, lh and mm fall
-// below half its last place once it holds some thousand products, always with the same sign (1.05e-5 for
-// K = 4096 and operands of one sign).  Distance from float64 (relative, 2-norm), here / one chain of fp32
-// MFMAs:
+// An fp32 value, times 2^16, is the sum of three bf16 values, 2^16 x = h + m + l, each the nearest bf16 to
+// what is left: exact for every x below 2^112 (the lowest bit of a subnormal, 2^-149, becomes a
+// subnormal bf16's, 2^-133; without the factor a value below 2^-110 lost bits).  x w = hh + (hm + mh) +
+// (hl + lh + mm) up to 2^-24 |x w|, of either sign: the products of bf16 values are exact in fp32 and
+// v_mfma_f32_32x32x16_bf16 adds 16 k of one of them per accumulator rounding, against one rounding per k
+// (or two) of a chain of fp32 fmas.  hh has an accumulator, the five small products share another, added
+// once at the end: in one accumulator the 2^-16 of hl, lh and mm fall below half its last place once it
+// holds some thousand products, always with the same sign (1.05e-5 for K = 4096 and operands of one
+// sign).  Distance from float64 (relative, 2-norm), here / one chain of fp32 MFMAs:
 //   K             64                1024              4096              8192
-//   uniform 0..1  0.6 / 1.2e-7      0.8 / 4.3e-7      3.0 / 8.4e-7      4.2e-7 / 1.2e-6
-//   normal        0.8 / 1.4e-7      1.2 / 5.7e-7      4.0e-7 / 1.2e-6   5.7e-7 / 1.6e-6
-// An operand that the split cannot carry (infinite or NaN) makes the sum non-finite, and every
-// non-finite sum is taken from the fp32 MFMAs instead (block_f32), so infinities and NaN come out as
-// fp32 arithmetic gives them.  The three-way split is that of G. Henry, P. Tang and A. Heinecke,
-// "Leveraging the bfloat16 artificial intelligence datatype for higher-precision computations" (2019).
+//   uniform 0..1  0.5 / 1.2e-7      0.7 / 4.3e-7      3.0 / 8.4e-7      4.2e-7 / 1.2e-6
+//   normal        0.5 / 1.4e-7      1.1 / 5.7e-7      4.0e-7 / 1.2e-6   5.7e-7 / 1.6e-6
+// An operand that the split cannot carry (infinite, NaN, from 2^112) or a sum from 2^96 is non-finite
+// here, and every non-finite sum is taken from the fp32 MFMAs instead (block_f32), so infinities and
+// NaN come out as fp32 arithmetic gives them.  The three-way split is that of G. Henry, P. Tang and
+// A. Heinecke, "Leveraging the bfloat16 artificial intelligence datatype for higher-precision
+// computations" (2019).
 //
 // Six bf16 MFMAs carry 16 k in 192 cycles per 32 x 32 block where the fp32 MFMAs take 512.  [2046, 4096] x
-// [2048, 4096]^T: 394 us with fp32 MFMAs and register staging, 188 us here (183 TFLOP/s; the fp32 MFMA
-// peak is 157; 184 us with one accumulator); [1, 8192] x [4096, 8192]^T 694 -> 45 us.
+// [2048, 4096]^T: 382 us with fp32 MFMAs and register staging, 197 us here (174 TFLOP/s; the fp32 MFMA
+// peak is 157); [1, 8192] x [4096, 8192]^T 694 -> 50 us.
 //
-// What bounds it is the vector ALU work of the splits (11 instructions per pair of values, done by
-// every wave that reads them) beside the MFMAs: either takes about 55 % of the cycles, and they
-// overlap only in part (rounding the parts instead of truncating them, 1.5 times the MFMAs per split,
-// two waves per SIMD: all within 4 % of the same time).  The splits of the next 16 k are therefore interleaved with the MFMAs of the current ones, and
-// the raw values of the 16 k after those are read from LDS meanwhile (two register sets of each).
+// What bounds it is the vector ALU work of the splits (13 instructions per pair of values, done by
+// every wave that reads them) beside the MFMAs: either takes more than half of the cycles, and they
+// overlap only in part (without the factor 2^16, 11 instructions: 184 us).  The splits of the next 16 k
+// are therefore interleaved with the MFMAs of the current ones, and the raw values of the 16 k after
+// those are read from LDS meanwhile (two register sets of each).
 #pragma once
 
 #include "gemm_tile.h"
@@ -37,22 +38,23 @@ struct Split3 {
   bf16x8_t h, m, l;
 };
 
-// the high halves of a (low word) and b (high word): both truncated to bf16
+// the high halves of a (low word) and b (high word)
 __device__ inline uint32_t top_halves(float a, float b) {
   return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
 }
-__device__ inline float below_top(float a) { return a - __uint_as_float(__float_as_uint(a) & 0xffff0000u); }
 
+// the parts of 2^16 x: its lowest bit is a bf16 (2^-149 of a subnormal comes to 2^-133)
 __device__ inline Split3 split3(u32x4_t lo, u32x4_t hi) {
   u32x4_t h, m, l;
 #pragma unroll
   for (int j = 0; j < 4; j++) {
-    const float a = __uint_as_float(j < 2 ? lo[2 * j] : hi[2 * j - 4]);
-    const float b = __uint_as_float(j < 2 ? lo[2 * j + 1] : hi[2 * j - 3]);
-    const float a1 = below_top(a), b1 = below_top(b);
-    h[j] = top_halves(a, b);
-    m[j] = top_halves(a1, b1);
-    l[j] = top_halves(below_top(a1), below_top(b1));
+    const float a = __uint_as_float(j < 2 ? lo[2 * j] : hi[2 * j - 4]) * 0x1p16f;
+    const float b = __uint_as_float(j < 2 ? lo[2 * j + 1] : hi[2 * j - 3]) * 0x1p16f;
+    h[j] = pack_bf16x2(a, b);
+    const float a1 = a - __uint_as_float(h[j] << 16), b1 = b - __uint_as_float(h[j] & 0xffff0000u);
+    m[j] = pack_bf16x2(a1, b1);
+    const float a2 = a1 - __uint_as_float(m[j] << 16), b2 = b1 - __uint_as_float(m[j] & 0xffff0000u);
+    l[j] = top_halves(a2, b2);
   }
   return {as_bf16x8(h), as_bf16x8(m), as_bf16x8(l)};
 }
@@ -123,8 +125,10 @@ __device__ __attribute__((always_inline)) inline void tile_loop_f32(lds_u8_t* ld
         c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(u, v, c, 0, 0, 0);
       }
   };
+  // 13 vector instructions per pair of values of the four, and some of the addresses' (with room for just
+  // 52 the compiler takes 284 registers instead of 244, which is one wave per SIMD: 240 us instead of 197)
   auto pin = [&]() __attribute__((always_inline)) {
-    constexpr int V = (NR * 44 + 6 * MB * NB - 1) / (6 * MB * NB);
+    constexpr int V = (NR * 56 + 6 * MB * NB - 1) / (6 * MB * NB);
 #pragma unroll
     for (int j = 0; j < 6 * MB * NB; j++) {
       __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);  // MFMA
@@ -167,7 +171,7 @@ __device__ __attribute__((always_inline)) inline void tile_loop_f32(lds_u8_t* ld
 #pragma unroll
   for (int m = 0; m < MB; m++)
 #pragma unroll
-    for (int n = 0; n < NB; n++) acc[m][n] += low[m][n];
+    for (int n = 0; n < NB; n++) acc[m][n] = (acc[m][n] + low[m][n]) * 0x1p-32f;
 }
 
 // Block (mb, nb) of this wave's part of the tile by fp32 MFMAs, operands from memory; arguments and layout

@@ -157,8 +157,8 @@ def test_linear_fp32_one_sign(dev, T, N, K, sign):
 @pytest.mark.parametrize("T,N,K", [(40, 130, 4096), (300, 600, 96)])    # with and without splits
 def test_linear_fp32_special_values(dev, T, N, K):
     """Infinities, NaN, values whose bf16 rounding overflows and subnormals come out as fp32 arithmetic
-    gives them: the same places infinite and NaN, the rest within the fp32 bound plus what the split
-    leaves of an operand below 2^-110, at most 2^-133 (the last bit of a subnormal bf16)."""
+    gives them: the same places infinite and NaN, the rest within the fp32 bound and the rounding of a
+    subnormal result."""
     from smla import ops
     announce(f"linear fp32 special values T={T} N={N} K={K}")
     g = torch.Generator().manual_seed(T)
@@ -175,9 +175,37 @@ def test_linear_fp32_special_values(dev, T, N, K):
     assert torch.equal(torch.isinf(y), inf) and torch.equal(y[inf].double(), ref[inf])
     ok = torch.isfinite(ref)
     xf, wf = torch.nan_to_num(x.double(), 0, 0, 0), torch.nan_to_num(w.double(), 0, 0, 0)
-    tol = (K + 8) * 2.0 ** -23 * (xf.abs() @ wf.abs().t()) \
-        + 2.0 ** -133 * (xf.abs().sum(1)[:, None] + wf.abs().sum(1)[None]) + K * 2.0 ** -149
+    tol = (K + 8) * 2.0 ** -23 * (xf.abs() @ wf.abs().t()) + K * 2.0 ** -149
     assert bool(((y.double() - ref).abs()[ok] <= tol[ok]).all())
+
+
+@pytest.mark.parametrize("N,K", [(130, 4096), (1030, 96)])       # 64 x 64 tiles with splits, 128 x 128
+def test_linear_fp32_every_magnitude(dev, N, K):
+    """Rows of every binary magnitude an fp32 operand can have, the smallest subnormal to the largest that
+    leaves the sums finite: the fp32 bound throughout, plus what a result below 2^-126 is rounded by."""
+    from smla import ops
+    announce(f"linear fp32 magnitudes N={N} K={K}")
+    g = torch.Generator().manual_seed(K)
+    e = torch.arange(-149, 119).double()
+    x = (torch.randn(e.numel(), K, generator=g).double() * torch.exp2(e)[:, None]).float()
+    w = torch.randn(N, K, generator=g) * 0.05
+    for a, b in ((x, w), (w, x)):
+        y = ops.linear_op(a.to(dev), b.to(dev), 1, torch.float32).cpu().double()
+        ref, mag = a.double() @ b.double().t(), a.double().abs() @ b.double().abs().t()
+        assert bool(((y - ref).abs() <= (K + 8) * 2.0 ** -23 * mag + 16 * 2.0 ** -150).all())
+
+
+def test_linear_fp32_single_products(dev):
+    """Sums of one term: the split leaves out at most 2^-24 of a product and one addition rounds."""
+    from smla import ops
+    announce("linear fp32 single products")
+    g = torch.Generator(device=dev).manual_seed(8)
+    K = 1024
+    x = torch.diag(1.0 + torch.rand(K, generator=g, device=dev))
+    w = 1.0 + torch.rand(2048, K, generator=g, device=dev)
+    y = ops.linear_op(x, w, 1, torch.float32).double()
+    ref = x.diagonal().double()[:, None] * w.double().t()
+    assert ((y - ref).abs() / ref).max().item() <= 2.0 ** -23
 
 
 @pytest.mark.parametrize("T,N,K", [(300, 600, 8192), (1024, 2048, 4096)])
