@@ -58,15 +58,14 @@ def compressor_prefill(x, wkv, wgate, ape, norm_w, head_dim=512, ratio=4, rope_h
 
 def project_pair(x, wkv, wgate):
     """(x @ wkv^T, x @ wgate^T) as fp32 [b, s, 2*head_dim] each, from one launch: fp32 operands unless
-    x and both weights are bf16.  The two weights are read where they are when they match (shape,
-    dtype, alignment) and the tiled GEMM takes them; else they are stacked first."""
+    x and both weights are bf16.  Weights of one shape and that dtype go to ``linear_pair``, which reads
+    them where they are when it can; others are converted and stacked here.  Shapes and dtypes only: it
+    is traced and exported, and tensors without memory have no alignment."""
     b, s, dim = x.shape
     dt = torch.bfloat16 if x.dtype == wkv.dtype == wgate.dtype == torch.bfloat16 else torch.float32
     x = x.to(dt).reshape(b * s, dim)
     n = wkv.shape[0]
-    if (b * s > 8 and dim % 64 == 0 and 128 <= dim <= 1 << 20 and wkv.dim() == 2 and wkv.shape == wgate.shape
-            and wkv.shape[1] == dim and all(w.dtype == dt and w.is_contiguous() and w.data_ptr() % 16 == 0
-                                            for w in (wkv, wgate)) and x.data_ptr() % 16 == 0):
+    if wkv.dim() == 2 and wkv.shape == wgate.shape and wkv.shape[1] == dim and wkv.dtype == wgate.dtype == dt:
         y = ops.linear_pair_op(x, wkv, wgate)
     else:
         y = ops.linear_op(x, torch.cat([wkv, wgate], dim=0).to(dt), 1, torch.float32)

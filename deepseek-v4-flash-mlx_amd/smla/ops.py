@@ -515,16 +515,20 @@ linear_op = _with_eager_route(linear_op, _linear)
 
 
 def _linear_pair(x: torch.Tensor, w0: torch.Tensor, w1: torch.Tensor) -> torch.Tensor:
-    """x [T, K], w0 and w1 [N, K] (all bf16 or all fp32; K a multiple of 64 from 128) -> fp32 [T, 2N] =
-    [x @ w0^T, x @ w1^T], one launch of the tiled GEMM."""
+    """x [T, K], w0 and w1 [N, K] (all bf16 or all fp32) -> fp32 [T, 2N] = [x @ w0^T, x @ w1^T]: one launch
+    of the tiled GEMM over both weights where they are, for more than 8 rows of 16-byte aligned tensors
+    with K a multiple of 64 from 128 to 2^20; otherwise ``linear`` of the stacked weights."""
     _on_gpu(x, w0, w1)
     if w0.shape != w1.shape or x.dim() != 2 or w0.dim() != 2 or x.shape[1] != w0.shape[1]:
         raise ValueError("linear_pair: x [T, K] and w0, w1 [N, K] do not agree")
     if not x.dtype == w0.dtype == w1.dtype:
         raise TypeError("linear_pair: x, w0 and w1 share a dtype")
-    x, w0, w1 = x.contiguous(), w0.contiguous(), w1.contiguous()
+    x = x.contiguous()
     T, K = x.shape
     N = w0.shape[0]
+    if (T <= 8 or K % 64 or not 128 <= K <= 1 << 20 or not (w0.is_contiguous() and w1.is_contiguous())
+            or (x.data_ptr() | w0.data_ptr() | w1.data_ptr()) % 16):
+        return _linear(x, torch.cat([w0, w1], dim=0), 1, torch.float32)
     y = torch.empty(T, 2 * N, dtype=torch.float32, device=x.device)
     wsb = _lib.lib().smla_linear_pair_workspace(T, N, K, dtype_code(x))
     ws = torch.empty(wsb, dtype=torch.uint8, device=x.device) if wsb else None
