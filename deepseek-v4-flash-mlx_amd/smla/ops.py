@@ -36,35 +36,59 @@ def _stream(t):
 # nothing that needs the op itself skip it and run the op's own body.  linear of one token: 17 -> 10 us.
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
 _VALUES = (int, float, bool, type(None), torch.dtype)
-_raw_stream = torch._C._cuda_getCurrentRawStream
+try:
+    _raw_stream = torch._C._cuda_getCurrentRawStream
+except AttributeError:      # a torch built without it
+    def _raw_stream(index):
+        return torch.cuda.current_stream(index).cuda_stream
+try:
+    _dispatch_modes, _function_modes = torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack
+    _transform, _tracer = torch._C._functorch.peek_interpreter_stack, torch._C._get_tracing_state
+    _levels, _profiler, _compiling = torch.autograd.forward_ad, torch.autograd.profiler, torch.compiler.is_compiling
+    _has_eager = _levels._current_level >= -1 and _profiler._is_profiler_enabled in (False, True)
+except (AttributeError, TypeError):     # a torch without one of these names: every call takes the op
+    _has_eager = False
 
 
 def _eager(args):
-    """Whether a call with these arguments needs nothing of the registered op: plain CUDA tensors, none
-    differentiated, and no compiler, tracer, functorch transform, forward-mode level or torch
-    function / dispatch mode around it."""
-    if (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
-            or torch._C._functorch.peek_interpreter_stack() is not None or torch._C._get_tracing_state() is not None
-            or torch.autograd.forward_ad._current_level >= 0):
+    """Whether a call with these arguments needs nothing of the registered op: plain CUDA tensors whose
+    memory holds their values (no negative bit), none differentiated, and no compiler, tracer, functorch
+    transform, forward-mode level, torch function / dispatch mode or profiler (which lists ops by name)
+    around it."""
+    if (not _has_eager or _compiling() or _dispatch_modes() or _function_modes() or _transform() is not None
+            or _tracer() is not None or _levels._current_level >= 0 or _profiler._is_profiler_enabled):
         return False
     grad = torch.is_grad_enabled()
     for a in args:
         if type(a) in _PLAIN:
-            if not a.is_cuda or (grad and a.requires_grad):
+            if not a.is_cuda or a.is_neg() or (grad and a.requires_grad):
                 return False
         elif type(a) not in _VALUES:
             return False
     return True
 
 
-def _with_eager_route(op, body):
-    """The registered op, with calls that need nothing of it going straight to its body."""
-    def call(*args, **kwargs):
-        if not kwargs and _eager(args):
-            return body(*args)
-        return op(*args, **kwargs)
-    call.__name__, call.__doc__, call.op = body.__name__, body.__doc__, op
-    return call
+class _with_eager_route:
+    """The registered op, with calls that need nothing of it going straight to its body.  The op's methods
+    (register_autograd, register_kernel, ...) are this object's too; a caller that asks for one changes the
+    op, and every call goes through it from then on."""
+
+    def __init__(self, op, body):
+        self.op, self.body = op, body
+        self.__name__, self.__doc__ = body.__name__, body.__doc__
+
+    def __call__(self, *args, **kwargs):
+        if self.body is not None and not kwargs and _eager(args):
+            return self.body(*args)
+        return self.op(*args, **kwargs)
+
+    def __getattr__(self, name):    # what this object does not have itself
+        if name.startswith("__") or "op" not in self.__dict__:
+            raise AttributeError(name)
+        value = getattr(self.op, name)
+        if not name.startswith("_"):
+            self.body = None
+        return value
 
 
 def _on_gpu(*ts):

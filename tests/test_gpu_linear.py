@@ -460,3 +460,45 @@ def test_ops_eager_route(dev):
     assert len(seen) >= 6 and not any(seen)
     with torch.no_grad():
         assert ops._eager((leaf, w, 1, torch.float32))
+
+
+def test_ops_eager_route_negative_bit(dev):
+    """A tensor with the negative bit set (its memory holds the negated values) gives the op's result."""
+    from smla import ops
+    announce("ops eager route, negative bit")
+    x = torch.randn(4, 512, device=dev)
+    w = torch.randn(64, 512, device=dev)
+    neg = torch._neg_view(x)
+    assert neg.is_neg() and neg.is_contiguous()
+    assert torch.equal(ops.linear_op(neg, w, 1, torch.float32), ops.linear_op(-x, w, 1, torch.float32))
+    idx = ops.topk_op(torch._neg_view(x), 8, None, 0)
+    assert torch.equal(idx, ops.topk_op(-x, 8, None, 0))
+
+
+def test_ops_eager_route_keeps_the_op(dev):
+    """Under a profiler the call is listed by the op's name, the op's own methods are there, and an op that a
+    caller has extended is used from then on."""
+    from smla import ops
+    announce("ops eager route, profiler and methods")
+    x, w = torch.randn(4, 512, device=dev), torch.randn(64, 512, device=dev)
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
+        ops.linear_op(x, w, 1, torch.float32)
+    assert any(e.key == "smla::linear" for e in prof.key_averages())
+
+    @torch.library.custom_op("smla_test::twice", mutates_args=(), device_types="cuda")
+    def twice(a: torch.Tensor) -> torch.Tensor:
+        return 2 * a
+
+    called = []
+
+    def body(a):
+        called.append(a)
+        return 2 * a
+
+    op = ops._with_eager_route(twice, body)
+    assert torch.equal(op(x), 2 * x) and len(called) == 1
+    op.register_autograd(lambda ctx, g: 2 * g)
+    leaf = x.clone().requires_grad_()
+    op(leaf).sum().backward()
+    assert torch.equal(leaf.grad, torch.full_like(x, 2.0))
+    assert torch.equal(op(x), 2 * x) and len(called) == 1
