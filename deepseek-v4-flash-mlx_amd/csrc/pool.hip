@@ -260,7 +260,9 @@ __global__ __launch_bounds__(kPoolThreads) void gated_pool_kernel(
   const int64_t G = N / ratio;
   const int64_t bg = blockIdx.x;
   const f32x2_t y = gated_pool_body(bg / G, bg % G, kv, score, ape, norm_w, cos_t, sin_t, d, ratio, rd, eps, sim, ld, ldb);
-  *(f32x2_t*)(out + bg * (int64_t)d + 2 * threadIdx.x) = y;
+  float* o = out + bg * (int64_t)d + 2 * threadIdx.x;  // 4-byte aligned: the entry asks no more of out
+  o[0] = y[0];
+  o[1] = y[1];
 }
 
 // the ring step of sequence b, run by one workgroup of d/2 threads

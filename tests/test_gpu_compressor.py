@@ -220,3 +220,26 @@ def test_project_pair(dev, s, dim, n, xdt, wdt, gdt):
         assert got.dtype == torch.float32 and got.shape == (2, s, n)
         ref, mag = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
         assert bool(((got.double() - ref).abs() <= (dim + 8) * 2.0 ** -23 * mag).all())   # a dim-term fp32 sum
+
+
+def test_gated_pool_unaligned_output(dev):
+    """smla_gated_pool takes any float pointer for its result: rows written 4 bytes past an 8-byte boundary are
+    the rows, and nothing around them is touched."""
+    from smla import _lib
+    announce("gated pool, output at an odd float")
+    g = torch.Generator(device=dev).manual_seed(3)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev)  # noqa: E731
+    B, N, d, r, rd = 2, 12, 128, 4, 64
+    kv, sc, ape, nw, cs, sn = rnd(B, N, 2 * d), rnd(B, N, 2 * d), rnd(r, 2 * d), rnd(d), rnd(N, rd // 2), rnd(N, rd // 2)
+    n = B * (N // r) * d
+    out = torch.full((2, n + 2), 7.0, device=dev)
+    assert (out[1].data_ptr() + 4) % 8 == 4
+
+    def call(ptr):
+        _lib.call("smla_gated_pool", kv.data_ptr(), sc.data_ptr(), ape.data_ptr(), nw.data_ptr(), cs.data_ptr(),
+                  sn.data_ptr(), B, N, d, r, rd, 1e-6, _lib.SIM_NONE, ptr, torch.cuda.current_stream().cuda_stream)
+
+    call(out[0].data_ptr())
+    call(out[1].data_ptr() + 4)
+    assert torch.equal(out[0, :n], out[1, 1:n + 1])
+    assert out[1, 0] == 7.0 and out[1, n + 1] == 7.0 and bool((out[0, n:] == 7.0).all())
