@@ -683,8 +683,8 @@ int64_t gemm_tiled_workspace(int64_t T, int64_t G, int64_t N, int64_t K, bool f3
 // y [T, G*N] (row stride G*N) = grouped x [T, G*K] (row stride ldx elements) times w [G*N, K]^T.
 // x and w both bf16 (f32_operands false) or both fp32; y bf16 or fp32.  With pos (bf16 only), inverse RoPE
 // of the last 64 dims of every head_dim-wide head of x on load.  16-byte aligned rows (K % 8 for
-// bf16, K % 4 for fp32).  ws: gemm_tiled_workspace bytes for the partial sums of a split K range, or
-// less (null): the plan without splits.  With w2, G = 2 groups of weights w and w2 that both multiply
+// bf16, K % 4 for fp32).  ws: gemm_tiled_workspace bytes, 16-byte aligned, for the partial sums of a split
+// K range, or less (null): the plan without splits.  With w2, G = 2 groups of weights w and w2 that both multiply
 // the same x [T, K] (shapes the ring kernels take, else SMLA_E_UNSUPPORTED).  Returns SMLA_OK or a hipError_t.
 int launch_gemm_tiled(const void* x, int64_t ldx, bool f32_operands, const void* w, int64_t T, int64_t G, int64_t N,
                       int64_t K, const int32_t* pos, const float* cos_t, const float* sin_t, int64_t head_dim,
@@ -692,7 +692,7 @@ int launch_gemm_tiled(const void* x, int64_t ldx, bool f32_operands, const void*
   const int64_t ldy = G * N;
   if (f32_operands ? f32_takes(ldx, K) : ring_takes(ldx, K) && (!pos || head_dim % 64 == 0)) {
     const int64_t need = gemm_tiled_workspace(T, G, N, K, f32_operands);
-    const bool split = need > 0 && ws && ws_bytes >= (size_t)need;
+    const bool split = need > 0 && usable_workspace(ws, ws_bytes, (size_t)need);
     const RingPlan p = f32_operands ? f32_plan(T, G, N, K, split) : ring_plan(T, G, N, K, split);
     const int bm = f32_operands ? kFormF32B[p.form] : kFormBM[p.form], bn = f32_operands ? bm : kFormBN[p.form];
     const int64_t nt = (T + bm - 1) / bm, nn = (N + bn - 1) / bn, wgs = nt * nn * G * p.splits;

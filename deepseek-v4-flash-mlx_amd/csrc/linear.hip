@@ -426,7 +426,7 @@ extern "C" int smla_linear_ws(const void* x, int x_dtype, const void* w, int w_d
                               void* stream) {
   int rc = check_linear(x, x_dtype, w, w_dtype, T, G, N, K, y, y_dtype);
   if (rc) return rc;
-  if (!decode_runs(x_dtype, T, G, N, K, true, workspace && workspace_bytes >= smla_linear_workspace(T, G, N, K, x_dtype)))
+  if (!decode_runs(x_dtype, T, G, N, K, true, usable_workspace(workspace, workspace_bytes, smla_linear_workspace(T, G, N, K, x_dtype))))
     return launch_gemm_tiled(x, G * K, x_dtype == SMLA_F32, w, T, G, N, K, nullptr, nullptr, nullptr, 0, y, y_dtype,
                              workspace, workspace_bytes, (hipStream_t)stream);
   return launch_linear(x, w, T, G, N, K, nullptr, nullptr, nullptr, 0, 0, y, y_dtype, (hipStream_t)stream);
@@ -522,7 +522,7 @@ extern "C" int smla_o_proj_ws(const void* o, int o_dtype, const int32_t* pos, co
   if (rc) return rc;
   const bool rot64 = !pos || rd == 64;  // the tiled GEMM rotates exactly the last 64 dims of each head
   const bool dform = decode_runs(o_dtype, T, G, R, Kg, rot64,
-                                 workspace && workspace_bytes >= smla_linear_workspace(T, G, R, Kg, SMLA_BF16),
+                                 usable_workspace(workspace, workspace_bytes, smla_linear_workspace(T, G, R, Kg, SMLA_BF16)),
                                  pos != nullptr);
   if (pos) {
     rc = check_rope_args(pos, cos_t, sin_t, n_pos, heads, head_dim, rd);
@@ -538,7 +538,7 @@ extern "C" int smla_o_proj_ws(const void* o, int o_dtype, const int32_t* pos, co
                            workspace_bytes, st);
   if (rc) return rc;
   if (!decode_runs(SMLA_BF16, T, 1, dim, G * R, true,
-                   workspace && workspace_bytes >= smla_linear_workspace(T, 1, dim, G * R, SMLA_BF16)))
+                   usable_workspace(workspace, workspace_bytes, smla_linear_workspace(T, 1, dim, G * R, SMLA_BF16))))
     return launch_gemm_tiled(mid, G * R, false, wo_b, T, 1, dim, G * R, nullptr, nullptr, nullptr, 0, y, y_dtype,
                              workspace, workspace_bytes, st);
   return launch_linear(mid, wo_b, T, 1, dim, G * R, nullptr, nullptr, nullptr, 0, 0, y, y_dtype, st);

@@ -305,6 +305,11 @@ int launch_gemm_tiled(const void* x, int64_t ldx, bool f32_operands, const void*
 bool gemm_tiled_takes(int64_t G, int64_t K);
 int64_t gemm_tiled_workspace(int64_t T, int64_t G, int64_t N, int64_t K, bool f32_operands);
 
+// whether a caller's workspace can hold `need` bytes of partial sums (read and written 16 bytes at a time)
+inline bool usable_workspace(const void* ws, size_t bytes, size_t need) {
+  return ws && ((uintptr_t)ws & 15) == 0 && bytes >= need;
+}
+
 // the prompt's q up projection with the per-head norm and RoPE (gemm.hip)
 int launch_gemm_heads(const void* x, const void* w, int64_t T, int64_t heads, int64_t K, const int32_t* pos,
                       const float* cos_t, const float* sin_t, int64_t n_pos, float eps, void* out, hipStream_t st);

@@ -470,8 +470,8 @@ int smla_linear(const void* x, int x_dtype, const void* w, int w_dtype, int64_t 
 
 /* smla_linear with a workspace of smla_linear_workspace(...) bytes (may be 0): products whose output
  * has too few tiles to occupy the device split their K range over workgroups, whose fp32 partial sums
- * go through the workspace and are added in a fixed order.  With less workspace (or NULL) it is
- * smla_linear: the same product without the split. */
+ * go through the workspace and are added in a fixed order.  With less workspace (or NULL, or one that
+ * is not 16-byte aligned) it is smla_linear: the same product without the split. */
 size_t smla_linear_workspace(int64_t T, int64_t G, int64_t N, int64_t K, int x_dtype);
 int smla_linear_ws(const void* x, int x_dtype, const void* w, int w_dtype, int64_t T, int64_t G,
                    int64_t N, int64_t K, void* y, int y_dtype, void* workspace, size_t workspace_bytes,

@@ -426,6 +426,28 @@ def test_apply_rotary_emb_mirror(dev, shape, dt, inverse):
     assert got.dtype == x.dtype and torch.equal(got, ref)
 
 
+@pytest.mark.parametrize("T,K,dt", [(20, 4096, torch.bfloat16), (100, 4096, torch.bfloat16), (40, 4096, torch.float32)])
+def test_linear_unaligned_workspace(dev, T, K, dt):
+    """A workspace that 16-byte accesses cannot use is not used: the result of smla_linear, and the bytes of the
+    workspace as they were."""
+    from smla import _lib
+    announce(f"linear, workspace at 4 bytes T={T} K={K} {dt}")
+    g = torch.Generator(device=dev).manual_seed(T)
+    N, code = 1000 if T > 32 else 1024, _lib.BF16 if dt == torch.bfloat16 else _lib.F32
+    x = torch.randn(T, K, generator=g, device=dev).to(dt)
+    w = (torch.randn(N, K, generator=g, device=dev) * 0.05).to(dt)
+    y, ref = torch.empty(T, N, device=dev), torch.empty(T, N, device=dev)
+    need = _lib.lib().smla_linear_workspace(T, 1, N, K, code)
+    assert need > 0
+    ws = torch.full((need + 16,), 9, dtype=torch.uint8, device=dev)
+    st = torch.cuda.current_stream().cuda_stream
+    args = (x.data_ptr(), code, w.data_ptr(), code, T, 1, N, K)
+    _lib.call("smla_linear", *args, ref.data_ptr(), _lib.F32, st)
+    _lib.call("smla_linear_ws", *args, y.data_ptr(), _lib.F32, ws.data_ptr() + 4, need, st)
+    assert torch.equal(y, ref) and bool((ws == 9).all())
+    _check_linear(y, x.cpu(), w.cpu(), 1, torch.float32)
+
+
 def test_ops_eager_route(dev):
     """Plain CUDA tensors skip the registered op and give its result; whatever needs the op (a
     differentiated input, forward-mode level, functorch transform, fake tensors, a tracer, a CPU
