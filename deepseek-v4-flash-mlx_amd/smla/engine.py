@@ -112,14 +112,6 @@ class DecodeLayer:
             self.cuts.append(self.cuts[-1] + t.shape[0])
 
     # -- pieces (each mirrors one span of decode_engine.py) --------------------------------------
-    def q_path(self, qa_f, pos):
-        """``decode_engine.py:78-80``: q [rows, 64, 512] bf16 from the q_down projection qa_f
-        [rows, 1024] of tokens at positions pos [rows], per-head normed, rope dims rotated."""
-        rows = qa_f.shape[0]
-        qa = torch.empty(rows, qa_f.shape[1], dtype=torch.bfloat16, device=qa_f.device)
-        ops.row_epilogue(qa_f, self.q_a_norm, None, None, None, 0, _lib.SIM_NONE, qa)
-        return self._q_up(qa, pos)
-
     def _q_up(self, qa, pos):
         """``decode_engine.py:79-80``: q [rows, 64, 512] bf16 from the normed q down projection."""
         rows = qa.shape[0]
@@ -162,12 +154,6 @@ class DecodeLayer:
             return ids
         return self._select(pos, scores, k)
 
-    def q_and_ids(self, qa_f, pos, scores=None, k=2048):
-        """``q_path`` and ``index_list`` of one decode step, with the per-head q epilogue and the id
-        build in one launch (``smla_row_epilogue_ids``): the same q and ids.  Runs after the ring
-        step, whose emitted row the id build copies."""
-        return self._q_ids_from(self._q_proj(qa_f), pos, scores, k)
-
     def _q_proj(self, qa_f):
         """``decode_engine.py:78``: the fp32 q projection [rows * 64, 512] from the q_down projection."""
         qa = torch.empty(qa_f.shape[0], qa_f.shape[1], dtype=torch.bfloat16, device=qa_f.device)
@@ -175,6 +161,9 @@ class DecodeLayer:
         return _proj(qa, self.w.wq_b).view(-1, HEAD_DIM)
 
     def _q_ids_from(self, q_f, pos, scores, k):
+        """``decode_engine.py:79-80,110-114``: q [rows, 64, 512] bf16 from its fp32 projection and the step's
+        ids (those of ``index_list``), with the per-head q epilogue and the id build in one launch
+        (``smla_row_epilogue_ids``).  Runs after the ring step, whose emitted row the id build copies."""
         q = torch.empty(q_f.shape[0] // N_HEADS, N_HEADS, HEAD_DIM, dtype=torch.bfloat16, device=q_f.device)
         comp = (self.comp32, self.comp) if self.ring_ratio else (None, None)
         take_all = scores is None or not self.ring_ratio
