@@ -410,6 +410,63 @@ def test_o_proj_graph_replays(dev):
         torch.cuda.synchronize()
 
 
+def _split_case(dev, dt):
+    """A product whose plan splits K (checked), and the output path with a workspace."""
+    from smla import _lib
+    from smla import norm_rope as snr
+    g = torch.Generator(device=dev).manual_seed(21)
+    T, N, K = 64, 1024, 4096
+    assert _lib.lib().smla_linear_workspace(T, 1, N, K, _lib.BF16 if dt == torch.bfloat16 else _lib.F32) > 0
+    assert _lib.lib().smla_o_proj_workspace(T, 64, 512, 8, 1024, 4096) > 0
+    x = torch.randn(T, K, generator=g, device=dev).to(dt)
+    w = (torch.randn(N, K, generator=g, device=dev) * 0.05).to(dt)
+    o = torch.randn(T, 64, 512, generator=g, device=dev).to(torch.bfloat16)
+    wa = (torch.randn(8192, 4096, generator=g, device=dev) * 0.02).to(torch.bfloat16)
+    wb = (torch.randn(4096, 8192, generator=g, device=dev) * 0.02).to(torch.bfloat16)
+    pos = torch.randint(0, 4096, (T,), generator=g, device=dev, dtype=torch.int32)
+    return x, w, (o, pos, *snr.rope_tables(64, 4096, device=dev), wa, wb, 8, torch.bfloat16)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+def test_split_products_graph_replays(dev, dt):
+    """Products with split K ranges captured in a HIP graph, their workspaces from the graph's pool: every
+    replay, with eager work and synchronisations between replays, equals the eager result bit for bit."""
+    from smla import ops
+    announce(f"split products graph replay {dt}")
+    x, w, op_args = _split_case(dev, dt)
+    run = lambda: (ops.linear_op(x, w, 1, torch.float32), ops.o_proj_op(*op_args))  # noqa: E731
+    eager = run()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = run()
+    for r in range(3):
+        for t in out:
+            t.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(out, eager)), f"replay {r}"
+        run()                                               # eager work between replays
+        torch.cuda.synchronize()
+
+
+def test_split_products_on_streams(dev):
+    """The same products issued on two streams in turn, each call with a workspace of its own."""
+    from smla import ops
+    announce("split products on two streams")
+    x, w, op_args = _split_case(dev, torch.bfloat16)
+    eager = (ops.linear_op(x, w, 1, torch.float32), ops.o_proj_op(*op_args))
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream(dev) for _ in range(2)]
+    got = []
+    for _ in range(10):
+        for st in streams:
+            with torch.cuda.stream(st):
+                got.append((ops.linear_op(x, w, 1, torch.float32), ops.o_proj_op(*op_args)))
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, b) for pair in got for a, b in zip(pair, eager))
+
+
 @pytest.mark.parametrize("shape,dt", [((2, 5, 64), torch.float32), ((2, 5, 8, 64), torch.bfloat16),
                                       ((1, 7, 64, 64), torch.float32)])
 @pytest.mark.parametrize("inverse", [False, True])
