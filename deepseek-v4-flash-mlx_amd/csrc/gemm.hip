@@ -246,6 +246,7 @@ struct RingArgs {
   uint8_t* y;
   int64_t ldy, split_stride;  // elements
   int vec;                    // rows and groups of y start at multiples of 16 bytes
+  int pair;                   // 2: the tiles of two groups side by side, else 1
 };
 
 // The tile's outputs from the accumulators (layout of tile_loop) to rows t0 .., columns n0 .. of group g
@@ -316,7 +317,11 @@ __device__ __attribute__((always_inline)) inline void store_tile(smla_attn::lds_
 
 // Workgroup order: the launch deals workgroups to the 8 XCDs round-robin; each XCD takes a
 // contiguous run of tiles, ordered in groups of 4 token tiles over all output tiles, so that the
-// tiles running together on an XCD share x and w rows in its L2.  Splits are outermost.
+// tiles running together on an XCD share x and w rows in its L2.  Splits are outermost.  With pair, the 4
+// token tiles of two groups take turns at every output tile: rows of x 64 KB apart fall in the same
+// sets of an L2, which 8 token tiles of one group want at the same column, and two groups spread over
+// twice the sets (8 groups of [4096, 4096] x [1024, 4096]^T 257 -> 225 us, [2000, 4096] 135 -> 120; four
+// or eight groups, with as many times the weights, 247 and 255; tiles started 4 or 8 us apart 250 and 240).
 struct TileId {
   int sp, g, tm, tn;  // split, group, token tile, output tile
 };
@@ -324,14 +329,17 @@ __device__ inline TileId tile_id(const RingArgs& p) {
   const uint32_t tot = gridDim.x, per = tot / kXcds, rem = tot % kXcds, xcd = blockIdx.x % kXcds;
   uint32_t id = xcd * per + (xcd < rem ? xcd : rem) + blockIdx.x / kXcds;
   const uint32_t tiles = (uint32_t)p.nt * p.nn;
-  const uint32_t sg = id / tiles;  // split * G + group
+  uint32_t sg = id / (tiles * p.pair) * p.pair;  // split * G + group
   id -= sg * tiles;
-  const uint32_t grp = id / (4u * p.nn), gs = min(4u, (uint32_t)p.nt - 4 * grp), in = id - grp * 4u * p.nn;
+  const uint32_t blk = 4u * p.nn * p.pair;
+  const uint32_t grp = id / blk, gs = min(4u, (uint32_t)p.nt - 4 * grp), in = id - grp * blk;
+  const uint32_t col = in / gs;  // output tile, of the pair's groups in turn
+  sg += col % p.pair;
   TileId t;
   t.sp = sg / p.G;
   t.g = sg - t.sp * p.G;
   t.tm = 4 * grp + in % gs;
-  t.tn = in / gs;
+  t.tn = col / p.pair;
   return t;
 }
 
@@ -700,8 +708,9 @@ int launch_gemm_tiled(const void* x, int64_t ldx, bool f32_operands, const void*
     const int64_t es = f32_operands ? 4 : 2;
     const uint32_t hs = pos ? (uint32_t)(head_dim / 64) : 1u;
     RingArgs a{(const uint8_t*)x, (const uint8_t*)w, (const uint8_t*)w2, ldx * es, w2 ? 0 : K * es, (int)T, (int)N, (int)K, (int)G, (int)nt,
-               (int)nn, p.splits, pos, cos_t, sin_t, hs, hs > 1 ? (uint32_t)(((1ull << 32) + hs - 1) / hs) : 0u, (uint8_t*)(p.splits > 1 ? ws : y), ldy, T * ldy, 0};
+               (int)nn, p.splits, pos, cos_t, sin_t, hs, hs > 1 ? (uint32_t)(((1ull << 32) + hs - 1) / hs) : 0u, (uint8_t*)(p.splits > 1 ? ws : y), ldy, T * ldy, 0, 1};
     const int odt = p.splits > 1 ? SMLA_F32 : y_dtype;
+    if (!f32_operands && p.form == 3 && G % 2 == 0 && !w2 && a.ldx % 65536 == 0) a.pair = 2;
     a.vec = N % (odt == SMLA_BF16 ? 8 : 4) == 0 && ((uintptr_t)a.y & 15) == 0;
     const int rc = f32_operands  ? (p.form == 0 ? launch_f32<0>(a, wgs, odt, st) : launch_f32<1>(a, wgs, odt, st))
                    : p.form == 0 ? launch_ring<0>(a, wgs, pos != nullptr, odt, st)
@@ -749,7 +758,7 @@ int launch_gemm_heads(const void* x, const void* w, int64_t T, int64_t heads, in
   const int64_t nt = (T + F::BM - 1) / F::BM, wgs = nt * heads;
   if (wgs > 0x7fffffff) return SMLA_E_UNSUPPORTED;
   RingArgs a{(const uint8_t*)x, (const uint8_t*)w, nullptr, K * 2, 0, (int)T, (int)(heads * 512), (int)K, 1, (int)nt,
-             (int)heads, 1, pos, cos_t, sin_t, 8, 0, (uint8_t*)out, heads * 512, 0, 1};
+             (int)heads, 1, pos, cos_t, sin_t, 8, 0, (uint8_t*)out, heads * 512, 0, 1, 1};
   static std::atomic<uint64_t> lds_attr{0};
   if (hipError_t e = smla_set_dynamic_lds((const void*)gemm_heads_kernel, L::LDS, lds_attr); e != hipSuccess) return (int)e;
   hipLaunchKernelGGL(gemm_heads_kernel, dim3((unsigned)wgs), dim3(L::NW * 64), L::LDS, st, a, n_pos, eps);

@@ -55,9 +55,8 @@ struct Tile {
 // times rows 0 .. BN-1 of w (likewise), over nk >= D steps of 64 k.  Accumulator register r of block
 // (mb, nb) is row WM wm + 32 mb + 8 (r / 4) + 4 (lane / 32) + r mod 4 of x, row WN wn + 32 nb +
 // lane mod 32 of w, for wave wm + (BM / WM) wn.  BM ldx and BN ldw fit 31 bits.
-// An output is one chain of fp32 accumulations over k = 0, 16, 32 ..: tiles whose rows of x lie 64 KB apart
-// (the same sets of an L2) ran 4 steps apart once (8 groups of [4096, 4096] x [1024, 4096]^T 281 -> 262 us),
-// but a token's sums then depended on where it stands in the prompt.  landed(step, stage, Int<first>): run
+// An output is one chain of fp32 accumulations over k = 0, 16, 32 .., whichever tile it is in: a token's sums
+// do not depend on where it stands in the prompt.  landed(step, stage, Int<first>): run
 // after a step's stage has landed and before it is read.
 template <int BM, int BN, int WM, int WN, int D, class F>
 __device__ __attribute__((always_inline)) inline void tile_loop(lds_u8_t* lds, const uint8_t* __restrict__ xk,

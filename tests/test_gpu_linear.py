@@ -105,6 +105,17 @@ def test_linear_tile_forms(dev, T, G, N, K, out_dtype):
 
 
 @pytest.mark.parametrize("T,G,N,K", [
+    (1300, 8, 1024, 4096),   # 6 token tiles of 256: groups of 4 and 2, the last tile ragged
+    (2305, 2, 1500, 16384),  # two groups, ragged outputs
+    (1100, 16, 700, 2048),
+    (4000, 1, 1024, 32768),  # one group: no pairs
+])
+def test_linear_rows_64k_apart(dev, T, G, N, K):
+    """Rows of x 64 KB apart take the tiles of two groups side by side: every tile of every group is there."""
+    test_linear_tile_forms(dev, T, G, N, K, torch.bfloat16)
+
+
+@pytest.mark.parametrize("T,G,N,K", [
     # both sides of the lines between the weight-streaming kernels and the tiled GEMM
     (16, 1, 8192, 512), (9, 1, 8208, 512),            # 512 and 513 workgroups of 16 outputs
     (9, 2, 4096, 4096), (16, 1, 8192, 4608),          # 512 x 4096 and beyond
