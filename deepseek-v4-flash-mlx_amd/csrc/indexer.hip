@@ -228,7 +228,7 @@ __global__ __launch_bounds__(256) void indexer_kernel(const void* __restrict__ q
 // + j mod 4.  The head chain walks the 16-lane rows: after the four heads of row g, every row takes
 // row g's sum (two lane swaps).
 //
-// Di = 128 doubles the chain and the registers of a key row, and q is converted where it is used: 1024
+// Di = 128 doubles the chain and the registers of a key row (q is converted where it is used): 1024
 // queries x 64 heads over 2048 fp4 keys with the top-k take 310 us at three waves per SIMD (bf16 q, keys
 // of at most 256 bytes; 321 at two, where fp32 q or keys stay) against 676 on the vector ALUs, which read
 // q from LDS.  Bound by the MFMA chain: 64 cycles a dependent step, tiles past nvis skip theirs.
@@ -306,7 +306,9 @@ void indexer_mfma_kernel(const void* __restrict__ q, const void* __restrict__ ke
   }
   const int64_t nv = nvis ? (int64_t)nvl : N;
   __syncthreads();
-  if (kb >= nv) {  // no key of the wave's tile is visible (wave-uniform; no barrier follows)
+  // no key of the wave's tile is visible (wave-uniform; no barrier follows).  Not in the short chains of 64-dim
+  // fp4 keys, which the test makes 1 % longer (201 queries over 1700 keys 31.9 -> 32.4 us; e4m3 57.8 -> 55.6)
+  if ((DI == 128 || KDT != kFp4) && kb >= nv) {
     const int64_t n = kb + lane;
     if (lane < KT && n < N) scores[bs * N + n] = -SMLA_INF;
     return;
@@ -317,15 +319,24 @@ void indexer_mfma_kernel(const void* __restrict__ q, const void* __restrict__ ke
 #pragma unroll
   for (int v = 0; v < QW; v++) asm volatile("" : "+v"(qw[v]));
   auto wrow = [&](int h) -> float { return w_s[h]; };
-  // q[lane][d] for a constant d, converted where it is used (beside a 64-cycle MFMA): an array of 128
-  // floats ahead of the chain would cost a second wave its registers
-  auto qval = [&](int d) __attribute__((always_inline)) -> float {
+  // q[lane][d] for a constant d.  64 dims are converted ahead of the chain (1024 queries over 2048 fp4 keys 154 us,
+  // 160 with the conversions in it); of 128 each is converted where it is used, beside a 64-cycle MFMA:
+  // an array of 128 floats would cost a second wave its registers
+  auto convert = [&](int d) __attribute__((always_inline)) -> float {
     if constexpr (QDT == SMLA_BF16) {
       const uint32_t w = qw[d / 8][d % 8 / 2];
       return __uint_as_float(d & 1 ? w & 0xffff0000u : w << 16);
     } else {
       return __uint_as_float(qw[d / 4][d % 4]);
     }
+  };
+  float qf[DI == 64 ? DI : 1];
+  if constexpr (DI == 64)
+#pragma unroll
+    for (int d = 0; d < DI; d++) qf[d] = convert(d);
+  auto qval = [&](int d) __attribute__((always_inline)) -> float {
+    if constexpr (DI == 64) return qf[d];
+    else return convert(d);
   };
   // 16 values of the key row starting at d0 = 16 db, as fp32 (fold: see fp4_block16)
   auto block16 = [&](int db, float (&o)[16], auto fold) {
