@@ -15,7 +15,8 @@
 //   33, 8 groups of [300, 4096] x [1024, 4096]^T 100 -> 33, [1024, 4096] x [1024, 4096]^T 83 -> 17,
 //   [4096, 8192] x [4096, 8192]^T 244 -> 210, [4096, 1024] x [32768, 1024]^T 291 -> 265.
 //
-// gemm_kernel (fp32 operands, and K tails): 4 waves computing a 128 x 128 tile, each wave a
+// gemm_kernel (the K that the ring kernels do not take: bf16 below 128 or not a multiple of 64, fp32 below 64
+// or not a multiple of 32, rows past 31-bit offsets): 4 waves computing a 128 x 128 tile, each wave a
 // 64 x 64 quarter as 2 x 2 blocks of v_mfma_f32_32x32x16_bf16 (bf16 operands) or
 // v_mfma_f32_32x32x2f32 (fp32 operands), accumulating in fp32.  K advances in steps of 128 bytes
 // per row (64 bf16 / 32 fp32): the next step's tiles are loaded into registers while the current
@@ -434,8 +435,9 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const RingArgs p) {
   tile_loop_f32<BM, BN, WM, WN, D>((lds_u8_t*)lds_g, xk, p.ldx, p.T - 1 - t0, wk, (int64_t)p.K * 4, p.N - 1 - n0, k1 - k0,
                                    acc);
   store_tile<F, YDT>((lds_u8_t*)lds_g, p, id.sp, id.g, t0, n0, acc);
-  // a sum that is infinite or NaN may be so only because an operand has no split, and every sum of a wave
-  // that met a value below 2^-110 may have lost some of it: they are taken from the fp32 MFMAs, a wave's block of 32 x 32 at a time, and stored again behind the first store
+  // a sum that is infinite or NaN may be so only because an operand has no split or the scaled sum no
+  // room: it is taken from the fp32 MFMAs, a wave's block of 32 x 32 at a time, and stored again behind
+  // the first store
   uint64_t bad = 0;
 #pragma unroll
   for (int i = 0; i < L::MB * L::NB * 16; i++)
@@ -465,9 +467,10 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const RingArgs p) {
 // 128 tokens x one head of 512, so the head's RMS norm (weightless, v4mlx/mla.py:26-28) and the RoPE of
 // its last 64 dims run on the accumulators and bf16 leaves.  As two launches the fp32 projection went
 // out and came back (1.07 GB for 4096 tokens x 64 heads).  Two stages of (128 + 512) x 64 k fill the 160 KB
-// of LDS.  4096 tokens, K 1024: 287 us, against 283 of fp32 product and 277 of epilogue; about 190 of them
-// are the K loop (1.46 us a step, 80 KB of operands per CU), the rest the 268 MB of rows, which leave when
-// the tiles end together.
+// of LDS.  4096 tokens, K 1024: 297-310 us repeated alone (the fp32 product 278-286 and the epilogue 276-280
+// as two launches), about 350 in a layer, where the operands come from memory; 8 tiles per CU one after
+// the other, each a K loop of 16 steps, then the norms, then 128 KB of rows, and nothing of one tile
+// overlaps the next (the same product in 256 x 256 tiles with bf16 results takes 232-245).
 struct HeadForm {
   static constexpr int BM = 128, BN = 512, WM = 64, WN = 128, D = 2;
 };

@@ -117,7 +117,8 @@ class DecodeLayer:
         rows = qa.shape[0]
         q = torch.empty(rows, N_HEADS, HEAD_DIM, dtype=torch.bfloat16, device=qa.device)
         # from 192 tokens the projection's tiles of 128 tokens x one head fill the device and take the
-        # epilogue with them (31 against 21 + 15 us at 192 tokens, 287 against 283 + 277 at 4096)
+        # epilogue with them (34 against 21 + 17 us at 192 tokens, 297 against 278 + 276 at 4096); the
+        # same bits either way
         wq_b = self.w.wq_b
         if (rows >= 192 and wq_b.dtype == torch.bfloat16 and wq_b.is_contiguous() and wq_b.data_ptr() % 16 == 0
                 and wq_b.shape[1] % 64 == 0 and wq_b.shape[1] >= 128 and pos.dtype == torch.int32 and pos.dim() == 1

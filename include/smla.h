@@ -489,8 +489,8 @@ int smla_linear_pair_ws(const void* x, int x_dtype, const void* w0, const void* 
 /* smla_q_up: a prompt's q up projection with its per-head epilogue, oracle/decode_engine.py:78-80:
  * out [T, heads, 512] BF16 = x [T, K] w^T (w [heads*512, K], both BF16), every head RMS-normed without
  * weights (v4mlx/mla.py:26-28, eps), its last 64 dims rotated to position pos[t] in [0, n_pos) (cos/sin
- * [n_pos, 32], ref_torch/norm_rope.py:53-62): smla_linear with an fp32 result followed by
- * smla_row_epilogue, in one launch without the fp32 rows.  K a multiple of 64 from 128
+ * [n_pos, 32], ref_torch/norm_rope.py:53-62): smla_linear (without workspace) with an fp32
+ * result followed by smla_row_epilogue, bit for bit, in one launch without the fp32 rows.  K a multiple of 64 from 128
  * (SMLA_E_UNSUPPORTED otherwise), 16-byte aligned pointers. */
 int smla_q_up(const void* x, const void* w, int64_t T, int64_t heads, int64_t K, const int32_t* pos,
               const float* cos_t, const float* sin_t, int64_t n_pos, float eps, void* out, void* stream);
