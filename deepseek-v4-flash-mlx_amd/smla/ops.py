@@ -45,6 +45,7 @@ try:
     _dispatch_modes, _function_modes = torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack
     _transform, _tracer = torch._C._functorch.peek_interpreter_stack, torch._C._get_tracing_state
     _levels, _profiler, _compiling = torch.autograd.forward_ad, torch.autograd.profiler, torch.compiler.is_compiling
+    _grad_enabled = torch.is_grad_enabled
     _has_eager = _levels._current_level >= -1 and _profiler._is_profiler_enabled in (False, True)
 except (AttributeError, TypeError):     # a torch without one of these names: every call takes the op
     _has_eager = False
@@ -58,7 +59,7 @@ def _eager(args):
     if (not _has_eager or _compiling() or _dispatch_modes() or _function_modes() or _transform() is not None
             or _tracer() is not None or _levels._current_level >= 0 or _profiler._is_profiler_enabled):
         return False
-    grad = torch.is_grad_enabled()
+    grad = _grad_enabled()
     for a in args:
         if type(a) in _PLAIN:
             if not a.is_cuda or a.is_neg() or (grad and a.requires_grad):
@@ -68,27 +69,29 @@ def _eager(args):
     return True
 
 
-class _with_eager_route:
+def _with_eager_route(op, body):
     """The registered op, with calls that need nothing of it going straight to its body.  The op's methods
-    (register_autograd, register_kernel, ...) are this object's too; a caller that asks for one changes the
-    op, and every call goes through it from then on."""
+    (register_autograd, register_kernel, ...) are the function's too; one that is called changes the op, and
+    every call goes through it from then on."""
+    plain = True
 
-    def __init__(self, op, body):
-        self.op, self.body = op, body
-        self.__name__, self.__doc__ = body.__name__, body.__doc__
+    def call(*args, **kwargs):
+        if plain and not kwargs and _eager(args):
+            return body(*args)
+        return op(*args, **kwargs)
 
-    def __call__(self, *args, **kwargs):
-        if self.body is not None and not kwargs and _eager(args):
-            return self.body(*args)
-        return self.op(*args, **kwargs)
+    def method(name):
+        def changed(*args, **kwargs):
+            nonlocal plain
+            plain = False
+            return getattr(op, name)(*args, **kwargs)
+        return changed
 
-    def __getattr__(self, name):    # what this object does not have itself
-        if name.startswith("__") or "op" not in self.__dict__:
-            raise AttributeError(name)
-        value = getattr(self.op, name)
+    for name in dir(op):
         if not name.startswith("_"):
-            self.body = None
-        return value
+            setattr(call, name, method(name))
+    call.__name__, call.__doc__, call.op = body.__name__, body.__doc__, op
+    return call
 
 
 def _on_gpu(*ts):
